@@ -23,6 +23,8 @@
 // exp(s - max), the sum and the value accumulation; the output is scaled by
 // 1/sum at the end. Rows of the block that belong to different prompts are
 // processed one prompt at a time.
+#include <algorithm>
+
 #include "decode.h"
 #include "gemm_common.h"
 #include "internal.h"
@@ -637,6 +639,201 @@ __global__ __launch_bounds__(512) void attn_prompt_kernel(AttnArgs a, AttnRope r
 
 bool attention_mfma_takes(int64_t hd, int64_t vd, int64_t groups) {
     return groups >= 1 && ((hd == 64 && vd == 64) || (hd == 128 && vd == 128) || (hd == 192 && vd == 128));
+}
+
+// ---------------------------------------------------------------------------
+// Attention of a few rows (decode steps, short prompts): one workgroup per
+// (row, KV head, up to G of its query heads), its waves walking the row's own
+// keys. The 16-row blocks above stage each prompt's keys through LDS one
+// prompt at a time, so a decode step's rows (a prompt each) run one after
+// another on a workgroup per KV head: 116 us for 16 prompts of 32 to 96 keys
+// (2 KV heads of 64), 69 us for one row of 500 keys (8 KV heads of 128).
+// Here a row's keys and values are read once, straight into registers, by
+// 4 to 16 waves with several rows of the cache in flight each: 5 and 9 us.
+// What bounds it is that read (3.4 TB/s over 48 rows of 300 to 900 keys; one
+// CU's loads for a single row) and two barriers.
+//
+// The products are f32 multiply-adds. Scores: 16 lanes share a key (lane c
+// holds dims 4 c + 64 j .. +4), a wave takes 4 keys a step and all G heads of
+// them. Softmax in the reference's order over the scores in LDS: the maximum,
+// Cephes exp of the difference, the sum. Values: VD / 4 lanes share a row of
+// the cache, the waves' partial outputs are added in LDS in wave order and
+// scaled by 1 / sum. Any rows may be mixed; rows outside the cache are
+// skipped.
+constexpr int ROW_MAXK = 1024;  // keys a row may have (the KV cache's limit)
+
+// workgroup barrier that orders LDS only: global loads stay in flight
+__device__ __forceinline__ void attn_lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+template <int HD, int VD, int G>
+__global__ __launch_bounds__(1024) void attn_row_kernel(AttnArgs a) {
+    constexpr int QJ = HD / 64;             // float4s of a key a lane holds
+    constexpr int VL = VD / 4, VS = 64 / VL;  // lanes of a value row, rows a step
+    constexpr int U = 4;                    // steps whose loads are in flight together
+    extern __shared__ __attribute__((aligned(16))) float row_lds[];
+    float *sc = row_lds;                    // [key][G] scores, then exp; then the waves' outputs
+    __shared__ float inv_s[G];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, NW = blockDim.x >> 6;
+    const int64_t r = blockIdx.x, hkv = blockIdx.y;
+    const int64_t pos = a.rows[r].pos, b = a.rows[r].b;
+    if (b >= a.nb || pos >= a.T) return;  // outside the KV cache: the row is skipped
+    const int n_keys = (int)pos + 1;
+    const int h0 = blockIdx.z * G, ng = (int)(a.groups - h0 < G ? a.groups - h0 : G);
+    const int64_t head = hkv * a.groups + h0;
+    const float *kb = a.kc + b * a.T * a.kvd + hkv * a.hd, *vb = a.vc + b * a.T * a.kvd + hkv * a.hd;
+
+    // scores
+    {
+        const int sub = lane >> 4, c16 = lane & 15;
+        float4 q[G][QJ];
+#pragma unroll
+        for (int h = 0; h < G; h++)
+#pragma unroll
+            for (int j = 0; j < QJ; j++)
+                q[h][j] = *(const float4 *)(a.q + (r * a.heads + head + (h < ng ? h : 0)) * HD + 64 * j + 4 * c16);
+        for (int p0 = 4 * wave; p0 < n_keys; p0 += 4 * NW * U) {
+            float4 k[U][QJ];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                int p = p0 + 4 * NW * u + sub;
+                p = p < n_keys ? p : n_keys - 1;
+#pragma unroll
+                for (int j = 0; j < QJ; j++) k[u][j] = *(const float4 *)(kb + p * a.kvd + 64 * j + 4 * c16);
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int p = p0 + 4 * NW * u + sub;
+                float mine = 0.f;
+#pragma unroll
+                for (int h = 0; h < G; h++) {
+                    float s = 0.f;
+#pragma unroll
+                    for (int j = 0; j < QJ; j++) {
+                        s = __builtin_fmaf(k[u][j].x, q[h][j].x, s);
+                        s = __builtin_fmaf(k[u][j].y, q[h][j].y, s);
+                        s = __builtin_fmaf(k[u][j].z, q[h][j].z, s);
+                        s = __builtin_fmaf(k[u][j].w, q[h][j].w, s);
+                    }
+                    s = row16_sum(s);
+                    if (c16 == h) mine = s;
+                }
+                if (c16 < G && p < n_keys) sc[p * G + c16] = __fmul_rn(mine, a.scale);
+            }
+        }
+    }
+    // the first values' loads before the softmax
+    const int vsub = lane / VL, vc4 = (lane % VL) * 4;
+    float4 v[U];
+    auto load_v = [&](int p0) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            int p = p0 + VS * NW * u + vsub;
+            p = p < n_keys ? p : n_keys - 1;
+            v[u] = *(const float4 *)(vb + p * a.kvd + vc4);
+        }
+    };
+    load_v(VS * wave);
+    attn_lds_barrier();
+    for (int h = wave; h < G; h += NW) {
+        float m = -INFINITY;
+        for (int p = lane; p < n_keys; p += 64) m = fmaxf(m, sc[p * G + h]);
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+        float sum = 0.f;
+        for (int p = lane; p < n_keys; p += 64) {
+            const float e = exp_cephes(__fsub_rn(sc[p * G + h], m));
+            sc[p * G + h] = e;
+            sum = __fadd_rn(sum, e);
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) sum = __fadd_rn(sum, __shfl_xor(sum, o, 64));
+        if (lane == 0) inv_s[h] = __fdiv_rn(1.0f, sum);
+    }
+    attn_lds_barrier();
+    // values
+    float4 o[G];
+#pragma unroll
+    for (int h = 0; h < G; h++) o[h] = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int p0 = VS * wave; p0 < n_keys; p0 += VS * NW * U) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int p = p0 + VS * NW * u + vsub;
+            const bool in = p < n_keys;
+            const float *pr = sc + (in ? p : 0) * G;
+#pragma unroll
+            for (int h = 0; h < G; h++) {
+                const float e = in ? pr[h] : 0.f;
+                o[h].x = in ? __builtin_fmaf(e, v[u].x, o[h].x) : o[h].x;
+                o[h].y = in ? __builtin_fmaf(e, v[u].y, o[h].y) : o[h].y;
+                o[h].z = in ? __builtin_fmaf(e, v[u].z, o[h].z) : o[h].z;
+                o[h].w = in ? __builtin_fmaf(e, v[u].w, o[h].w) : o[h].w;
+            }
+        }
+        if (p0 + VS * NW * U < n_keys) load_v(p0 + VS * NW * U);
+    }
+#pragma unroll
+    for (int h = 0; h < G; h++)
+#pragma unroll
+        for (int d = VL; d < 64; d <<= 1) {
+            o[h].x = __fadd_rn(o[h].x, __shfl_xor(o[h].x, d, 64));
+            o[h].y = __fadd_rn(o[h].y, __shfl_xor(o[h].y, d, 64));
+            o[h].z = __fadd_rn(o[h].z, __shfl_xor(o[h].z, d, 64));
+            o[h].w = __fadd_rn(o[h].w, __shfl_xor(o[h].w, d, 64));
+        }
+    attn_lds_barrier();  // every wave has read its weights: the scores' LDS takes the outputs
+    if (lane < VL) {
+#pragma unroll
+        for (int h = 0; h < G; h++) *(float4 *)&sc[(wave * G + h) * VD + vc4] = o[h];
+    }
+    attn_lds_barrier();
+    for (int i = threadIdx.x; i < ng * VD; i += blockDim.x) {
+        const int h = i / VD;
+        float s = 0.f;
+        for (int w = 0; w < NW; w++) s = __fadd_rn(s, sc[w * G * VD + i]);
+        a.out[(r * a.heads + head) * VD + i] = __fmul_rn(s, inv_s[h]);
+    }
+}
+
+template <int HD, int VD, int G>
+static void launch_attn_row(const AttnArgs &a, int64_t kv_heads, hipStream_t s) {
+    // a wave per 32 positions of the cache, 4 to 16
+    const int64_t nw = std::min<int64_t>(16, std::max<int64_t>(4, (a.T + 31) / 32));
+    const size_t lds = (size_t)std::max<int64_t>(a.T * G, nw * G * VD) * 4;
+    const dim3 grid((unsigned)a.n, (unsigned)kv_heads, (unsigned)((a.groups + G - 1) / G));
+    hipLaunchKernelGGL((attn_row_kernel<HD, VD, G>), grid, dim3((unsigned)(nw * 64)), lds, s, a);
+}
+
+template <int HD, int VD>
+static void launch_attn_rows_g(const AttnArgs &a, int64_t kv_heads, hipStream_t s) {
+    if (a.groups >= 5) launch_attn_row<HD, VD, 8>(a, kv_heads, s);
+    else if (a.groups >= 2) launch_attn_row<HD, VD, 4>(a, kv_heads, s);
+    else launch_attn_row<HD, VD, 1>(a, kv_heads, s);
+}
+
+// The line at 128 rows: below it this kernel was faster for prompts as well
+// as for decode steps (head_dim 128, 8 KV heads, groups of 4: one prompt of
+// 120 tokens 16 against 46 us for the dense check and the prompt kernels,
+// four of 30 tokens 9 against 22; head_dim 64, 2 KV heads, groups of 7: two
+// of 60 tokens 8 against 23). A decode step has at most as many rows as the
+// cache has prompts, whatever their number: 48 rows of 300 to 900 keys 66
+// against 1 295 us, 120 rows of 67 to 200 keys (head_dim 64) 14 against 217.
+// With more rows than prompts and 128 rows or more, prompts share their keys
+// through LDS in the kernels below.
+bool attention_rows_takes(int64_t hd, int64_t vd, int64_t groups, int64_t n, int64_t nb, int64_t T) {
+    return attention_mfma_takes(hd, vd, groups) && (n < 128 || n <= nb) && T <= ROW_MAXK;
+}
+
+void launch_attention_rows(const AttnArgs &a, int64_t kv_heads, hipStream_t s) {
+    DITCH_CHECK(attention_rows_takes(a.hd, a.vd, a.groups, a.n, a.nb, a.T), DITCH_INVALID_ARGUMENT,
+                "attention: the row kernel does not take this shape");
+    if (a.hd == 64) launch_attn_rows_g<64, 64>(a, kv_heads, s);
+    else if (a.hd == 128) launch_attn_rows_g<128, 128>(a, kv_heads, s);
+    else launch_attn_rows_g<192, 128>(a, kv_heads, s);
+    DITCH_TRY_HIP(hipGetLastError());
 }
 
 template <int HD, int VD, int NW>

@@ -1479,7 +1479,8 @@ void model_forward(ditch_hip_model *m, const uint32_t *d_tokens, const ditch_row
         const bool mfma_attn = attention_mfma_takes(hd, vd, nh / nkv);
         const bool frag_epi = attn_split_fragments && frags && mfma_attn && (nh * vd) % 128 == 0 &&
                               frag_only(L.o, n) && !mx_only(L.o, n);
-        const bool prompt_attn = mfma_attn && !frag_epi && attention_prompt_takes(hd, vd, T);
+        const bool row_attn = attention_rows_takes(hd, vd, nh / nkv, n, B, T);
+        const bool prompt_attn = mfma_attn && !row_attn && !frag_epi && attention_prompt_takes(hd, vd, T);
         const bool q_rope_in_attn = prompt_attn && !c.mla && hd == 128 && c.rotary_dim == 128 &&
                                     c.rope_style == DITCH_ROPE_NEOX && !c.qk_norm;
         if (prompt_attn && !dense_checked) {
@@ -1532,7 +1533,8 @@ void model_forward(ditch_hip_model *m, const uint32_t *d_tokens, const ditch_row
             aact = Act{att, aa.xs, aa.ldk};
         }
         if (prompt_attn) aa.dense = dense_flag;
-        if (q_rope_in_attn) launch_attention_mfma_rope(aa, AttnRope{m->rope_cos, m->rope_sin, (int64_t)c.rope_len}, nkv, s);
+        if (row_attn) launch_attention_rows(aa, nkv, s);
+        else if (q_rope_in_attn) launch_attention_mfma_rope(aa, AttnRope{m->rope_cos, m->rope_sin, (int64_t)c.rope_len}, nkv, s);
         else if (mfma_attn) launch_attention_mfma(aa, nkv, s);
         else hipLaunchKernelGGL(attention_kernel, dim3((unsigned)((n * nh + 3) / 4)), dim3(256), 0, s, aa);
         DITCH_TRY_HIP(hipGetLastError());

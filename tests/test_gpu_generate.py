@@ -196,6 +196,56 @@ def test_cache_chunked_prefill_equals_one_shot(dev, ref):
     assert np.abs(lg - lc).max() <= 1e-3 * np.abs(lc).max()
 
 
+# Attention of few rows (a workgroup per row and KV head): query groups of 7
+# (one pass of 8), 10 (8 + 2), 3 and 1, MLA's 192/128 head; decode rows at
+# the first and last position of a 1024-position cache, on both sides of the
+# wave counts' edges, and more rows than 127 (one a prompt).
+ROW_ATTN = {
+    "gqa7_hd64": (dict(heads=7, kv_heads=1, head_dim=64), [1, 33, 128, 90]),
+    "gqa10_hd64_129_prompts": (dict(heads=10, kv_heads=1, head_dim=64), [1, 2, 3] * 43),
+    "gqa3_hd128_full_cache": (dict(heads=6, kv_heads=2, head_dim=128), [1023, 1]),
+    "gqa1_hd128": (dict(heads=2, kv_heads=2, head_dim=128), [129, 511, 2]),
+    "mla_hd192": (None, [5, 64, 130]),
+}
+
+
+@pytest.mark.parametrize("name", list(ROW_ATTN))
+def test_decode_rows_attention_matches_oracle(dev, ref, name):
+    """A decode step after a prefill, against the oracle's one-shot forward."""
+    shape, lens = ROW_ATTN[name]
+    if shape is None:
+        spec = mg.mla("bf16", heads=2, q_lora=64, kv_lora=64, nope=128, rope=64, v_dim=128, layers=1, vocab=512)
+    else:
+        spec = mg.dense("bf16", hidden=256, inter=256, layers=1, vocab=512, seed=2, **shape)
+    B, V = len(lens), spec.config["vocab"]
+    tokens, rows, last = mg.batch(B, [n + 1 for n in lens], V, seed=9)
+    rows = np.asarray(rows, dtype=np.uint32)
+    step = np.zeros(len(tokens), dtype=bool)
+    step[last] = True
+    gm = Model(dev, spec)
+    cache = gm.kv_cache(B, max(lens) + 1)
+    blog = hipmem.Buffer(B * V * 4)
+    try:
+        for sel in (~step, step):
+            bt, br = (hipmem.Buffer.from_array(np.ascontiguousarray(a[sel])) for a in (tokens, rows))
+            bl = hipmem.Buffer.from_array(np.arange(B, dtype=np.uint64))
+            dev.check(dev.lib.ditch_hip_forward_cached(gm.h, cache, bt.ptr, br.ptr, int(sel.sum()), bl.ptr,
+                                                       B if sel is step else 0, blog.ptr, B * V * 4))
+            dev.sync()
+        lg = blog.download(np.float32, (B, V))
+    finally:
+        gm.kv_cache_free(cache)
+        gm.free()
+    cm = RefModel(spec)
+    try:
+        _, lc = cm.forward(tokens, [tuple(r) for r in rows], logit_rows=last)
+    finally:
+        cm.free()
+    # two-term products (2^-18 an activation) and another summation order
+    # through one layer: 1e-5 of the largest logit, ten times that allowed
+    assert np.abs(lg - lc).max() <= 1e-4 * np.abs(lc).max()
+
+
 def test_generation_stops_at_eos_and_full_cache(dev):
     spec = GEN_MODELS["dense_mxfp4"]()
     rng = np.random.default_rng(9)
