@@ -41,6 +41,7 @@ FLAGS = [
 EXTRA = {"gemm_tile.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form", "-mllvm", "-disable-machine-sink"],
          "gemv.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form", "-mllvm", "-pragma-unroll-threshold=1000000"],
          "attention.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+         "gemm_few.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
          "gemm_wide.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 

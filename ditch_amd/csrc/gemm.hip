@@ -3,6 +3,7 @@
 // (the GEMV regime lives in gemv.hip).
 #include "gemm_common.h"
 #include "gemm_f32.h"
+#include "gemm_few.h"
 
 namespace ditch {
 
@@ -133,6 +134,22 @@ static void dispatch_tf(int tf, const GemmParams &p, int64_t max_rows, int64_t n
 void launch_matmul(const TileView &w, float *out, const float *x, int64_t n, const MatmulEpilogue &ep, hipStream_t s,
                    const int32_t *row_index, DevBuf *ws) {
     if (n <= 0 || w.rows <= 0) return;
+    if (few_gemm_takes(w, n, ep.exact != 0)) {
+        const int xt = ep.exact ? 3 : 2;
+        const bool rows = !row_index && few_reads_rows(w, n, x, w.cols);
+        const size_t xb = rows ? 0 : split_bytes_ldk(n, few_ldk(w), xt);
+        // (fragments past a borrowed scratch: the products below need less)
+        if (rows || (ws && !(ws->borrowed && xb > ws->bytes))) {
+            const FewMat m{w, out, ep.bias, ep.delta_b, ep.delta_xa, ep.delta_rank, ep.accumulate};
+            void *xs = nullptr;
+            if (!rows) {
+                xs = ws->get<uint8_t>(xb);
+                launch_split(xs, x, row_index, n, w.cols, w.cols, few_ldk(w), xt, s);
+            }
+            launch_few_gemm(&m, 1, rows ? x : nullptr, w.cols, xs, few_ldk(w), n, xt, s);
+            return;
+        }
+    }
     if (ws && !ep.exact && mx_gemm_takes(w, n)) {
         const int64_t ldst = w.units_k;
         void *xm = ws->get<uint8_t>(mx_frag_bytes(n, ldst));
@@ -190,6 +207,11 @@ void launch_matmul_act(const TileView &w, float *out, const Act &x, int64_t n, c
             launch_matmul(w, out, x.f32, n, ep, s, nullptr, ws);
             return;
         }
+    }
+    if (x.xs && !ep.exact && few_gemm_takes(w, n, false) && x.ldk >= few_ldk(w)) {
+        const FewMat m{w, out, ep.bias, ep.delta_b, ep.delta_xa, ep.delta_rank, ep.accumulate};
+        launch_few_gemm(&m, 1, nullptr, 0, x.xs, x.ldk, n, 2, s);
+        return;
     }
     if (x.xs && !ep.exact && tile_gemm_takes(w, n) && x.ldk >= split_k_tiles(w)) {
         const size_t pb = ws ? tile_part_bytes(w, n, 2) : 0;

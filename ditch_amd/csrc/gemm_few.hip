@@ -1,0 +1,432 @@
+// gemm_few.hip — the product of few tokens: out[n][rows] = x[n][cols] . W^T
+// (tensor.matmulT, tensor.zig:1023-1045) for decode steps, short prompts and
+// ragged small batches, on tensors the conversion instructions decode exactly
+// (TileView::fast: bf16, FP8, MXFP4, INT4, Q8_0).
+//
+// A call of this size reads every weight once and does little with it, so it
+// is bound by the weight read where the matrix is large (14336 x 4096 on one
+// token: FP8 13.3 us = 4.4 TB/s) and by one wave's chain of loads and decode
+// below that (4096 x 4096: 5 to 7 us). Both ask for many short waves:
+//
+//   - a workgroup takes NT groups of 16 rows and MT blocks of 16 tokens; its W
+//     waves take contiguous slices of K and add them through LDS in wave order
+//     (no partial sums in memory, no second launch);
+//   - K advances in steps of 128 columns (1, 2 or 4 weight units a row group);
+//     two register sets alternate, the next step's codes, scale words and
+//     activations requested before the current one is decoded and multiplied.
+//     No branch inside the loop, so every wait is a count of later loads;
+//   - the weights are decoded by the tiled product's instructions
+//     (tile_decode.h). The element decoders of the GEMV (gemv.hip), which
+//     follow NaN and infinity rules these tensors cannot meet, took 100 us for
+//     FP8 and 29 us for MXFP4 at 4096 x 4096 on one token;
+//   - up to 8 tokens (NX) each wave splits its slice of the f32 rows into bf16
+//     terms itself, in its own LDS slot; more tokens come as fragments
+//     (split_kernel's layout), which producers write directly;
+//   - one launch may hold up to three matrices over the same activations.
+//
+// Measured, us a call with its split (before: the GEMV up to 16 tokens, the
+// register-staged or the tiled product above), 4096 x 4096:
+//   n            1            8           16           24           64
+//   FP8     100 -> 6.3   105 -> 9.7  103 -> 10.7  431 -> 12.1  29 -> 15.9
+//   MXFP4    29 -> 5.1    35 -> 8.8   32 -> 10.9  175 -> 11.5  28 -> 15.0
+//   INT4     47 -> 6.2    54 -> 9.6   51 -> 10.9  302 -> 12.5  31 -> 16.1
+#include "gemm_few.h"
+#include "tile_decode.h"
+
+namespace ditch {
+
+namespace {
+
+// MATS matrices in one launch; end[i]: row blocks up to and including matrix i
+template <int MATS> struct FewParams {
+    FewMat mat[MATS];
+    int end[MATS];
+    int tblocks;  // token blocks (of 16 MT tokens)
+    const float *x;
+    const uint8_t *xs;
+    int64_t n, ldx, ldk;
+};
+
+// weight units and side words per row group of a 128-column step
+template <int TF> struct Few {
+    static constexpr int UPS = TF == TF_BF16 ? 4 : (TF == TF_FP8 || TF == TF_Q8) ? 2 : 1;
+    static constexpr int NS = TF == TF_BF16 ? 0 : TF == TF_MX4 ? 1 : 2;
+    static constexpr int NSA = NS ? NS : 1;
+};
+
+// A wave's activation slot (NX > 0): the words of a step in fragment order,
+// [term][k tile][k quarter][token] x 16 bytes, each quarter padded by one word
+// (two or more tokens) so that a wave's writes fall in distinct banks.
+template <int XT, int NX> struct FewSlot {
+    static constexpr int QS = NX > 1 ? NX + 1 : 1;  // words of a (k tile, quarter)
+    static constexpr int TS = 4 * QS, ES = 4 * TS;  // of a k tile, of a term
+    static constexpr int WORDS = NX > 0 ? XT * ES : 0;
+};
+
+// One step's operands of a wave in registers.
+template <int TF, int MT, int NT, int XT, int NX> struct FewSet {
+    u32x4 raw[NT][Few<TF>::UPS];
+    uint32_t side[NT][Few<TF>::NSA];
+    u32x4 xa[NX ? 1 : MT][NX ? 1 : 4][NX ? 1 : XT];
+    float2 x1;                       // NX = 1: columns 2 lane, 2 lane + 1
+    float4 xp[NX > 1 ? NX / 2 : 1];  // NX > 1: token 2 m + lane / 32, columns 4 (lane % 32) .. +4
+};
+
+// two f32 values' bf16 term; the values are left holding the remainders
+__device__ __forceinline__ uint32_t next_term(float &a, float &b) {
+    const uint32_t wd = cvt_pk_bf16(a, b);
+    a = __fsub_rn(a, u2f(wd << 16));
+    b = __fsub_rn(b, u2f(wd & 0xffff0000u));
+    return wd;
+}
+
+template <int TF, int MT, int NT, int W, int XT, int NX, int MATS>
+__global__ __launch_bounds__(64 * W) void few_kernel(FewParams<MATS> p) {
+    constexpr int UPS = Few<TF>::UPS, NS = Few<TF>::NS;
+    typedef FewSlot<XT, NX> Slot;
+    constexpr int RED = W * MT * NT * 64;
+    __shared__ u32x4 lds[W * Slot::WORDS > RED ? W * Slot::WORDS : RED];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int c16 = lane & 15, kq = lane >> 4;
+    // (row block, token block): consecutive workgroups go to the 8 XCDs in
+    // turn, so the token blocks of a row block are 8 apart (one XCD reads the
+    // row block's weights once from memory and then from its L2)
+    int rb = blockIdx.x, tb = 0;
+    if (NX == 0 && p.tblocks > 1) {
+        const int nb = p.end[MATS - 1], full = nb / 8 * 8 * p.tblocks, L = blockIdx.x;
+        if (L < full) {
+            tb = L / 8 % p.tblocks;
+            rb = L / (8 * p.tblocks) * 8 + L % 8;
+        } else {
+            const int rest = nb % 8;
+            tb = (L - full) / rest;
+            rb = nb / 8 * 8 + (L - full) % rest;
+        }
+    }
+    int mi = 0;
+#pragma unroll
+    for (int i = 0; i + 1 < MATS; i++) mi += rb >= p.end[i];
+    if (mi) rb -= p.end[mi - 1];
+    const FewMat &mat = p.mat[mi];
+    const TileView &w = mat.w;
+    const int64_t groups = (w.rows + 15) / 16, g0 = (int64_t)rb * NT, units = w.units_k, K = w.cols;
+    const int steps = (int)((units + UPS - 1) / UPS), per = (steps + W - 1) / W;
+    const int s0 = wave * per < steps ? wave * per : steps, s1 = s0 + per < steps ? s0 + per : steps;
+
+    const uint8_t *wb[NT];
+    const uint32_t *sb[NT];
+    const uint32_t woff = (uint32_t)lane * 16;
+    SideStep st{1, 0};
+    if constexpr (TF == TF_FP8 || TF == TF_INT4) st = side_step<TF>(w);
+#pragma unroll
+    for (int i = 0; i < NT; i++) {
+        const int64_t g = g0 + i < groups ? g0 + i : groups - 1;
+        wb[i] = w.codes + g * units * 1024;
+        if constexpr (NS > 0) sb[i] = w.side + side_row(w, g, lane);
+    }
+    // fragment bases of the token blocks; lanes past the tokens repeat the
+    // last one (each output row of the MFMA depends on its own token only)
+    const uint8_t *xb[MT];
+    uint32_t xo[MT];
+    if constexpr (NX == 0) {
+        const int64_t nblk = (p.n + 15) / 16;
+#pragma unroll
+        for (int m = 0; m < MT; m++) {
+            int64_t blk = (int64_t)tb * MT + m;
+            blk = blk < nblk ? blk : nblk - 1;
+            const int cnt = (int)(p.n - 16 * blk < 16 ? p.n - 16 * blk : 16);
+            xb[m] = p.xs + blk * p.ldk * XT * 1024;
+            xo[m] = (uint32_t)((kq * 16 + (c16 < cnt ? c16 : cnt - 1)) * 16);
+        }
+    }
+
+    typedef FewSet<TF, MT, NT, XT, NX> Set;
+    auto fetch = [&](Set &v, int s) __attribute__((always_inline)) {
+        if constexpr (NX == 1) {
+            const int64_t k = (int64_t)s * 128 + 2 * lane;
+            v.x1 = gload<float2>(p.x + (k < K ? k : K - 2));
+        } else if constexpr (NX > 1) {
+            const int64_t k = (int64_t)s * 128 + 4 * (lane & 31), kc = k < K ? k : K - 4;
+#pragma unroll
+            for (int m = 0; m < NX / 2; m++) {
+                const int64_t tok = 2 * m + (lane >> 5);
+                v.xp[m] = gload<float4>(p.x + (tok < p.n ? tok : p.n - 1) * p.ldx + kc);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < NT; i++) {
+#pragma unroll
+            for (int j = 0; j < UPS; j++) {
+                int64_t u = (int64_t)s * UPS + j;
+                u = u < units ? u : units - 1;
+                v.raw[i][j] = gload<u32x4>(wb[i] + u * 1024 + woff);
+                if constexpr (TF == TF_Q8) v.side[i][j] = gload<uint32_t>(sb[i] + u * 16);
+                if constexpr (TF == TF_FP8)
+                    v.side[i][j] = gload<uint32_t>(sb[i] + (st.sh >= 0 ? (uint32_t)u >> st.sh : (uint32_t)u / st.per));
+            }
+            if constexpr (TF == TF_MX4) v.side[i][0] = gload<uint32_t>(sb[i] + s);
+            if constexpr (TF == TF_INT4) {
+#pragma unroll
+                for (int j = 0; j < 2; j++) {
+                    const uint32_t u = 2u * s + j;
+                    uint32_t c = st.sh >= 0 ? u >> st.sh : u / st.per;
+                    c = c < (uint32_t)w.side_cols ? c : (uint32_t)w.side_cols - 1;  // the step's half past K
+                    v.side[i][j] = gload<uint32_t>(sb[i] + c);
+                }
+            }
+        }
+        if constexpr (NX == 0) {
+#pragma unroll
+            for (int m = 0; m < MT; m++)
+#pragma unroll
+                for (int t = 0; t < 4; t++)
+#pragma unroll
+                    for (int e = 0; e < XT; e++)
+                        v.xa[m][t][e] = gload<u32x4>(xb[m] + (((int64_t)s * 4 + t) * XT + e) * 1024 + xo[m]);
+        }
+    };
+
+    floatx4 acc[MT][NT];
+#pragma unroll
+    for (int m = 0; m < MT; m++)
+#pragma unroll
+        for (int i = 0; i < NT; i++) acc[m][i] = floatx4{0.f, 0.f, 0.f, 0.f};
+
+    u32x4 *slot = lds + wave * Slot::WORDS;
+    auto compute = [&](Set &v, int s) __attribute__((always_inline)) {
+        // the wave's own slot: its LDS accesses complete in order, no barrier
+        if constexpr (NX == 1) {
+            const bool in = (int64_t)s * 128 + 2 * lane < K;
+            float a = in ? v.x1.x : 0.f, b = in ? v.x1.y : 0.f;
+            uint32_t *d = (uint32_t *)slot + lane;  // (k tile lane / 16, quarter lane / 4 % 4, pair lane % 4)
+#pragma unroll
+            for (int e = 0; e < XT; e++) d[e * Slot::ES * 4] = next_term(a, b);
+        } else if constexpr (NX > 1) {
+            const int c = lane & 31;
+            const bool in = (int64_t)s * 128 + 4 * c < K;
+            uint2 *d = (uint2 *)(slot + (c >> 3) * Slot::TS + (c >> 1 & 3) * Slot::QS + (lane >> 5)) + (c & 1);
+#pragma unroll
+            for (int m = 0; m < NX / 2; m++) {
+                float4 a = v.xp[m];
+                if (!in) a = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+                for (int e = 0; e < XT; e++) {
+                    const uint32_t lo = next_term(a.x, a.y);
+                    d[(e * Slot::ES + 2 * m) * 2] = make_uint2(lo, next_term(a.z, a.w));
+                }
+            }
+        }
+#pragma unroll
+        for (int j = 1; j < UPS; j++)
+            if ((int64_t)s * UPS + j >= units) {  // past the matrix: zero weights
+#pragma unroll
+                for (int i = 0; i < NT; i++) {
+                    v.raw[i][j] = u32x4{0, 0, 0, 0};
+                    if constexpr (TF == TF_Q8 || TF == TF_FP8) v.side[i][j] = 0;
+                }
+            }
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            u32x4 xa[MT][XT];
+            if constexpr (NX > 0) {
+#pragma unroll
+                for (int e = 0; e < XT; e++)
+                    xa[0][e] = slot[e * Slot::ES + t * Slot::TS + kq * Slot::QS + (c16 < NX ? c16 : NX - 1)];
+            } else {
+#pragma unroll
+                for (int m = 0; m < MT; m++)
+#pragma unroll
+                    for (int e = 0; e < XT; e++) xa[m][e] = v.xa[m][t][e];
+            }
+            constexpr int TU = 4 / UPS;  // k tiles of a unit
+            const int j = t / TU;
+#pragma unroll
+            for (int i = 0; i < NT; i++) {
+                u32x4 b;
+                float ts = 1.f;
+                if constexpr (TF == TF_BF16) b = v.raw[i][j];
+                else {
+                    const u32x4 c[1] = {v.raw[i][j]};
+                    const uint32_t sd[2] = {v.side[i][UPS > 1 ? j : 0], v.side[i][UPS > 1 ? j : Few<TF>::NSA - 1]};
+                    b = decode_tile_lds<TF>(w, c, sd, t % TU, true);
+                    if constexpr (TF == TF_Q8) ts = f16_to_f32_hw((uint16_t)((sd[0] >> (16 * (t % TU))) & 0xffffu));
+                }
+#pragma unroll
+                for (int m = 0; m < MT; m++) mac<TF, XT>(acc[m][i], xa[m], b, b, ts);
+            }
+        }
+    };
+
+    if (s0 < s1) {
+        Set a, b;
+        fetch(a, s0);
+        int s = s0;
+        for (; s + 1 < s1; s += 2) {
+            fetch(b, s + 1);
+            compute(a, s);
+            fetch(a, s + 2 < s1 ? s + 2 : s1 - 1);
+            compute(b, s + 1);
+        }
+        if (s < s1) compute(a, s);
+    }
+
+    // the W slices added in wave order, a (token block, row group) tile a wave
+    floatx4 *red = (floatx4 *)lds;
+    __syncthreads();  // the slots are read: their LDS takes the sums
+#pragma unroll
+    for (int m = 0; m < MT; m++)
+#pragma unroll
+        for (int i = 0; i < NT; i++) red[(wave * MT * NT + m * NT + i) * 64 + lane] = acc[m][i];
+    __syncthreads();
+    GemmParams e{};
+    e.w.rows = w.rows;
+    e.out = mat.out;
+    e.n = p.n;
+    e.bias = mat.bias;
+    e.accumulate = mat.accumulate;
+    e.delta_b = mat.delta_b;
+    e.delta_xa = mat.delta_xa;
+    e.delta_rank = e.delta_stride = mat.delta_rank;
+    for (int q = wave; q < MT * NT; q += W) {
+        floatx4 v[1][1] = {{red[q * 64 + lane]}};
+#pragma unroll
+        for (int k = 1; k < W; k++) {
+            const floatx4 o = red[(k * MT * NT + q) * 64 + lane];
+#pragma unroll
+            for (int r = 0; r < 4; r++) v[0][0][r] = __fadd_rn(v[0][0][r], o[r]);
+        }
+        const int64_t tok[1] = {((int64_t)tb * MT + q / NT) * 16 + 4 * kq}, row[1] = {(g0 + q % NT) * 16 + c16};
+        store_block(e, tok, row, v);
+    }
+}
+
+struct FewCall {
+    const FewMat *mats;
+    int nmat;
+    const float *x;
+    int64_t ldx;
+    const void *xs;
+    int64_t ldk, n;
+    hipStream_t s;
+};
+
+template <int TF, int MT, int NT, int W, int XT, int NX, int MATS>
+void launch_mats(const FewCall &c) {
+    FewParams<MATS> p{};
+    int end = 0;
+    for (int i = 0; i < MATS; i++) {
+        if (i < c.nmat) {
+            p.mat[i] = c.mats[i];
+            end += (int)((c.mats[i].w.rows + 16 * NT - 1) / (16 * NT));
+        }
+        p.end[i] = end;
+    }
+    p.tblocks = NX ? 1 : (int)((c.n + 16 * MT - 1) / (16 * MT));
+    p.x = c.x;
+    p.xs = (const uint8_t *)c.xs;
+    p.n = c.n;
+    p.ldx = c.ldx;
+    p.ldk = c.ldk;
+    hipLaunchKernelGGL((few_kernel<TF, MT, NT, W, XT, NX, MATS>), dim3((unsigned)(end * p.tblocks)), dim3(64 * W), 0,
+                       c.s, p);
+}
+
+template <int TF, int MT, int NT, int W, int XT, int NX>
+void launch_cfg(const FewCall &c) {
+    if (c.nmat == 1) launch_mats<TF, MT, NT, W, XT, NX, 1>(c);
+    else launch_mats<TF, MT, NT, W, XT, NX, 3>(c);
+}
+
+template <int TF, int XT, int NX>
+void launch_rows(const FewCall &c, int64_t groups, int64_t steps) {
+    // 32 rows and four K slices where that gives at least 256 workgroups
+    // (14336 x 4096 on 8 tokens: MXFP4 12.0 us, 14.8 to 15.4 with 16 rows);
+    // below that 16 rows, and eight slices of more than one step each (FP8
+    // 4096 x 14336 on 8 tokens 17.4 us, 16 slices 16.6, four 24; 896 x 896
+    // 4.7, four slices 4.4)
+    if (groups >= 512) launch_cfg<TF, 1, 2, 4, XT, NX>(c);
+    else if (steps > 8) launch_cfg<TF, 1, 1, 8, XT, NX>(c);
+    else launch_cfg<TF, 1, 1, 4, XT, NX>(c);
+}
+
+template <int TF, int XT>
+void launch_tf(const FewCall &c) {
+    int64_t groups = 0;
+    for (int i = 0; i < c.nmat; i++) groups += (c.mats[i].w.rows + 15) / 16;
+    const int64_t steps = (c.mats[0].w.cols + 127) / 128, tb = (c.n + 15) / 16;
+    if (c.x) {
+        if (c.n == 1) launch_rows<TF, XT, 1>(c, groups, steps);
+        else if (c.n == 2) launch_rows<TF, XT, 2>(c, groups, steps);
+        else if (c.n <= 4) launch_rows<TF, XT, 4>(c, groups, steps);
+        else launch_rows<TF, XT, 8>(c, groups, steps);
+        return;
+    }
+    // Few row groups x token blocks: eight K slices over 16 rows (1024 x 4096
+    // on 16 tokens: FP8 8.6 us, 10.3 with four over 32). Otherwise every
+    // weight decoded feeds MT token blocks and every activation word NT row
+    // groups; the larger tiles pay once the grid still fills the CUs (4096 x
+    // 4096: MXFP4 on 48 tokens 13.0 us with 2 x 2, 15.0 with 1 x 2; on 96
+    // tokens 19.1 with 2 x 4, 20.7; 14336 x 4096 on 16 tokens 15.4 with 1 x 2,
+    // 19.6 with 2 x 2). Three-term products hold half as many again.
+    const int64_t units = groups * tb;
+    if (units <= 256 && steps > 16) launch_cfg<TF, 1, 1, 8, XT, 0>(c);
+    else if (XT == 3 || tb == 1 || units < 640) launch_cfg<TF, 1, 2, 4, XT, 0>(c);
+    else if constexpr (XT == 2) {
+        // (FP8 on 128 tokens: 14336 x 4096 55 us with 2 x 2, 66 with 2 x 4)
+        if (units < 1536 || TF == TF_FP8) launch_cfg<TF, 2, 2, 4, XT, 0>(c);
+        else if constexpr (TF != TF_FP8) launch_cfg<TF, 2, 4, 4, XT, 0>(c);
+    }
+}
+
+}  // namespace
+
+// Up to 32 tokens for every shape; above that while the product is small
+// enough that the tiled and scaled-MFMA products, which multiply at twice the
+// rate and more, lose to their split-K passes and idle CUs. The lines, in
+// tokens x rows x columns, lie where the two measured the same (us here /
+// there): bf16 4096 x 4096 on 128 tokens 22 / 26, on 256 34 / 32, 14336 x
+// 4096 on 32 33 / 42, on 48 49 / 44; INT4 4096 x 4096 on 128 23 / 32, on 256
+// 37 / 37; MXFP4 14336 x 4096 on 96 37 / 47, 4096 x 4096 on 128 22 / 49. On
+// long rows the tiled product leaves most CUs without a tile: 4096 x 14336 on
+// 128 tokens FP8 52 / 57, INT4 55 / 60, Q8_0 51 / 167; bf16 on 64 49 / 51.
+bool few_gemm_takes(const TileView &w, int64_t n, bool exact) {
+    if (!w.fast || n < 1 || n > 255 || w.cols < 4) return false;
+    const bool bf16 = w.tf == TF_BF16, mx4 = w.tf == TF_MX4, q8 = w.tf == TF_Q8;
+    if (!bf16 && !mx4 && !q8 && w.tf != TF_FP8 && w.tf != TF_INT4) return false;
+    if (n <= 32) return true;
+    if (exact) return false;
+    const double work = (double)n * w.rows * w.cols;
+    const bool long_k = w.cols >= 8192 && w.rows <= 4096;
+    if (mx4) return work <= (long_k ? 1.5e10 : 5.7e9);
+    if (q8) return work <= (long_k ? 1.5e10 : n > 64 ? 4.4e9 : 2.6e9);
+    return work <= (long_k ? (bf16 ? 3.8e9 : 7.6e9) : 2.6e9);
+}
+
+bool few_reads_rows(const TileView &w, int64_t n, const float *x, int64_t ldx) {
+    return n <= 8 && w.cols % 4 == 0 && ldx % 4 == 0 && ((uintptr_t)x & 15) == 0;
+}
+
+void launch_few_gemm(const FewMat *mats, int nmat, const float *x, int64_t ldx, const void *xs, int64_t ldk, int64_t n,
+                     int xt, hipStream_t s) {
+    const FewCall c{mats, nmat, x, ldx, xs, ldk, n, s};
+    DITCH_CHECK(nmat >= 1 && nmat <= 3 && n >= 1, DITCH_INVALID_ARGUMENT, "few-token product: 1 to 3 matrices");
+    for (int i = 0; i < nmat; i++)
+        DITCH_CHECK(mats[i].w.tf == mats[0].w.tf && mats[i].w.cols == mats[0].w.cols && mats[i].w.fast,
+                    DITCH_INVALID_ARGUMENT, "few-token product: matrices of one format and width");
+    DITCH_CHECK(x ? few_reads_rows(mats[0].w, n, x, ldx) : xs && ldk >= few_ldk(mats[0].w), DITCH_INVALID_ARGUMENT,
+                "few-token product: activations not in a form it reads");
+#define FEW_TF(TF) \
+    case TF: xt == 3 ? launch_tf<TF, 3>(c) : launch_tf<TF, 2>(c); break;
+    switch (mats[0].w.tf) {
+        FEW_TF(TF_BF16)
+        FEW_TF(TF_Q8)
+        FEW_TF(TF_FP8)
+        FEW_TF(TF_MX4)
+        FEW_TF(TF_INT4)
+    default: throw Error{DITCH_UNSUPPORTED, "few-token product: format"};
+    }
+#undef FEW_TF
+    DITCH_TRY_HIP(hipGetLastError());
+}
+
+}  // namespace ditch

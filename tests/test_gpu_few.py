@@ -1,0 +1,75 @@
+"""The few-token product (csrc/gemm_few.hip) against the oracle at the edges of
+its dispatch and tiles: every format, up to 8 tokens from f32 rows and more
+from fragments, K of less than one 128-column step, of partial units and steps
+and of K slices of unequal length, rows that leave a row group and a row block
+part empty, the grids on both sides of each tile choice, and the last token
+count it takes."""
+import numpy as np
+import pytest
+
+import weights_gen as wg
+from ditch_amd import hipmem
+from test_gpu_kernels import TOL_MATMUL, dequant_f32, split_bound
+
+pytestmark = pytest.mark.gpu
+
+# kind, n, rows, cols
+CASES = [
+    ("bf16", 1, 17, 36), ("bf16", 3, 33, 132), ("bf16", 4, 40, 30), ("bf16", 8, 8208, 160),
+    ("bf16", 9, 50, 96), ("bf16", 16, 64, 4128), ("bf16", 49, 4096, 288), ("bf16", 255, 100, 160),
+    ("fp8", 1, 520, 4160), ("fp8", 2, 31, 64), ("fp8", 7, 130, 1216), ("fp8", 12, 48, 4160),
+    ("fp8", 33, 3000, 320), ("fp8", 200, 1100, 128),
+    ("mxfp4", 1, 48, 160), ("mxfp4", 5, 130, 4256), ("mxfp4", 8, 8200, 128), ("mxfp4", 17, 24, 4096),
+    ("mxfp4", 31, 700, 544), ("mxfp4", 100, 4096, 256), ("mxfp4", 200, 72, 640),
+    ("int4", 1, 130, 192), ("int4", 4, 72, 4224), ("int4", 8, 16, 128), ("int4", 10, 260, 2240),
+    ("int4", 48, 4000, 256), ("int4", 130, 72, 1024),
+    ("q8_0", 2, 8208, 96), ("q8_0", 6, 70, 4128), ("q8_0", 15, 33, 1056), ("q8_0", 64, 3080, 64), ("q8_0", 129, 40, 416),
+]
+
+
+@pytest.mark.parametrize("kind,n,rows,cols", CASES)
+def test_few_token_product(dev, ref, kind, n, rows, cols):
+    """Two-term products with bias and accumulate on a resident tensor."""
+    rng = np.random.default_rng(n * 7919 + rows + cols)
+    w = wg.make(kind, rows, cols, rng)
+    x = rng.standard_normal((n, cols)).astype(np.float32)
+    bias = rng.standard_normal(rows).astype(np.float32)
+    prior = rng.standard_normal((n, rows)).astype(np.float32)
+    t = dev.upload(w)
+    try:
+        bx, bb, bo = (hipmem.Buffer.from_array(a) for a in (x, bias, prior))
+        t.matmul_device(bo.ptr, bx.ptr, n, d_bias=bb.ptr, accumulate=True)
+        dev.sync()
+        got = bo.download(np.float32, (n, rows))
+    finally:
+        t.free()
+    want = prior.astype(np.float64) + ref.matmulT(x, w).astype(np.float64) + bias
+    # the activations' two terms: 2^-18 of each (split_bound's bf16 form, four times it)
+    bound = split_bound("bf16", x, dequant_f32(ref, w))
+    bad = np.abs(got - want) > TOL_MATMUL["atol"] + TOL_MATMUL["rtol"] * np.abs(want) + bound
+    assert not bad.any(), f"{bad.sum()} of {bad.size} outside the bound"
+
+
+@pytest.mark.parametrize("kind", ["bf16", "fp8", "mxfp4", "int4", "q8_0"])
+@pytest.mark.parametrize("n", [1, 6, 16, 32])
+def test_few_token_exact_product(dev, ref, kind, n):
+    """Three-term products (the VTable entry) at the reference's tolerance."""
+    rng = np.random.default_rng(n)
+    w = wg.make(kind, 600, 1216, rng)
+    x = rng.standard_normal((n, 1216)).astype(np.float32)
+    got, want = dev.matmulT(x, w), ref.matmulT(x, w)
+    bad = np.abs(got - want) > TOL_MATMUL["atol"] + TOL_MATMUL["rtol"] * np.abs(want)
+    assert not bad.any()
+
+
+@pytest.mark.parametrize("n", [6, 20])
+def test_non_finite_activations_stay_in_their_token(dev, ref, n):
+    rng = np.random.default_rng(3)
+    w = wg.make("fp8", 96, 320, rng)
+    x = rng.standard_normal((n, 320)).astype(np.float32)
+    clean = dev.matmulT(x, w)
+    x[2, 5], x[4, 300] = np.inf, np.nan
+    got = dev.matmulT(x, w)
+    others = [i for i in range(n) if i not in (2, 4)]
+    assert not np.isfinite(got[[2, 4]]).any()
+    np.testing.assert_array_equal(got[others], clean[others])
