@@ -42,6 +42,7 @@ EXTRA = {"gemm_tile.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form", "-mllvm", "-disab
          "gemv.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form", "-mllvm", "-pragma-unroll-threshold=1000000"],
          "attention.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
          "gemm_few.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+         "gemm_f32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form", "-mllvm", "-disable-machine-sink"],
          "gemm_wide.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 

@@ -4,20 +4,16 @@
 //
 // The products run on the fp32 MFMA (v_mfma_f32_16x16x4_f32), which forms
 // every product exactly; it issues a 16 x 16 x 4 step in 32 cycles, so the
-// product is MFMA-bound and what matters is keeping every SIMD busy:
+// product is MFMA-bound and what matters is keeping every SIMD busy. Eight
+// rank-4 steps per 16 x 16 tile and 32-column unit pair register s of A with
+// register s of B (k = 8 (l / 16) + s): the tile layout holds the lane's 8
+// weights of a unit together, and an activation row's 8 columns are two
+// 16-byte words.
 //
-//   - a wave owns 64 tokens x 32 rows (4 x 2 tiles, 32 accumulator VGPRs),
-//     and takes its operands straight from memory into registers: per
-//     32-column unit the lane's 8 weights of each row group (the tile layout:
-//     row l % 16, columns 8 (l / 16) .. +8) and the same 8 columns of each
-//     of its tokens' activation rows; eight rank-4 steps per tile and unit
-//     pair register s of A with register s of B (k = 8 (l / 16) + s);
-//   - the next unit's operands are requested before a unit's products (two
-//     register sets, alternating);
-//   - a workgroup is 4 waves: 4 / KS tiles, each over KS k slices whose sums
-//     are added in slice order through LDS; KS grows until the grid gives
-//     every SIMD four waves (the attention and small projections of a 0.5B
-//     model have only a few hundred 64 x 32 tiles).
+//   - rows of whole units (K a multiple of 32, 16-byte aligned):
+//     f32_tile_kernel, operands staged in LDS by DMA;
+//   - other rows: f32_gemm_kernel, operands loaded to registers with bounds
+//     on every column.
 #include "gemm_f32.h"
 
 namespace ditch {
@@ -43,10 +39,10 @@ __device__ __forceinline__ void f32_weights(const uint8_t *unit, int lane, float
     }
 }
 
-// VEC: K a multiple of 32 and rows 16-byte aligned: every activation load is
-// two unguarded float4 (no branch in the loop, so the next unit's loads stay
-// in flight across the current unit's products)
-template <int TF, int KS, bool VEC>
+// A wave owns 64 tokens x 32 rows (4 x 2 tiles) and takes its operands straight
+// from memory into two alternating register sets; a workgroup is 4 / KS tiles,
+// each over KS k slices whose sums are added in slice order through LDS.
+template <int TF, int KS>
 __global__ __launch_bounds__(256) void f32_gemm_kernel(GemmParams p, int tiles_m, int tiles) {
     constexpr int TW = 4 / KS;  // tiles per workgroup
     constexpr int UB = TF == TF_F32 ? 2048 : 1024;
@@ -83,14 +79,8 @@ __global__ __launch_bounds__(256) void f32_gemm_kernel(GemmParams p, int tiles_m
         const int64_t k0 = u * 32 + 8 * q;
 #pragma unroll
         for (int m = 0; m < FM; m++) {
-            if constexpr (VEC) {
-                const float4 lo = *(const float4 *)(xr[m] + k0), hi = *(const float4 *)(xr[m] + k0 + 4);
-                a[m][0] = lo.x; a[m][1] = lo.y; a[m][2] = lo.z; a[m][3] = lo.w;
-                a[m][4] = hi.x; a[m][5] = hi.y; a[m][6] = hi.z; a[m][7] = hi.w;
-            } else {
 #pragma unroll
-                for (int j = 0; j < 8; j++) a[m][j] = k0 + j < K ? xr[m][k0 + j] : 0.f;
-            }
+            for (int j = 0; j < 8; j++) a[m][j] = k0 + j < K ? xr[m][k0 + j] : 0.f;
         }
     };
 
@@ -120,9 +110,6 @@ __global__ __launch_bounds__(256) void f32_gemm_kernel(GemmParams p, int tiles_m
         };
         load(u0, a0, b0);
         int64_t u = u0;
-        // no branch inside the loop: every wait is a fixed count of loads
-        // (pinning each set's loads ahead of the other set's products with
-        // scheduling barriers measured 30-40 % slower)
         for (; u + 1 < u1; u += 2) {
             load(u + 1, a1, b1);
             products(a0, b0);
@@ -159,7 +146,209 @@ __global__ __launch_bounds__(256) void f32_gemm_kernel(GemmParams p, int tiles_m
     store_block(p, tb, rw, acc);
 }
 
-template <int TF, bool VEC>
+// ---------------------------------------------------------------------------
+// Rows of whole units: every operand travels global -> LDS by DMA, a stage of
+// 32 columns ahead: weight units as the tile layout holds them, eight
+// activation rows' 128 bytes a copy, so that its lanes read whole lines (the
+// 16-byte words of row r permuted by xor r % 8, so that the reads of 8 rows
+// fall in distinct banks; with 16-byte pieces of 16 rows a copy, 10 % slower).
+// Loaded to registers instead, as above, a unit's operands are sunk by the
+// compiler to a few MFMAs before their use.
+//
+// A workgroup is KS slices of K times WG x WG waves of 32 x 32 outputs each.
+// While a unit is multiplied from registers (32 MFMAs, 1024 cycles), the next
+// one's operands are read from LDS and the copies of the one after it run.
+// WG = 1: a wave's pieces are its own and it waits for its copies alone. The
+// slices' tiles are added in slice order through LDS.
+//
+// OCC waves a SIMD at most: more of them finish their MFMAs together and then
+// wait together (4096 x 4096 on 2048 tokens: 505 us = 136 TFLOP/s at two, 579
+// at three, 649 at four and five; the register-staged kernel 667; the fp32
+// matrix peak is 157 TFLOP/s).
+typedef __attribute__((address_space(3))) void lds_void;
+
+template <int TF, int WG, int KS, int OCC>
+__global__ __launch_bounds__(64 * WG * WG * KS) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void f32_tile_kernel(
+    GemmParams p, int tiles_m, int tiles) {
+    constexpr int NWS = WG * WG, NW = NWS * KS;       // waves of a slice, of the workgroup
+    constexpr int AP = 4 * WG;                        // 1 KiB activation pieces of a slice's unit
+    constexpr int BH = TF == TF_F32 ? 2 : 1;          // pieces of a weight unit of 16 rows
+    constexpr int BP = 2 * WG * BH;
+    constexpr int CA = AP / NWS, CB = (BP + NWS - 1) / NWS;  // a wave's copies
+    constexpr int ST = KS * (AP + BP) * 64;           // 16-byte words of a stage
+    __shared__ u32x4 buf0[ST], buf1[ST];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int ks = wave / NWS, ws = wave % NWS, wm = ws / WG, wn = ws % WG, q = lane >> 4;
+    // each XCD a contiguous run of tiles, token blocks fastest: the run's
+    // weights and the activations are read from its own L2
+    const int per = tiles / 8, L = blockIdx.x, tile = L < per * 8 ? L % 8 * per + L / 8 : L;
+    const int tm = tile % tiles_m, tn = tile / tiles_m;
+    const TileView &w = p.w;
+    const int U = (int)w.units_k, groups = (int)((w.rows + 15) / 16);
+    const int nu = (U + KS - 1) / KS, u0 = ks * nu, u1 = u0 + nu < U ? u0 + nu : U;  // u0 >= u1: an empty slice
+
+    // sources of this wave's copies at unit 0 (tokens and rows past the end
+    // repeat the last one: their outputs are not stored)
+    const char *asrc[CA];
+#pragma unroll
+    for (int j = 0; j < CA; j++) {
+        int64_t tok = (int64_t)tm * (32 * WG) + (ws * CA + j) * 8 + (lane >> 3);
+        tok = tok < p.n ? tok : p.n - 1;
+        asrc[j] = (const char *)(p.x + (p.row_index ? (int64_t)p.row_index[tok] : tok) * p.ldx +
+                                 4 * ((lane & 7) ^ (lane >> 3)));
+    }
+    const char *bsrc[CB];
+#pragma unroll
+    for (int j = 0; j < CB; j++) {
+        int g = tn * (2 * WG) + (ws * CB + j) / BH;
+        g = g < groups ? g : groups - 1;
+        bsrc[j] = (const char *)w.codes + ((int64_t)g * U * BH + (ws * CB + j) % BH) * 1024 + lane * 16;
+    }
+    u32x4 *const mine0 = buf0 + ks * (AP + BP) * 64, *const mine1 = buf1 + ks * (AP + BP) * 64;
+    auto copy = [&](int u, u32x4 *dst) __attribute__((always_inline)) {
+        const int64_t uu = u < U ? u : U - 1;
+#pragma unroll
+        for (int j = 0; j < CA; j++)
+            __builtin_amdgcn_global_load_lds((const void *)(asrc[j] + uu * 128),
+                                             (lds_void *)&dst[(ws * CA + j) * 64], 16, 0, 0);
+#pragma unroll
+        for (int j = 0; j < CB; j++)
+            if (BP % NWS == 0 || ws * CB + j < BP)
+                __builtin_amdgcn_global_load_lds((const void *)(bsrc[j] + uu * BH * 1024),
+                                                 (lds_void *)&dst[(AP + ws * CB + j) * 64], 16, 0, 0);
+    };
+    // this wave's copies have landed and its reads returned (and, sharing the
+    // buffers, everyone's)
+    auto landed = [&]() __attribute__((always_inline)) {
+        if constexpr (WG > 1) __syncthreads();
+        else {
+            __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
+            __builtin_amdgcn_wave_barrier();
+        }
+    };
+
+    floatx4 acc[2][2];
+#pragma unroll
+    for (int m = 0; m < 2; m++)
+#pragma unroll
+        for (int i = 0; i < 2; i++) acc[m][i] = floatx4{0.f, 0.f, 0.f, 0.f};
+    struct Ops {
+        float a[2][8], b[2][8];
+    };
+    auto read = [&](Ops &o, const u32x4 *src) __attribute__((always_inline)) {
+#pragma unroll
+        for (int m = 0; m < 2; m++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const u32x4 v = src[(wm * 2 + m) * 128 + (lane & 15) * 8 + ((2 * q + h) ^ (lane & 7))];
+#pragma unroll
+                for (int j = 0; j < 4; j++) o.a[m][4 * h + j] = u2f(v[j]);
+            }
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const u32x4 *bp = src + (AP + (wn * 2 + i) * BH) * 64 + lane;
+            if constexpr (TF == TF_F32) {
+                const u32x4 lo = bp[0], hi = bp[64];
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    o.b[i][j] = u2f(lo[j]);
+                    o.b[i][4 + j] = u2f(hi[j]);
+                }
+            } else {
+                const u32x4 v = bp[0];
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    o.b[i][2 * j] = f16_to_f32_hw((uint16_t)(v[j] & 0xffffu));
+                    o.b[i][2 * j + 1] = f16_to_f32_hw((uint16_t)(v[j] >> 16));
+                }
+            }
+        }
+    };
+    auto products = [&](const Ops &o) __attribute__((always_inline)) {
+#pragma unroll
+        for (int s = 0; s < 8; s++)
+#pragma unroll
+            for (int m = 0; m < 2; m++)
+#pragma unroll
+                for (int i = 0; i < 2; i++) acc[m][i] = mfma_f32(o.a[m][s], o.b[i][s], acc[m][i]);
+    };
+
+    // every slice runs nu units (past its own: copied again, not multiplied)
+    Ops even, odd;
+    copy(u0, mine0);
+    landed();
+    read(even, mine0);
+    if (nu > 1) copy(u0 + 1, mine1);
+    for (int s = 0; s < nu; s += 2) {
+        landed();
+        if (s + 1 < nu) read(odd, mine1);
+        if (s + 2 < nu) copy(u0 + s + 2, mine0);
+        if (u0 + s < u1) products(even);
+        if (s + 1 >= nu) break;
+        landed();
+        if (s + 2 < nu) read(even, mine0);
+        if (s + 3 < nu) copy(u0 + s + 3, mine1);
+        if (u0 + s + 1 < u1) products(odd);
+    }
+
+    if constexpr (KS == 1) {
+        const int64_t t0 = (int64_t)tm * (32 * WG) + wm * 32, r0 = (int64_t)tn * (32 * WG) + wn * 32;
+        const int64_t tb[2] = {t0 + 4 * q, t0 + 16 + 4 * q}, rw[2] = {r0 + (lane & 15), r0 + 16 + (lane & 15)};
+        store_block(p, tb, rw, acc);
+    } else {
+        constexpr int NT = 4 * NWS;  // 16 x 16 tiles of the workgroup: [slice][wave of the slice][m, i]
+        // the sums in the first stage buffer where it holds them
+        constexpr bool FITS = NT * KS * 64 <= ST;
+        __shared__ floatx4 own[FITS ? 1 : NT * KS * 64];
+        floatx4 *red = FITS ? (floatx4 *)buf0 : own;
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < 2; m++)
+#pragma unroll
+            for (int i = 0; i < 2; i++) red[((ks * NWS + ws) * 4 + m * 2 + i) * 64 + lane] = acc[m][i];
+        __syncthreads();
+        for (int t = wave; t < NT; t += NW) {
+            floatx4 v[1][1] = {{red[t * 64 + lane]}};
+#pragma unroll
+            for (int k = 1; k < KS; k++) {
+                const floatx4 o = red[(k * NT + t) * 64 + lane];
+#pragma unroll
+                for (int r = 0; r < 4; r++) v[0][0][r] = __fadd_rn(v[0][0][r], o[r]);
+            }
+            const int wt = t / 4, m = t / 2 % 2, i = t % 2;
+            const int64_t tb[1] = {(int64_t)tm * (32 * WG) + (wt / WG) * 32 + 16 * m + 4 * q};
+            const int64_t rw[1] = {(int64_t)tn * (32 * WG) + (wt % WG) * 32 + 16 * i + (lane & 15)};
+            store_block(p, tb, rw, v);
+        }
+    }
+}
+
+template <int TF, int WG, int KS, int OCC>
+void launch_tiles(const GemmParams &p, int tiles_m, int64_t tiles, hipStream_t s) {
+    hipLaunchKernelGGL((f32_tile_kernel<TF, WG, KS, OCC>), dim3((unsigned)tiles), dim3(64 * WG * WG * KS), 0, s, p,
+                       tiles_m, (int)tiles);
+}
+
+// 64 x 64 tiles in one slice (87 % of the fp32 matrix rate over full rounds of
+// the 256 CUs, once there are enough for two waves a SIMD) or, up to one round,
+// in two slices (76 %); 32 x 32 tiles in four slices (63 %). The cheapest by
+// rounds over rate, in units of a 32 x 32 tile a CU. Measured (us, 64 x 64 in
+// one or two slices / 32 x 32): 896 x 4864 on 512 tokens 87 / 50, on 1024 85 /
+// 97; 4864 x 896 on 256 32 / 32, on 1024 78 / 112; 4096 x 4096 on 64 73 / 23,
+// on 256 75 / 81, on 512 128 / 161.
+template <int TF>
+void launch_staged(const GemmParams &p, hipStream_t s) {
+    const int64_t m64 = (p.n + 63) / 64, t64 = m64 * ((p.w.rows + 63) / 64);
+    const int64_t m32 = (p.n + 31) / 32, t32 = m32 * ((p.w.rows + 31) / 32);
+    const double big = t64 > 256 ? (double)((t64 + 255) / 256) * 4 / 0.87 : 4 / 0.76;
+    const double small = (double)((t32 + 255) / 256) / 0.63;
+    if (small < big) launch_tiles<TF, 1, 4, 1>(p, (int)m32, t32, s);
+    else if (t64 > 256) launch_tiles<TF, 2, 1, 2>(p, (int)m64, t64, s);
+    else launch_tiles<TF, 2, 2, 2>(p, (int)m64, t64, s);
+}
+
+// rows with bounds on every column
+template <int TF>
 void launch_tf(const GemmParams &p, hipStream_t s) {
     const int64_t groups = (p.w.rows + 15) / 16;
     const int tiles_m = (int)((p.n + 63) / 64), tiles = tiles_m * (int)((groups + FN - 1) / FN);
@@ -168,9 +357,9 @@ void launch_tf(const GemmParams &p, hipStream_t s) {
     int ks = 1;
     while (ks < 4 && (int64_t)tiles * ks < 4096 && p.w.units_k / (2 * ks) >= 2) ks *= 2;
     const dim3 grid((unsigned)((tiles + 4 / ks - 1) / (4 / ks)));
-    if (ks == 1) hipLaunchKernelGGL((f32_gemm_kernel<TF, 1, VEC>), grid, dim3(256), 0, s, p, tiles_m, tiles);
-    else if (ks == 2) hipLaunchKernelGGL((f32_gemm_kernel<TF, 2, VEC>), grid, dim3(256), 0, s, p, tiles_m, tiles);
-    else hipLaunchKernelGGL((f32_gemm_kernel<TF, 4, VEC>), grid, dim3(256), 0, s, p, tiles_m, tiles);
+    if (ks == 1) hipLaunchKernelGGL((f32_gemm_kernel<TF, 1>), grid, dim3(256), 0, s, p, tiles_m, tiles);
+    else if (ks == 2) hipLaunchKernelGGL((f32_gemm_kernel<TF, 2>), grid, dim3(256), 0, s, p, tiles_m, tiles);
+    else hipLaunchKernelGGL((f32_gemm_kernel<TF, 4>), grid, dim3(256), 0, s, p, tiles_m, tiles);
 }
 
 }  // namespace
@@ -180,8 +369,8 @@ bool f32_gemm_takes(const TileView &w, int64_t n) { return (w.tf == TF_F32 || w.
 void launch_f32_gemm(const GemmParams &p, hipStream_t s) {
     DITCH_CHECK(f32_gemm_takes(p.w, p.n) && !p.segs, DITCH_INVALID_ARGUMENT, "f32 product: weight or batch not taken");
     const bool vec = p.w.cols % 32 == 0 && p.ldx % 4 == 0 && ((uintptr_t)p.x & 15) == 0;
-    if (p.w.tf == TF_F32) vec ? launch_tf<TF_F32, true>(p, s) : launch_tf<TF_F32, false>(p, s);
-    else vec ? launch_tf<TF_F16, true>(p, s) : launch_tf<TF_F16, false>(p, s);
+    if (vec) p.w.tf == TF_F32 ? launch_staged<TF_F32>(p, s) : launch_staged<TF_F16>(p, s);
+    else p.w.tf == TF_F32 ? launch_tf<TF_F32>(p, s) : launch_tf<TF_F16>(p, s);
     DITCH_TRY_HIP(hipGetLastError());
 }
 

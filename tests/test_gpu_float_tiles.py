@@ -1,0 +1,46 @@
+"""Products on f32 / f16 weights above 16 tokens (csrc/gemm_f32.hip) at the
+edges of the staged tiles: each tile and slice count of the dispatch, K of one
+unit (slices without any) and of slices of unequal length, ragged rows and
+tokens, rows that are not whole units, and a gathered non-finite activation
+that must stay in its token."""
+import numpy as np
+import pytest
+
+import weights_gen as wg
+from ditch_amd import hipmem
+from test_gpu_kernels import TOL_MATMUL, close
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("kind", ["f32", "f16"])
+@pytest.mark.parametrize("n,rows,cols", [(17, 33, 32), (40, 130, 160), (100, 1000, 96), (1024, 896, 160),
+                                         (1100, 950, 96), (1090, 1030, 32), (50, 70, 72)])
+def test_float_tiles(dev, ref, kind, n, rows, cols):
+    rng = np.random.default_rng(n + rows + cols)
+    w = wg.float_random(kind, rows, cols, rng)
+    x = rng.standard_normal((n, cols)).astype(np.float32)
+    bias = rng.standard_normal(rows).astype(np.float32)
+    prior = rng.standard_normal((n, rows)).astype(np.float32)
+    t = dev.upload(w)
+    try:
+        bx, bb, bo = (hipmem.Buffer.from_array(a) for a in (x, bias, prior))
+        t.matmul_device(bo.ptr, bx.ptr, n, d_bias=bb.ptr, accumulate=True)
+        dev.sync()
+        got = bo.download(np.float32, (n, rows))
+    finally:
+        t.free()
+    close(got, prior.astype(np.float64) + ref.matmulT(x, w).astype(np.float64) + bias, **TOL_MATMUL)
+
+
+def test_infinite_activation_keeps_its_sign(dev, ref):
+    """Exact products: an infinite activation gives infinities in its own
+    token's outputs, as f32 multiply-adds do, and nothing elsewhere."""
+    rng = np.random.default_rng(1)
+    w = wg.float_random("f32", 100, 96, rng)
+    x = rng.standard_normal((40, 96)).astype(np.float32)
+    x[7, 5] = np.inf
+    got, want = dev.matmulT(x, w), ref.matmulT(x, w)
+    np.testing.assert_array_equal(np.isinf(got), np.isinf(want))
+    assert np.isinf(want[7]).all() and (np.sign(got[7]) == np.sign(want[7])).all()
+    close(np.delete(got, 7, 0), np.delete(want, 7, 0), **TOL_MATMUL)
