@@ -147,36 +147,39 @@ __global__ __launch_bounds__(256) void f32_gemm_kernel(GemmParams p, int tiles_m
 }
 
 // ---------------------------------------------------------------------------
-// Rows of whole units: every operand travels global -> LDS by DMA, a stage of
-// 32 columns ahead: weight units as the tile layout holds them, eight
-// activation rows' 128 bytes a copy, so that its lanes read whole lines (the
-// 16-byte words of row r permuted by xor r % 8, so that the reads of 8 rows
-// fall in distinct banks; with 16-byte pieces of 16 rows a copy, 10 % slower).
-// Loaded to registers instead, as above, a unit's operands are sunk by the
-// compiler to a few MFMAs before their use.
+// Rows of whole units: every operand travels global -> LDS by DMA, three
+// stages of 32 columns ahead: weight units as the tile layout holds them,
+// eight activation rows' 128 bytes a copy, so that its lanes read whole lines
+// (the 16-byte words of row r permuted by xor r % 8, so that the reads of 8
+// rows fall in distinct banks; 16-byte pieces of 16 rows a copy were 10 %
+// slower). Loaded to registers instead, as above, a unit's operands are sunk
+// by the compiler to a few MFMAs before their use.
 //
 // A workgroup is KS slices of K times WG x WG waves of 32 x 32 outputs each.
 // While a unit is multiplied from registers (32 MFMAs, 1024 cycles), the next
-// one's operands are read from LDS and the copies of the one after it run.
-// WG = 1: a wave's pieces are its own and it waits for its copies alone. The
-// slices' tiles are added in slice order through LDS.
+// one's operands are read from LDS and the copies of the three after it run
+// (one stage ahead, the first read of a weight from memory still showed: the
+// f32 forward of 24 layers, 16 x 64 tokens, 9.48 ms against 8.70). WG = 1: a
+// wave's pieces are its own and it waits for its copies alone. The slices'
+// tiles are added in slice order through LDS.
 //
-// OCC waves a SIMD at most: more of them finish their MFMAs together and then
-// wait together (4096 x 4096 on 2048 tokens: 505 us = 136 TFLOP/s at two, 579
-// at three, 649 at four and five; the register-staged kernel 667; the fp32
-// matrix peak is 157 TFLOP/s).
+// The four stage buffers leave two waves a SIMD (one at WG = 1), which is also
+// the fastest: more finish their MFMAs together and then wait together (4096 x
+// 4096 on 2048 tokens with two stage buffers: 505 us at two waves, 579 at
+// three, 649 at four and five; the register-staged kernel 667).
+// MFMA-bound: 4096 x 4096 on 2048 tokens 534 us = 129 TFLOP/s of the 157 of
+// the fp32 matrix cores; 4864 x 896 on 1024 tokens 104 -> 79 us.
 typedef __attribute__((address_space(3))) void lds_void;
 
-template <int TF, int WG, int KS, int OCC>
-__global__ __launch_bounds__(64 * WG * WG * KS) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void f32_tile_kernel(
-    GemmParams p, int tiles_m, int tiles) {
+template <int TF, int WG, int KS>
+__global__ __launch_bounds__(64 * WG * WG * KS) void f32_tile_kernel(GemmParams p, int tiles_m, int tiles) {
     constexpr int NWS = WG * WG, NW = NWS * KS;       // waves of a slice, of the workgroup
     constexpr int AP = 4 * WG;                        // 1 KiB activation pieces of a slice's unit
     constexpr int BH = TF == TF_F32 ? 2 : 1;          // pieces of a weight unit of 16 rows
     constexpr int BP = 2 * WG * BH;
-    constexpr int CA = AP / NWS, CB = (BP + NWS - 1) / NWS;  // a wave's copies
+    constexpr int CA = AP / NWS, CB = BP / NWS;  // a wave's copies
     constexpr int ST = KS * (AP + BP) * 64;           // 16-byte words of a stage
-    __shared__ u32x4 buf0[ST], buf1[ST];
+    __shared__ u32x4 buf0[ST], buf1[ST], buf2[ST], buf3[ST];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int ks = wave / NWS, ws = wave % NWS, wm = ws / WG, wn = ws % WG, q = lane >> 4;
     // each XCD a contiguous run of tiles, token blocks fastest: the run's
@@ -204,27 +207,26 @@ __global__ __launch_bounds__(64 * WG * WG * KS) __attribute__((amdgpu_waves_per_
         g = g < groups ? g : groups - 1;
         bsrc[j] = (const char *)w.codes + ((int64_t)g * U * BH + (ws * CB + j) % BH) * 1024 + lane * 16;
     }
-    u32x4 *const mine0 = buf0 + ks * (AP + BP) * 64, *const mine1 = buf1 + ks * (AP + BP) * 64;
-    auto copy = [&](int u, u32x4 *dst) __attribute__((always_inline)) {
+    const int mine = ks * (AP + BP) * 64;  // the slice's part of a stage
+    auto copy = [&](int u, u32x4 *stage) __attribute__((always_inline)) {
         const int64_t uu = u < U ? u : U - 1;
+        u32x4 *dst = stage + mine;
 #pragma unroll
         for (int j = 0; j < CA; j++)
             __builtin_amdgcn_global_load_lds((const void *)(asrc[j] + uu * 128),
                                              (lds_void *)&dst[(ws * CA + j) * 64], 16, 0, 0);
 #pragma unroll
         for (int j = 0; j < CB; j++)
-            if (BP % NWS == 0 || ws * CB + j < BP)
-                __builtin_amdgcn_global_load_lds((const void *)(bsrc[j] + uu * BH * 1024),
-                                                 (lds_void *)&dst[(AP + ws * CB + j) * 64], 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((const void *)(bsrc[j] + uu * BH * 1024),
+                                             (lds_void *)&dst[(AP + ws * CB + j) * 64], 16, 0, 0);
     };
-    // this wave's copies have landed and its reads returned (and, sharing the
-    // buffers, everyone's)
+    // the copies of all stages but the newest have landed, and the reads of
+    // the stages before are done (sharing the buffers, everyone's)
+    static_assert(AP % NWS == 0 && BP % NWS == 0 && CA + CB < 16, "copies split evenly, counted by vmcnt");
     auto landed = [&]() __attribute__((always_inline)) {
-        if constexpr (WG > 1) __syncthreads();
-        else {
-            __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
-            __builtin_amdgcn_wave_barrier();
-        }
+        __builtin_amdgcn_s_waitcnt(0x70 | (CA + CB));  // vmcnt(copies of a stage) lgkmcnt(0)
+        if constexpr (WG > 1) __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
     };
 
     floatx4 acc[2][2];
@@ -235,7 +237,8 @@ __global__ __launch_bounds__(64 * WG * WG * KS) __attribute__((amdgpu_waves_per_
     struct Ops {
         float a[2][8], b[2][8];
     };
-    auto read = [&](Ops &o, const u32x4 *src) __attribute__((always_inline)) {
+    auto read = [&](Ops &o, const u32x4 *stage) __attribute__((always_inline)) {
+        const u32x4 *src = stage + mine;
 #pragma unroll
         for (int m = 0; m < 2; m++)
 #pragma unroll
@@ -273,23 +276,35 @@ __global__ __launch_bounds__(64 * WG * WG * KS) __attribute__((amdgpu_waves_per_
                 for (int i = 0; i < 2; i++) acc[m][i] = mfma_f32(o.a[m][s], o.b[i][s], acc[m][i]);
     };
 
-    // every slice runs nu units (past its own: copied again, not multiplied)
+    // every slice runs nu units (past its own: copied again, not multiplied;
+    // past nu: copied and never read, so that the wait count stays the same)
     Ops even, odd;
-    copy(u0, mine0);
+    copy(u0, buf0);
+    copy(u0 + 1, buf1);
     landed();
-    read(even, mine0);
-    if (nu > 1) copy(u0 + 1, mine1);
-    for (int s = 0; s < nu; s += 2) {
-        landed();
-        if (s + 1 < nu) read(odd, mine1);
-        if (s + 2 < nu) copy(u0 + s + 2, mine0);
-        if (u0 + s < u1) products(even);
-        if (s + 1 >= nu) break;
-        landed();
-        if (s + 2 < nu) read(even, mine0);
-        if (s + 3 < nu) copy(u0 + s + 3, mine1);
-        if (u0 + s + 1 < u1) products(odd);
+    read(even, buf0);
+    copy(u0 + 2, buf2);
+    auto step = [&](int s, const Ops &cur, Ops &next, u32x4 *nbuf, u32x4 *cbuf, bool own) __attribute__((always_inline)) {
+        landed();                  // stage s + 1
+        read(next, nbuf);
+        copy(u0 + s + 3, cbuf);    // into the buffer of stage s - 1
+        if (own || u0 + s < u1) products(cur);
+    };
+    const int common = U - (KS - 1) * nu;  // units that every slice has (the last one's)
+    int s = 0;
+    for (; s + 4 <= common; s += 4) {  // no branch inside: every wait is a count
+        step(s, even, odd, buf1, buf3, true);
+        step(s + 1, odd, even, buf2, buf0, true);
+        step(s + 2, even, odd, buf3, buf1, true);
+        step(s + 3, odd, even, buf0, buf2, true);
     }
+    for (; s < nu; s += 4) {
+        step(s, even, odd, buf1, buf3, false);
+        if (s + 1 < nu) step(s + 1, odd, even, buf2, buf0, false);
+        if (s + 2 < nu) step(s + 2, even, odd, buf3, buf1, false);
+        if (s + 3 < nu) step(s + 3, odd, even, buf0, buf2, false);
+    }
+    __builtin_amdgcn_s_waitcnt(0x70);  // vmcnt(0): no copy outlives its buffer
 
     if constexpr (KS == 1) {
         const int64_t t0 = (int64_t)tm * (32 * WG) + wm * 32, r0 = (int64_t)tn * (32 * WG) + wn * 32;
@@ -323,28 +338,28 @@ __global__ __launch_bounds__(64 * WG * WG * KS) __attribute__((amdgpu_waves_per_
     }
 }
 
-template <int TF, int WG, int KS, int OCC>
+template <int TF, int WG, int KS>
 void launch_tiles(const GemmParams &p, int tiles_m, int64_t tiles, hipStream_t s) {
-    hipLaunchKernelGGL((f32_tile_kernel<TF, WG, KS, OCC>), dim3((unsigned)tiles), dim3(64 * WG * WG * KS), 0, s, p,
+    hipLaunchKernelGGL((f32_tile_kernel<TF, WG, KS>), dim3((unsigned)tiles), dim3(64 * WG * WG * KS), 0, s, p,
                        tiles_m, (int)tiles);
 }
 
-// 64 x 64 tiles in one slice (87 % of the fp32 matrix rate over full rounds of
+// 64 x 64 tiles in one slice (0.85 of the fp32 matrix rate over full rounds of
 // the 256 CUs, once there are enough for two waves a SIMD) or, up to one round,
-// in two slices (76 %); 32 x 32 tiles in four slices (63 %). The cheapest by
+// in two slices (0.76); 32 x 32 tiles in four slices (0.63). The cheapest by
 // rounds over rate, in units of a 32 x 32 tile a CU. Measured (us, 64 x 64 in
-// one or two slices / 32 x 32): 896 x 4864 on 512 tokens 87 / 50, on 1024 85 /
-// 97; 4864 x 896 on 256 32 / 32, on 1024 78 / 112; 4096 x 4096 on 64 73 / 23,
-// on 256 75 / 81, on 512 128 / 161.
+// one or two slices / 32 x 32): 896 x 4864 on 512 tokens 87 / 50, on 1024 80 /
+// 97; 4864 x 896 on 256 32 / 32, on 1024 79 / 112; 4096 x 4096 on 64 73 / 23,
+// on 256 70 / 81, on 512 136 / 161.
 template <int TF>
 void launch_staged(const GemmParams &p, hipStream_t s) {
     const int64_t m64 = (p.n + 63) / 64, t64 = m64 * ((p.w.rows + 63) / 64);
     const int64_t m32 = (p.n + 31) / 32, t32 = m32 * ((p.w.rows + 31) / 32);
-    const double big = t64 > 256 ? (double)((t64 + 255) / 256) * 4 / 0.87 : 4 / 0.76;
+    const double big = t64 > 256 ? (double)((t64 + 255) / 256) * 4 / 0.85 : 4 / 0.76;
     const double small = (double)((t32 + 255) / 256) / 0.63;
-    if (small < big) launch_tiles<TF, 1, 4, 1>(p, (int)m32, t32, s);
-    else if (t64 > 256) launch_tiles<TF, 2, 1, 2>(p, (int)m64, t64, s);
-    else launch_tiles<TF, 2, 2, 2>(p, (int)m64, t64, s);
+    if (small < big) launch_tiles<TF, 1, 4>(p, (int)m32, t32, s);
+    else if (t64 > 256) launch_tiles<TF, 2, 1>(p, (int)m64, t64, s);
+    else launch_tiles<TF, 2, 2>(p, (int)m64, t64, s);
 }
 
 // rows with bounds on every column
