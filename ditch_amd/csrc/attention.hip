@@ -794,14 +794,30 @@ __global__ __launch_bounds__(1024) void attn_row_kernel(AttnArgs a) {
         const int h = i / VD;
         float s = 0.f;
         for (int w = 0; w < NW; w++) s = __fadd_rn(s, sc[w * G * VD + i]);
-        a.out[(r * a.heads + head) * VD + i] = __fmul_rn(s, inv_s[h]);
+        s = __fmul_rn(s, inv_s[h]);
+        if (a.out) a.out[(r * a.heads + head) * VD + i] = s;
+        if (a.xs) sc[i] = s;  // (this thread alone reads and writes element i of the first wave's part)
+    }
+    if (!a.xs) return;
+    // the o product's fragments: 8 consecutive dims of a head are one word a term
+    attn_lds_barrier();
+    for (int i = threadIdx.x; i < ng * VD / 8; i += blockDim.x) {
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j] = sc[8 * i + j];
+        u32x4 t[2];
+        a_words_cvt<2>(v, t);
+        const int64_t k0 = head * VD + 8 * i;
+        u32x4 *d = (u32x4 *)a.xs + ((r / 16 * a.ldk + k0 / 32) * 2) * 64 + k0 % 32 / 8 * 16 + r % 16;
+        d[0] = t[0];
+        d[64] = t[1];
     }
 }
 
 template <int HD, int VD, int G>
 static void launch_attn_row(const AttnArgs &a, int64_t kv_heads, hipStream_t s) {
-    // a wave per 32 positions of the cache, 4 to 16
-    const int64_t nw = std::min<int64_t>(16, std::max<int64_t>(4, (a.T + 31) / 32));
+    // a wave per 16 positions of the cache, 4 to 16
+    const int64_t nw = std::min<int64_t>(16, std::max<int64_t>(4, (a.T + 15) / 16));
     const size_t lds = (size_t)std::max<int64_t>(a.T * G, nw * G * VD) * 4;
     const dim3 grid((unsigned)a.n, (unsigned)kv_heads, (unsigned)((a.groups + G - 1) / G));
     hipLaunchKernelGGL((attn_row_kernel<HD, VD, G>), grid, dim3((unsigned)(nw * 64)), lds, s, a);
@@ -830,6 +846,8 @@ bool attention_rows_takes(int64_t hd, int64_t vd, int64_t groups, int64_t n, int
 void launch_attention_rows(const AttnArgs &a, int64_t kv_heads, hipStream_t s) {
     DITCH_CHECK(attention_rows_takes(a.hd, a.vd, a.groups, a.n, a.nb, a.T), DITCH_INVALID_ARGUMENT,
                 "attention: the row kernel does not take this shape");
+    DITCH_CHECK(!a.xs || ((a.heads * a.vd) % 128 == 0 && a.ldk * 32 >= a.heads * a.vd), DITCH_INVALID_ARGUMENT,
+                "attention: fragment output needs heads * v_head_dim a multiple of 128");
     if (a.hd == 64) launch_attn_rows_g<64, 64>(a, kv_heads, s);
     else if (a.hd == 128) launch_attn_rows_g<128, 128>(a, kv_heads, s);
     else launch_attn_rows_g<192, 128>(a, kv_heads, s);

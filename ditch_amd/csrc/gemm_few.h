@@ -26,4 +26,12 @@ bool few_reads_rows(const TileView &w, int64_t n, const float *x, int64_t ldx);
 void launch_few_gemm(const FewMat *mats, int nmat, const float *x, int64_t ldx, const void *xs, int64_t ldk, int64_t n,
                      int xt, hipStream_t s);
 
+// The MLP's first product: act(x gate^T) * (x up^T) (tensor.zig:1309-1337) of
+// two matrices of one format and shape the few-token product takes (no
+// deltas), as f32 rows y [n][rows] and/or as the next product's fragments
+// ys (ldk_y k tiles; rows a multiple of 128). Activations as above.
+bool few_glu_takes(const TileView &gate, const TileView &up, int64_t n);
+void launch_few_glu(const TileView &gate, const TileView &up, uint32_t act, float *y, void *ys, int64_t ldk_y,
+                    const float *x, int64_t ldx, const void *xs, int64_t ldk, int64_t n, hipStream_t s);
+
 }  // namespace ditch

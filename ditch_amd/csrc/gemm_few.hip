@@ -45,6 +45,11 @@ template <int MATS> struct FewParams {
     const float *x;
     const uint8_t *xs;
     int64_t n, ldx, ldk;
+    // GLU: f32 rows and fragments of act(x mat[0]^T) * (x mat[1]^T)
+    float *y;
+    uint8_t *ys;
+    int64_t ldk_y;
+    uint32_t act;
 };
 
 // weight units and side words per row group of a 128-column step
@@ -80,9 +85,12 @@ __device__ __forceinline__ uint32_t next_term(float &a, float &b) {
     return wd;
 }
 
-template <int TF, int MT, int NT, int W, int XT, int NX, int MATS>
+// GLU: mat[0] and mat[1] are gate and up; a workgroup takes OT row groups of
+// both, and its epilogue writes act(gate) * up of the summed tiles.
+template <int TF, int MT, int OT, int W, int XT, int NX, int MATS, bool GLU>
 __global__ __launch_bounds__(64 * W) void few_kernel(FewParams<MATS> p) {
     constexpr int UPS = Few<TF>::UPS, NS = Few<TF>::NS;
+    constexpr int NT = GLU ? 2 * OT : OT;  // row groups in registers
     typedef FewSlot<XT, NX> Slot;
     constexpr int RED = W * MT * NT * 64;
     __shared__ u32x4 lds[W * Slot::WORDS > RED ? W * Slot::WORDS : RED];
@@ -104,12 +112,14 @@ __global__ __launch_bounds__(64 * W) void few_kernel(FewParams<MATS> p) {
         }
     }
     int mi = 0;
+    if constexpr (!GLU) {
 #pragma unroll
-    for (int i = 0; i + 1 < MATS; i++) mi += rb >= p.end[i];
-    if (mi) rb -= p.end[mi - 1];
+        for (int i = 0; i + 1 < MATS; i++) mi += rb >= p.end[i];
+        if (mi) rb -= p.end[mi - 1];
+    }
     const FewMat &mat = p.mat[mi];
     const TileView &w = mat.w;
-    const int64_t groups = (w.rows + 15) / 16, g0 = (int64_t)rb * NT, units = w.units_k, K = w.cols;
+    const int64_t groups = (w.rows + 15) / 16, g0 = (int64_t)rb * OT, units = w.units_k, K = w.cols;
     const int steps = (int)((units + UPS - 1) / UPS), per = (steps + W - 1) / W;
     const int s0 = wave * per < steps ? wave * per : steps, s1 = s0 + per < steps ? s0 + per : steps;
 
@@ -120,9 +130,10 @@ __global__ __launch_bounds__(64 * W) void few_kernel(FewParams<MATS> p) {
     if constexpr (TF == TF_FP8 || TF == TF_INT4) st = side_step<TF>(w);
 #pragma unroll
     for (int i = 0; i < NT; i++) {
-        const int64_t g = g0 + i < groups ? g0 + i : groups - 1;
-        wb[i] = w.codes + g * units * 1024;
-        if constexpr (NS > 0) sb[i] = w.side + side_row(w, g, lane);
+        const TileView &wi = GLU && i >= OT ? p.mat[MATS - 1].w : w;
+        const int64_t g = g0 + i % OT < groups ? g0 + i % OT : groups - 1;
+        wb[i] = wi.codes + g * units * 1024;
+        if constexpr (NS > 0) sb[i] = wi.side + side_row(wi, g, lane);
     }
     // fragment bases of the token blocks; lanes past the tokens repeat the
     // last one (each output row of the MFMA depends on its own token only)
@@ -278,6 +289,54 @@ __global__ __launch_bounds__(64 * W) void few_kernel(FewParams<MATS> p) {
 #pragma unroll
         for (int i = 0; i < NT; i++) red[(wave * MT * NT + m * NT + i) * 64 + lane] = acc[m][i];
     __syncthreads();
+    auto total = [&](int q) {  // tile q's slices, in wave order
+        floatx4 v = red[q * 64 + lane];
+#pragma unroll
+        for (int k = 1; k < W; k++) {
+            const floatx4 o = red[(k * MT * NT + q) * 64 + lane];
+#pragma unroll
+            for (int r = 0; r < 4; r++) v[r] = __fadd_rn(v[r], o[r]);
+        }
+        return v;
+    };
+    if constexpr (GLU) {
+        __shared__ float turn[W][16][17];  // a wave's tile, [token][row]
+        for (int q = wave; q < MT * OT; q += W) {
+            const int m = q / OT, i = q % OT;
+            const floatx4 g = total(m * NT + i), u = total(m * NT + OT + i);
+            const int64_t blk = (int64_t)tb * MT + m, row = (g0 + i) * 16 + c16;
+            floatx4 v;
+#pragma unroll
+            for (int r = 0; r < 4; r++) v[r] = row < w.rows ? __fmul_rn(act_apply(p.act, g[r]), u[r]) : 0.f;
+            if (p.y) {
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int64_t tok = blk * 16 + 4 * kq + r;
+                    if (tok < p.n && row < w.rows) p.y[tok * w.rows + row] = v[r];
+                }
+            }
+            if (p.ys) {
+                // turned in the wave's own LDS (accesses in order): lane = token
+                // lane % 16, the tile's columns 8 (lane / 16) .. +8
+#pragma unroll
+                for (int r = 0; r < 4; r++) turn[wave][4 * kq + r][c16] = v[r];
+                __builtin_amdgcn_wave_barrier();
+                const int64_t k0 = (g0 + i) * 16 + 8 * kq;
+                if (lane < 32 && blk * 16 + c16 < p.n && k0 < w.rows) {
+                    float f[8];
+#pragma unroll
+                    for (int j = 0; j < 8; j++) f[j] = turn[wave][c16][8 * kq + j];
+                    u32x4 t[2];
+                    a_words_cvt<2>(f, t);
+                    u32x4 *d = (u32x4 *)p.ys + (blk * p.ldk_y + k0 / 32) * 128 + k0 % 32 / 8 * 16 + c16;
+                    d[0] = t[0];
+                    d[64] = t[1];
+                }
+                __builtin_amdgcn_wave_barrier();
+            }
+        }
+        return;
+    }
     GemmParams e{};
     e.w.rows = w.rows;
     e.out = mat.out;
@@ -288,13 +347,7 @@ __global__ __launch_bounds__(64 * W) void few_kernel(FewParams<MATS> p) {
     e.delta_xa = mat.delta_xa;
     e.delta_rank = e.delta_stride = mat.delta_rank;
     for (int q = wave; q < MT * NT; q += W) {
-        floatx4 v[1][1] = {{red[q * 64 + lane]}};
-#pragma unroll
-        for (int k = 1; k < W; k++) {
-            const floatx4 o = red[(k * MT * NT + q) * 64 + lane];
-#pragma unroll
-            for (int r = 0; r < 4; r++) v[0][0][r] = __fadd_rn(v[0][0][r], o[r]);
-        }
+        floatx4 v[1][1] = {{total(q)}};
         const int64_t tok[1] = {((int64_t)tb * MT + q / NT) * 16 + 4 * kq}, row[1] = {(g0 + q % NT) * 16 + c16};
         store_block(e, tok, row, v);
     }
@@ -308,33 +361,69 @@ struct FewCall {
     const void *xs;
     int64_t ldk, n;
     hipStream_t s;
+    uint32_t act = 0;
+    float *y = nullptr;
+    void *ys = nullptr;
+    int64_t ldk_y = 0;
 };
 
-template <int TF, int MT, int NT, int W, int XT, int NX, int MATS>
+template <int TF, int MT, int NT, int W, int XT, int NX, int MATS, bool GLU>
 void launch_mats(const FewCall &c) {
     FewParams<MATS> p{};
     int end = 0;
     for (int i = 0; i < MATS; i++) {
         if (i < c.nmat) {
             p.mat[i] = c.mats[i];
-            end += (int)((c.mats[i].w.rows + 16 * NT - 1) / (16 * NT));
+            if (!GLU || i == 0) end += (int)((c.mats[i].w.rows + 16 * NT - 1) / (16 * NT));
         }
         p.end[i] = end;
     }
+    p.y = c.y;
+    p.ys = (uint8_t *)c.ys;
+    p.ldk_y = c.ldk_y;
+    p.act = c.act;
     p.tblocks = NX ? 1 : (int)((c.n + 16 * MT - 1) / (16 * MT));
     p.x = c.x;
     p.xs = (const uint8_t *)c.xs;
     p.n = c.n;
     p.ldx = c.ldx;
     p.ldk = c.ldk;
-    hipLaunchKernelGGL((few_kernel<TF, MT, NT, W, XT, NX, MATS>), dim3((unsigned)(end * p.tblocks)), dim3(64 * W), 0,
+    hipLaunchKernelGGL((few_kernel<TF, MT, NT, W, XT, NX, MATS, GLU>), dim3((unsigned)(end * p.tblocks)), dim3(64 * W), 0,
                        c.s, p);
 }
 
 template <int TF, int MT, int NT, int W, int XT, int NX>
 void launch_cfg(const FewCall &c) {
-    if (c.nmat == 1) launch_mats<TF, MT, NT, W, XT, NX, 1>(c);
-    else launch_mats<TF, MT, NT, W, XT, NX, 3>(c);
+    if (c.nmat == 1) launch_mats<TF, MT, NT, W, XT, NX, 1, false>(c);
+    else if constexpr (XT == 2) launch_mats<TF, MT, NT, W, XT, NX, 3, false>(c);
+}
+
+// Gate and up: half the row groups of a matrix of their rows together
+template <int TF, int MT, int NT, int W, int NX>
+void launch_glu_cfg(const FewCall &c) {
+    launch_mats<TF, MT, NT, W, 2, NX, 2, true>(c);
+}
+template <int TF, int NX>
+void launch_glu_rows(const FewCall &c, int64_t groups, int64_t steps) {
+    if (groups >= 512 || steps <= 8) launch_glu_cfg<TF, 1, 1, 4, NX>(c);
+    else launch_glu_cfg<TF, 1, 1, 8, NX>(c);
+}
+template <int TF>
+void launch_glu(const FewCall &c) {
+    const int64_t groups = 2 * ((c.mats[0].w.rows + 15) / 16), steps = (c.mats[0].w.cols + 127) / 128, tb = (c.n + 15) / 16;
+    if (c.x) {
+        if (c.n == 1) launch_glu_rows<TF, 1>(c, groups, steps);
+        else if (c.n == 2) launch_glu_rows<TF, 2>(c, groups, steps);
+        else if (c.n <= 4) launch_glu_rows<TF, 4>(c, groups, steps);
+        else launch_glu_rows<TF, 8>(c, groups, steps);
+        return;
+    }
+    // the plain product's lines (launch_tf) for the two matrices together
+    const int64_t units = groups * tb;
+    if (units <= 256 && steps > 16) launch_glu_cfg<TF, 1, 1, 8, 0>(c);
+    else if (tb == 1 || units < 640) launch_glu_cfg<TF, 1, 1, 4, 0>(c);
+    else if (units < 1536 || TF == TF_FP8) launch_glu_cfg<TF, 2, 1, 4, 0>(c);
+    else launch_glu_cfg<TF, 2, 2, 4, 0>(c);
 }
 
 template <int TF, int XT, int NX>
@@ -409,7 +498,8 @@ bool few_reads_rows(const TileView &w, int64_t n, const float *x, int64_t ldx) {
 void launch_few_gemm(const FewMat *mats, int nmat, const float *x, int64_t ldx, const void *xs, int64_t ldk, int64_t n,
                      int xt, hipStream_t s) {
     const FewCall c{mats, nmat, x, ldx, xs, ldk, n, s};
-    DITCH_CHECK(nmat >= 1 && nmat <= 3 && n >= 1, DITCH_INVALID_ARGUMENT, "few-token product: 1 to 3 matrices");
+    DITCH_CHECK(nmat >= 1 && nmat <= 3 && n >= 1 && (nmat == 1 || xt == 2), DITCH_INVALID_ARGUMENT,
+                "few-token product: 1 to 3 matrices");
     for (int i = 0; i < nmat; i++)
         DITCH_CHECK(mats[i].w.tf == mats[0].w.tf && mats[i].w.cols == mats[0].w.cols && mats[i].w.fast,
                     DITCH_INVALID_ARGUMENT, "few-token product: matrices of one format and width");
@@ -426,6 +516,35 @@ void launch_few_gemm(const FewMat *mats, int nmat, const float *x, int64_t ldx, 
     default: throw Error{DITCH_UNSUPPORTED, "few-token product: format"};
     }
 #undef FEW_TF
+    DITCH_TRY_HIP(hipGetLastError());
+}
+
+bool few_glu_takes(const TileView &gate, const TileView &up, int64_t n) {
+    return gate.tf == up.tf && gate.rows == up.rows && gate.cols == up.cols && gate.units_k == up.units_k &&
+           few_gemm_takes(gate, n, false) && few_gemm_takes(up, n, false) &&
+           gate.scale_type == up.scale_type && gate.group == up.group && gate.block_cols == up.block_cols;
+}
+
+void launch_few_glu(const TileView &gate, const TileView &up, uint32_t act, float *y, void *ys, int64_t ldk_y,
+                    const float *x, int64_t ldx, const void *xs, int64_t ldk, int64_t n, hipStream_t s) {
+    DITCH_CHECK(few_glu_takes(gate, up, n) && (y || ys) && (!ys || (gate.rows % 128 == 0 && ldk_y * 32 >= gate.rows)),
+                DITCH_INVALID_ARGUMENT, "few-token gate/up: shapes or outputs");
+    DITCH_CHECK(x ? few_reads_rows(gate, n, x, ldx) : xs && ldk >= few_ldk(gate), DITCH_INVALID_ARGUMENT,
+                "few-token gate/up: activations not in a form it reads");
+    const FewMat mats[2] = {FewMat{gate, nullptr, nullptr, nullptr, nullptr, 0, 0}, FewMat{up, nullptr, nullptr, nullptr, nullptr, 0, 0}};
+    FewCall c{mats, 2, x, ldx, xs, ldk, n, s};
+    c.act = act;
+    c.y = y;
+    c.ys = ys;
+    c.ldk_y = ldk_y;
+    switch (gate.tf) {
+    case TF_BF16: launch_glu<TF_BF16>(c); break;
+    case TF_Q8: launch_glu<TF_Q8>(c); break;
+    case TF_FP8: launch_glu<TF_FP8>(c); break;
+    case TF_MX4: launch_glu<TF_MX4>(c); break;
+    case TF_INT4: launch_glu<TF_INT4>(c); break;
+    default: throw Error{DITCH_UNSUPPORTED, "few-token gate/up: format"};
+    }
     DITCH_TRY_HIP(hipGetLastError());
 }
 

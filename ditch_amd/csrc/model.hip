@@ -10,6 +10,7 @@
 #include "decode.h"
 #include "internal.h"
 #include "attention_rope.h"
+#include "gemm_few.h"
 #include "tiled.h"
 #include "model.h"
 
@@ -1110,6 +1111,17 @@ static bool frag_only(const Mat &mt, int64_t n) { return mt.ok() && mt.rank == 0
 // A product that reads MX fragments alone (MXFP4 on the scaled MFMA).
 static bool mx_only(const Mat &mt, int64_t n) { return mt.ok() && mt.rank == 0 && mx_gemm_takes(mt.t->v, n); }
 
+// Whether the few-token product takes every one of up to three matrices over
+// one activation in one launch (no deltas, one format and width).
+static bool few_together(std::initializer_list<const Mat *> mats, int64_t n) {
+    const Mat *first = *mats.begin();
+    for (const Mat *m : mats)
+        if (!m->ok() || m->rank != 0 || !few_gemm_takes(m->t->v, n, false) || m->t->v.tf != first->t->v.tf ||
+            m->t->v.cols != first->t->v.cols)
+            return false;
+    return true;
+}
+
 // Whether a routed layer's grouped products can be planned on the device:
 // every expert resident (no cache), gate/up/down of one tiled format and
 // shape (the fused GLU then the down product, whose epilogue adds each
@@ -1408,9 +1420,14 @@ void model_forward(ditch_hip_model *m, const uint32_t *d_tokens, const ditch_row
     // are kept only for consumers that need them.
     const bool frags = n >= 128;
     const int64_t ldk_h = split_ldk(hidden);
+    // Small batches run the few-token products: q, k and v in one launch, gate,
+    // up and the activation in another. Up to 8 rows they read f32 rows, more
+    // come as fragments from the norm, the attention and the gate/up product.
+    const bool few = n < 128, few_rows = n <= 8 && hidden % 4 == 0;
     for (int64_t li = 0; li < (int64_t)c.layers; li++) {
         Layer &L = m->layers[li];
         Act hact{h, nullptr, 0};
+        const bool few_qkv = few && !c.mla && few_together({&L.q, &L.k, &L.v}, n);
         const bool mx_qkv = frags && !c.mla && mx_only(L.q, n) && mx_only(L.k, n) && mx_only(L.v, n) &&
                             L.q.t->v.units_k == L.k.t->v.units_k && L.q.t->v.units_k == L.v.t->v.units_k;
         if (mx_qkv) {
@@ -1430,6 +1447,10 @@ void model_forward(ditch_hip_model *m, const uint32_t *d_tokens, const ditch_row
             launch_rmsnorm_split(hs, ldk_h, f32_needed ? h : nullptr, x, L.attn_norm.p, L.attn_norm.len, n, hidden,
                                  c.rms_eps, 0, s);
             hact = Act{f32_needed ? h : nullptr, hs, ldk_h};
+        } else if (few_qkv && !few_rows) {
+            void *hs = m->hs.get<uint8_t>(split_bytes_ldk(n, ldk_h, 2));
+            launch_rmsnorm_split(hs, ldk_h, nullptr, x, L.attn_norm.p, L.attn_norm.len, n, hidden, c.rms_eps, 0, s);
+            hact = Act{nullptr, hs, ldk_h};
         } else {
             launch_rmsnorm(h, x, L.attn_norm.p, L.attn_norm.len, n, hidden, c.rms_eps, 0, s);
         }
@@ -1463,6 +1484,11 @@ void model_forward(ditch_hip_model *m, const uint32_t *d_tokens, const ditch_row
                                    n, nh, hd, nope, rd, vd, kvl);
                 DITCH_TRY_HIP(hipGetLastError());
             }
+        } else if (few_qkv) {
+            const FewMat mats[3] = {FewMat{L.q.t->v, q, L.q_bias.p, nullptr, nullptr, 0, 0},
+                                    FewMat{L.k.t->v, kk, L.k_bias.p, nullptr, nullptr, 0, 0},
+                                    FewMat{L.v.t->v, vv, L.v_bias.p, nullptr, nullptr, 0, 0}};
+            launch_few_gemm(mats, 3, hact.f32, hidden, hact.xs, ldk_h, n, 2, s);
         } else {
             mm_act(m, L.q, q, hact, n, L.q_bias.p, 0, s);
             mm_act(m, L.k, kk, hact, n, L.k_bias.p, 0, s);
@@ -1533,6 +1559,14 @@ void model_forward(ditch_hip_model *m, const uint32_t *d_tokens, const ditch_row
             aact = Act{att, aa.xs, aa.ldk};
         }
         if (prompt_attn) aa.dense = dense_flag;
+        // few rows: the row kernel writes the o product's fragments (the f32
+        // rows too when a delta reads them)
+        if (row_attn && few && !few_rows && L.o.ok() && few_gemm_takes(L.o.t->v, n, false) && (nh * vd) % 128 == 0) {
+            aa.ldk = split_ldk(nh * vd);
+            aa.xs = m->atts.get<uint8_t>(split_bytes_ldk(n, aa.ldk, 2));
+            if (L.o.rank == 0) aa.out = nullptr;
+            aact = Act{aa.out, aa.xs, aa.ldk};
+        }
         if (row_attn) launch_attention_rows(aa, nkv, s);
         else if (q_rope_in_attn) launch_attention_mfma_rope(aa, AttnRope{m->rope_cos, m->rope_sin, (int64_t)c.rope_len}, nkv, s);
         else if (mfma_attn) launch_attention_mfma(aa, nkv, s);
@@ -1570,6 +1604,25 @@ void model_forward(ditch_hip_model *m, const uint32_t *d_tokens, const ditch_row
             void *as = m->acts.get<uint8_t>(split_bytes_ldk(n, ldk_i, 2));
             launch_tile_glu(L.gate.t->v, L.up.t->v, 0, nullptr, as, ldk_i, hs, ldk_h, n, s);
             mm_act(m, L.down, x, Act{nullptr, as, ldk_i}, n, nullptr, 1, s);  // x += down(act)
+            capture(li + 1);
+            continue;
+        }
+        if (few && !moe_layer && few_together({&L.gate, &L.up}, n) && few_glu_takes(L.gate.t->v, L.up.t->v, n) &&
+            (few_rows || (L.gate.t->v.rows % 128 == 0 && few_gemm_takes(L.down.t->v, n, false)))) {
+            const int64_t inter = L.gate.t->v.rows, ldk_i = split_ldk(inter);
+            if (few_rows) {
+                launch_rmsnorm(h, x, L.ffn_norm.p, L.ffn_norm.len, n, hidden, c.rms_eps, 0, s);
+                float *g = m->g.get<float>(n * inter);
+                launch_few_glu(L.gate.t->v, L.up.t->v, 0, g, nullptr, 0, h, hidden, nullptr, 0, n, s);
+                mm(m, L.down, x, g, n, nullptr, 1, s);  // x += down(act)
+            } else {
+                void *hs = m->hs.get<uint8_t>(split_bytes_ldk(n, ldk_h, 2));
+                launch_rmsnorm_split(hs, ldk_h, nullptr, x, L.ffn_norm.p, L.ffn_norm.len, n, hidden, c.rms_eps, 0, s);
+                float *g = L.down.rank > 0 ? m->g.get<float>(n * inter) : nullptr;
+                void *as = m->acts.get<uint8_t>(split_bytes_ldk(n, ldk_i, 2));
+                launch_few_glu(L.gate.t->v, L.up.t->v, 0, g, as, ldk_i, nullptr, 0, hs, ldk_h, n, s);
+                mm_act(m, L.down, x, Act{g, as, ldk_i}, n, nullptr, 1, s);  // x += down(act)
+            }
             capture(li + 1);
             continue;
         }

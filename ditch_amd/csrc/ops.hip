@@ -1,6 +1,8 @@
 // ops.hip — element-wise and reduction kernels of the forward pass and of
 // the VTable's per-row operations (compute.zig:107-119), plus row norms and
 // W^T y over resident weights (tensor.zig:1056-1122).
+#include <algorithm>
+
 #include "decode.h"
 #include "internal.h"
 #include "gemm_common.h"
@@ -121,6 +123,60 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(float *out, const flo
             if (wlen > 0) e[q] = __fmul_rn(e[q], gemma ? __fadd_rn(1.0f, w[i + q]) : w[i + q]);
         }
         o[64 * j + lane] = make_float4(e[0], e[1], e[2], e[3]);
+    }
+}
+
+// RMS norm of few rows: a workgroup per row, 8 consecutive columns a thread in
+// registers (rows up to 8192 columns, a multiple of 8), as f32 rows and/or as
+// bf16-term fragments (columns past len zero up to ldk k tiles). The kernels
+// above give a row to one wave, which at few rows is one wave's chain of 4096
+// columns: a single row took 12.4 us, here 3.
+__global__ __launch_bounds__(1024) void rmsnorm_few_kernel(u32x4 *xs, int64_t ldk, float *out, const float *x,
+                                                           const float *w, int64_t wlen, int64_t len, float eps,
+                                                           int gemma, const int64_t *row_index, int64_t n_src) {
+    __shared__ float sh[16];
+    const int64_t r = blockIdx.x;
+    int64_t src = row_index ? row_index[r] : r;
+    src = (uint64_t)src < (uint64_t)n_src ? src : n_src - 1;  // the row lists are unsigned
+    const int64_t k0 = 8 * (int64_t)threadIdx.x;
+    float v[8], wv[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        v[j] = 0.f;
+        wv[j] = 1.f;
+    }
+    if (k0 < len) {
+        const float4 a = *(const float4 *)(x + src * len + k0), b = *(const float4 *)(x + src * len + k0 + 4);
+        v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+        if (wlen > 0) {
+#pragma unroll
+            for (int j = 0; j < 8; j++) wv[j] = gemma ? __fadd_rn(1.0f, w[k0 + j]) : w[k0 + j];
+        }
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < 8; j++) ss = __builtin_fmaf(v[j], v[j], ss);
+    ss = block_sum(ss, sh);
+    const float inv = __fdiv_rn(1.0f, __fsqrt_rn(__fadd_rn(__fdiv_rn(ss, (float)len), eps)));
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        v[j] = __fmul_rn(v[j], inv);
+        if (wlen > 0) v[j] = __fmul_rn(v[j], wv[j]);
+    }
+    if (out && k0 < len) {
+        *(float4 *)(out + r * len + k0) = make_float4(v[0], v[1], v[2], v[3]);
+        *(float4 *)(out + r * len + k0 + 4) = make_float4(v[4], v[5], v[6], v[7]);
+    }
+    if (xs && k0 < ldk * 32) {
+        if (k0 >= len) {
+#pragma unroll
+            for (int j = 0; j < 8; j++) v[j] = 0.f;
+        }
+        u32x4 t[2];
+        a_words_cvt<2>(v, t);
+        u32x4 *d = xs + ((r / 16 * ldk + k0 / 32) * 2) * 64 + k0 % 32 / 8 * 16 + r % 16;
+        d[0] = t[0];
+        d[64] = t[1];
     }
 }
 
@@ -780,11 +836,31 @@ __global__ __launch_bounds__(512) void delta_xa_lds_kernel(float *xa, const floa
 // ---------------------------------------------------------------------------
 // Launchers
 
+// (at 4096 columns a row a workgroup stays ahead of a row a wave up to about
+// 1024 rows; above that both run at the memory rate)
+constexpr int64_t RMS_FEW = 1024;
+static bool rmsnorm_few_takes(const void *x, const void *out, const float *w, int64_t wlen, int64_t n, int64_t len) {
+    return n <= RMS_FEW && len % 8 == 0 && len <= 8192 && (wlen == 0 || wlen >= len) && ((uintptr_t)x & 15) == 0 &&
+           ((uintptr_t)out & 15) == 0;
+}
+static void launch_rmsnorm_few(void *xs, int64_t ldk, float *out, const float *x, const float *w, int64_t wlen, int64_t n,
+                               int64_t len, float eps, int gemma, hipStream_t s, const int64_t *row_index, int64_t ns) {
+    const int64_t cols = std::max<int64_t>(len, xs ? ldk * 32 : 0), threads = (cols / 8 + 63) / 64 * 64;
+    DITCH_CHECK(threads <= 1024, DITCH_INVALID_ARGUMENT, "rmsnorm: fragments wider than a workgroup");
+    hipLaunchKernelGGL(rmsnorm_few_kernel, dim3((unsigned)n), dim3((unsigned)threads), 0, s, (u32x4 *)xs, ldk, out, x, w,
+                       wlen, len, eps, gemma, row_index, ns);
+    DITCH_TRY_HIP(hipGetLastError());
+}
+
 void launch_rmsnorm(float *out, const float *x, const float *w, int64_t wlen, int64_t n, int64_t len, float eps,
                     int gemma, hipStream_t s, const int64_t *row_index, int64_t n_src) {
     if (n <= 0) return;
     const int64_t ns = row_index ? n_src : n;
     const dim3 g4((unsigned)((n + 3) / 4));
+    if (rmsnorm_few_takes(x, out, w, wlen, n, len)) {
+        launch_rmsnorm_few(nullptr, 0, out, x, w, wlen, n, len, eps, gemma, s, row_index, ns);
+        return;
+    }
     // rows of whole 256-column steps up to 4096, 16-byte aligned: a wave per row
     const bool rows = len % 256 == 0 && len <= 4096 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)out & 15) == 0;
     if (rows && len == 512) hipLaunchKernelGGL(rmsnorm_rows_kernel<2>, g4, dim3(256), 0, s, out, x, w, wlen, n, eps, gemma, row_index, ns);
@@ -800,6 +876,10 @@ void launch_rmsnorm_split(void *xs, int64_t ldk, float *out, const float *x, con
                           int64_t len, float eps, int gemma, hipStream_t s) {
     if (n <= 0) return;
     DITCH_CHECK(ldk * 32 >= len, DITCH_INVALID_ARGUMENT, "rmsnorm_split: fragments shorter than the row");
+    if (n < 128 && ldk <= 256 && rmsnorm_few_takes(x, out, w, wlen, n, len)) {
+        launch_rmsnorm_few(xs, ldk, out, x, w, wlen, n, len, eps, gemma, s, nullptr, n);
+        return;
+    }
     const dim3 grid((unsigned)((n + 15) / 16));
     // rows up to 4096 columns (fragments up to 128 k tiles): one read of each row
     if (ldk <= 32) hipLaunchKernelGGL(rmsnorm_split_rows_kernel<1>, grid, dim3(1024), 0, s, (u32x4 *)xs, ldk, out, x, w, wlen, len, eps, gemma, n);
