@@ -823,10 +823,19 @@ static void launch_attn_row(const AttnArgs &a, int64_t kv_heads, hipStream_t s) 
     hipLaunchKernelGGL((attn_row_kernel<HD, VD, G>), grid, dim3((unsigned)(nw * 64)), lds, s, a);
 }
 
+// Heads of a KV head a workgroup: four share each key's load where that still
+// gives every CU a workgroup, else two. us a call with 1, 2, 4 and 8 heads:
+//   n x keys, head_dim, KV heads x groups      1     2     4     8
+//   1 x 500, 128, 8 x 4                     12.8  12.3  16.2
+//   8 x 900, 128, 8 x 4                     23.0  21.0  25.4
+//   16 x 96, 64, 2 x 7                       5.5   6.0   7.4  11.8
+//   48 x 300, 64, 2 x 7                     17.7  14.0  13.2  15.7
+//   4 prompts of 30, 128, 8 x 4             14.2  12.8  10.8
 template <int HD, int VD>
 static void launch_attn_rows_g(const AttnArgs &a, int64_t kv_heads, hipStream_t s) {
-    if (a.groups >= 5) launch_attn_row<HD, VD, 8>(a, kv_heads, s);
-    else if (a.groups >= 2) launch_attn_row<HD, VD, 4>(a, kv_heads, s);
+    const bool four = a.n * kv_heads * ((a.groups + 3) / 4) >= 256;
+    if (a.groups > 2 && four) launch_attn_row<HD, VD, 4>(a, kv_heads, s);
+    else if (a.groups > 1) launch_attn_row<HD, VD, 2>(a, kv_heads, s);
     else launch_attn_row<HD, VD, 1>(a, kv_heads, s);
 }
 
