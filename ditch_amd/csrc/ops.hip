@@ -84,58 +84,34 @@ __global__ void rmsnorm_kernel(float *out, const float *x, const float *w, int64
     }
 }
 
-// rmsnorm_kernel for rows of 256 NV columns: a wave per row holds it in
-// registers (NV float4 a lane, one read of the row), sums its squares over
-// the wave and writes the normalised row; four rows a workgroup.
-template <int NV>
-__global__ __launch_bounds__(256) void rmsnorm_rows_kernel(float *out, const float *x, const float *w, int64_t wlen,
-                                                           int64_t n, float eps, int gemma, const int64_t *row_index,
+// RMS norm of rows of whole 8-column pieces up to 8192 columns: a workgroup per
+// row, 8 consecutive columns a thread in registers, as f32 rows and/or as
+// bf16-term fragments (columns past len zero up to ldk k tiles; the last
+// block's rows past n zero). Bound by the memory rate from about 1000 rows and
+// by one row's load, sum and store below. A wave a row, or a workgroup per 16
+// rows with the fragments turned in LDS, left a chain of a whole row to each
+// wave and, below 4096 rows, CUs without a workgroup. us a call, before ->
+// here, 4096 columns: f32 rows n = 1 12.4 -> 3, 128 10.0 -> 4.2, 1024 13.1 ->
+// 8.9, 8192 61 -> 46 (5.8 TB/s); fragments n = 128 22.0 -> 4.9, 1080 23.1 ->
+// 8.8, 4096 35.1 -> 32.4; 7168 columns, f32 rows n = 8192 168 -> 89, fragments
+// n = 256 77.7 -> 6.8, 4096 107 -> 51.
+__global__ __launch_bounds__(1024) void rmsnorm_row_kernel(u32x4 *xs, int64_t ldk, float *out, const float *x,
+                                                           const float *w, int64_t wlen, int64_t n, int64_t len,
+                                                           float eps, int gemma, const int64_t *row_index,
                                                            int64_t n_src) {
-    constexpr int64_t LEN = 256 * NV;
-    const int lane = threadIdx.x & 63;
-    const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (r >= n) return;
-    int64_t src = row_index ? row_index[r] : r;
-    src = (uint64_t)src < (uint64_t)n_src ? src : n_src - 1;  // the row lists are unsigned
-    const float4 *xr = (const float4 *)(x + src * LEN);
-    float4 v[NV];
-#pragma unroll
-    for (int j = 0; j < NV; j++) v[j] = xr[64 * j + lane];
-    float ss = 0.f;
-#pragma unroll
-    for (int j = 0; j < NV; j++) {
-        ss = __builtin_fmaf(v[j].x, v[j].x, ss);
-        ss = __builtin_fmaf(v[j].y, v[j].y, ss);
-        ss = __builtin_fmaf(v[j].z, v[j].z, ss);
-        ss = __builtin_fmaf(v[j].w, v[j].w, ss);
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) ss = __fadd_rn(ss, __shfl_xor(ss, o, 64));
-    const float inv = __fdiv_rn(1.0f, __fsqrt_rn(__fadd_rn(__fdiv_rn(ss, (float)LEN), eps)));
-    float4 *o = (float4 *)(out + r * LEN);
-#pragma unroll
-    for (int j = 0; j < NV; j++) {
-        const int64_t i = 4 * (64 * j + lane);
-        float e[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            e[q] = __fmul_rn(e[q], inv);
-            if (wlen > 0) e[q] = __fmul_rn(e[q], gemma ? __fadd_rn(1.0f, w[i + q]) : w[i + q]);
-        }
-        o[64 * j + lane] = make_float4(e[0], e[1], e[2], e[3]);
-    }
-}
-
-// RMS norm of few rows: a workgroup per row, 8 consecutive columns a thread in
-// registers (rows up to 8192 columns, a multiple of 8), as f32 rows and/or as
-// bf16-term fragments (columns past len zero up to ldk k tiles). The kernels
-// above give a row to one wave, which at few rows is one wave's chain of 4096
-// columns: a single row took 12.4 us, here 3.
-__global__ __launch_bounds__(1024) void rmsnorm_few_kernel(u32x4 *xs, int64_t ldk, float *out, const float *x,
-                                                           const float *w, int64_t wlen, int64_t len, float eps,
-                                                           int gemma, const int64_t *row_index, int64_t n_src) {
     __shared__ float sh[16];
-    const int64_t r = blockIdx.x;
+    // (xs: grid of whole 16-row blocks; full groups of 8 blocks keep a block's
+    // rows on one XCD, whose L2 joins their 16-byte pieces of a fragment line)
+    const int64_t b = blockIdx.x, group = b / 128 * 128;
+    const int64_t r = xs && group + 128 <= (int64_t)gridDim.x ? group + b % 8 * 16 + b % 128 / 8 : b;
+    if (r >= n) {  // the last block's rows past n are zero
+        const int64_t k0 = 8 * (int64_t)threadIdx.x;
+        if (k0 < ldk * 32) {
+            u32x4 *d = xs + ((r / 16 * ldk + k0 / 32) * 2) * 64 + k0 % 32 / 8 * 16 + r % 16;
+            d[0] = d[64] = u32x4{0, 0, 0, 0};
+        }
+        return;
+    }
     int64_t src = row_index ? row_index[r] : r;
     src = (uint64_t)src < (uint64_t)n_src ? src : n_src - 1;  // the row lists are unsigned
     const int64_t k0 = 8 * (int64_t)threadIdx.x;
@@ -395,103 +371,6 @@ __global__ __launch_bounds__(256) void rmsnorm_split_mx_kernel(uint8_t *xm, int6
             }
             mx_write_slot(v, xm + (m16 * ldst + st) * MX_BLOCK, l);
         }
-        __syncthreads();
-    }
-}
-
-// The same as rmsnorm_split_kernel with each row read once: wave w of 16
-// holds row 16 m16 + w in registers (lane l: columns 1024 j + 16 l .. +16,
-// j < NPH), sums its squares with a butterfly over the wave, normalises, and
-// writes each phase's two-term words (32 k tiles) into LDS in fragment
-// order; the workgroup then copies the phase's 64 KiB to the fragments in
-// whole 16-byte words.
-template <int NPH>
-__global__ __launch_bounds__(1024) void rmsnorm_split_rows_kernel(u32x4 *xs, int64_t ldk, float *out, const float *x,
-                                                                  const float *w, int64_t wlen, int64_t len,
-                                                                  float eps, int gemma, int64_t n) {
-    __shared__ u32x4 phase_buf[32 * 2 * 64];  // [k tile][term][lane], 64 KiB
-    const int64_t m16 = blockIdx.x;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int64_t r = m16 * 16 + wave;
-    const bool row_in = r < n;
-    const bool vec = (len % 4) == 0 && ((uintptr_t)x & 15) == 0;
-    float xv[NPH][16];
-#pragma unroll
-    for (int j = 0; j < NPH; j++) {
-        const int64_t k0 = 1024 * j + 16 * lane;
-        if (row_in && vec && k0 + 16 <= len) {
-#pragma unroll
-            for (int q = 0; q < 16; q += 4) {
-                const float4 a = *(const float4 *)(x + r * len + k0 + q);
-                xv[j][q] = a.x; xv[j][q + 1] = a.y; xv[j][q + 2] = a.z; xv[j][q + 3] = a.w;
-            }
-        } else {
-#pragma unroll
-            for (int q = 0; q < 16; q++) xv[j][q] = row_in && k0 + q < len ? x[r * len + k0 + q] : 0.f;
-        }
-    }
-    float ss = 0.f;
-#pragma unroll
-    for (int j = 0; j < NPH; j++)
-#pragma unroll
-        for (int q = 0; q < 16; q++) ss = __builtin_fmaf(xv[j][q], xv[j][q], ss);
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) ss = __fadd_rn(ss, __shfl_xor(ss, o, 64));
-    const float inv = row_in ? __fdiv_rn(1.0f, __fsqrt_rn(__fadd_rn(__fdiv_rn(ss, (float)len), eps))) : 0.f;
-#pragma unroll
-    for (int j = 0; j < NPH; j++) {
-        const int64_t kt0 = 32 * j;
-        if (kt0 >= ldk) break;
-        const int64_t k0 = 1024 * j + 16 * lane;
-        float v[16];
-#pragma unroll
-        for (int q = 0; q < 16; q += 4) {
-            float4 b = make_float4(1.f, 1.f, 1.f, 1.f);
-            if (wlen > 0 && (wlen % 4) == 0 && k0 + q + 4 <= wlen) b = *(const float4 *)(w + k0 + q);
-            else if (wlen > 0) {
-                b.x = k0 + q < wlen ? w[k0 + q] : 1.f;
-                b.y = k0 + q + 1 < wlen ? w[k0 + q + 1] : 1.f;
-                b.z = k0 + q + 2 < wlen ? w[k0 + q + 2] : 1.f;
-                b.w = k0 + q + 3 < wlen ? w[k0 + q + 3] : 1.f;
-            }
-            const float wb[4] = {b.x, b.y, b.z, b.w};
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                float y = 0.f;
-                if (row_in && k0 + q + u < len) {
-                    y = __fmul_rn(xv[j][q + u], inv);
-                    if (wlen > 0) y = __fmul_rn(y, gemma ? __fadd_rn(1.0f, wb[u]) : wb[u]);
-                }
-                v[q + u] = y;
-            }
-        }
-        if (out && row_in) {
-            if (vec && k0 + 16 <= len) {
-#pragma unroll
-                for (int q = 0; q < 16; q += 4) *(float4 *)(out + r * len + k0 + q) = make_float4(v[q], v[q + 1], v[q + 2], v[q + 3]);
-            } else {
-#pragma unroll
-                for (int q = 0; q < 16; q++)
-                    if (k0 + q < len) out[r * len + k0 + q] = v[q];
-            }
-        }
-        // k tile kt0 + lane / 2, its 8-column chunks 2 (lane % 2) and 2 (lane % 2) + 1
-        const int ktl = lane >> 1;
-#pragma unroll
-        for (int c = 0; c < 2; c++) {
-            float v8[8];
-#pragma unroll
-            for (int q = 0; q < 8; q++) v8[q] = v[8 * c + q];
-            u32x4 words[2];
-            a_words<false, 2>(v8, words);
-            const int slot = wave + 16 * (2 * (lane & 1) + c);
-            phase_buf[(ktl * 2 + 0) * 64 + slot] = words[0];
-            phase_buf[(ktl * 2 + 1) * 64 + slot] = words[1];
-        }
-        __syncthreads();
-        const int64_t nkt = ldk - kt0 < 32 ? ldk - kt0 : 32;
-        u32x4 *dst = xs + (m16 * ldk + kt0) * 2 * 64;
-        for (int64_t i = threadIdx.x; i < nkt * 128; i += 1024) dst[i] = phase_buf[i];
         __syncthreads();
     }
 }
@@ -836,19 +715,18 @@ __global__ __launch_bounds__(512) void delta_xa_lds_kernel(float *xa, const floa
 // ---------------------------------------------------------------------------
 // Launchers
 
-// (at 4096 columns a row a workgroup stays ahead of a row a wave up to about
-// 1024 rows; above that both run at the memory rate)
-constexpr int64_t RMS_FEW = 1024;
-static bool rmsnorm_few_takes(const void *x, const void *out, const float *w, int64_t wlen, int64_t n, int64_t len) {
-    return n <= RMS_FEW && len % 8 == 0 && len <= 8192 && (wlen == 0 || wlen >= len) && ((uintptr_t)x & 15) == 0 &&
+// the row kernel takes every row it can address; the general kernels keep odd
+// lengths, weights shorter than the row, unaligned bases and longer rows
+static bool rmsnorm_row_takes(const void *x, const void *out, int64_t wlen, int64_t len) {
+    return len % 8 == 0 && len <= 8192 && (wlen == 0 || wlen >= len) && ((uintptr_t)x & 15) == 0 &&
            ((uintptr_t)out & 15) == 0;
 }
-static void launch_rmsnorm_few(void *xs, int64_t ldk, float *out, const float *x, const float *w, int64_t wlen, int64_t n,
+static void launch_rmsnorm_row(void *xs, int64_t ldk, float *out, const float *x, const float *w, int64_t wlen, int64_t n,
                                int64_t len, float eps, int gemma, hipStream_t s, const int64_t *row_index, int64_t ns) {
     const int64_t cols = std::max<int64_t>(len, xs ? ldk * 32 : 0), threads = (cols / 8 + 63) / 64 * 64;
     DITCH_CHECK(threads <= 1024, DITCH_INVALID_ARGUMENT, "rmsnorm: fragments wider than a workgroup");
-    hipLaunchKernelGGL(rmsnorm_few_kernel, dim3((unsigned)n), dim3((unsigned)threads), 0, s, (u32x4 *)xs, ldk, out, x, w,
-                       wlen, len, eps, gemma, row_index, ns);
+    hipLaunchKernelGGL(rmsnorm_row_kernel, dim3((unsigned)(xs ? (n + 15) / 16 * 16 : n)), dim3((unsigned)threads), 0, s,
+                       (u32x4 *)xs, ldk, out, x, w, wlen, n, len, eps, gemma, row_index, ns);
     DITCH_TRY_HIP(hipGetLastError());
 }
 
@@ -856,36 +734,24 @@ void launch_rmsnorm(float *out, const float *x, const float *w, int64_t wlen, in
                     int gemma, hipStream_t s, const int64_t *row_index, int64_t n_src) {
     if (n <= 0) return;
     const int64_t ns = row_index ? n_src : n;
-    const dim3 g4((unsigned)((n + 3) / 4));
-    if (rmsnorm_few_takes(x, out, w, wlen, n, len)) {
-        launch_rmsnorm_few(nullptr, 0, out, x, w, wlen, n, len, eps, gemma, s, row_index, ns);
+    if (rmsnorm_row_takes(x, out, wlen, len)) {
+        launch_rmsnorm_row(nullptr, 0, out, x, w, wlen, n, len, eps, gemma, s, row_index, ns);
         return;
     }
-    // rows of whole 256-column steps up to 4096, 16-byte aligned: a wave per row
-    const bool rows = len % 256 == 0 && len <= 4096 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)out & 15) == 0;
-    if (rows && len == 512) hipLaunchKernelGGL(rmsnorm_rows_kernel<2>, g4, dim3(256), 0, s, out, x, w, wlen, n, eps, gemma, row_index, ns);
-    else if (rows && len == 1024) hipLaunchKernelGGL(rmsnorm_rows_kernel<4>, g4, dim3(256), 0, s, out, x, w, wlen, n, eps, gemma, row_index, ns);
-    else if (rows && len == 2048) hipLaunchKernelGGL(rmsnorm_rows_kernel<8>, g4, dim3(256), 0, s, out, x, w, wlen, n, eps, gemma, row_index, ns);
-    else if (rows && len == 4096) hipLaunchKernelGGL(rmsnorm_rows_kernel<16>, g4, dim3(256), 0, s, out, x, w, wlen, n, eps, gemma, row_index, ns);
-    else
-        hipLaunchKernelGGL(rmsnorm_kernel, dim3((unsigned)n), dim3(256), 0, s, out, x, w, wlen, len, eps, gemma,
-                           row_index, ns, len, len);
+    hipLaunchKernelGGL(rmsnorm_kernel, dim3((unsigned)n), dim3(256), 0, s, out, x, w, wlen, len, eps, gemma, row_index,
+                       ns, len, len);
     DITCH_TRY_HIP(hipGetLastError());
 }
 void launch_rmsnorm_split(void *xs, int64_t ldk, float *out, const float *x, const float *w, int64_t wlen, int64_t n,
                           int64_t len, float eps, int gemma, hipStream_t s) {
     if (n <= 0) return;
     DITCH_CHECK(ldk * 32 >= len, DITCH_INVALID_ARGUMENT, "rmsnorm_split: fragments shorter than the row");
-    if (n < 128 && ldk <= 256 && rmsnorm_few_takes(x, out, w, wlen, n, len)) {
-        launch_rmsnorm_few(xs, ldk, out, x, w, wlen, n, len, eps, gemma, s, nullptr, n);
+    if (ldk <= 256 && rmsnorm_row_takes(x, out, wlen, len)) {
+        launch_rmsnorm_row(xs, ldk, out, x, w, wlen, n, len, eps, gemma, s, nullptr, n);
         return;
     }
-    const dim3 grid((unsigned)((n + 15) / 16));
-    // rows up to 4096 columns (fragments up to 128 k tiles): one read of each row
-    if (ldk <= 32) hipLaunchKernelGGL(rmsnorm_split_rows_kernel<1>, grid, dim3(1024), 0, s, (u32x4 *)xs, ldk, out, x, w, wlen, len, eps, gemma, n);
-    else if (ldk <= 64) hipLaunchKernelGGL(rmsnorm_split_rows_kernel<2>, grid, dim3(1024), 0, s, (u32x4 *)xs, ldk, out, x, w, wlen, len, eps, gemma, n);
-    else if (ldk <= 128) hipLaunchKernelGGL(rmsnorm_split_rows_kernel<4>, grid, dim3(1024), 0, s, (u32x4 *)xs, ldk, out, x, w, wlen, len, eps, gemma, n);
-    else hipLaunchKernelGGL(rmsnorm_split_kernel, grid, dim3(256), 0, s, (u32x4 *)xs, ldk, out, x, w, wlen, len, eps, gemma, n);
+    hipLaunchKernelGGL(rmsnorm_split_kernel, dim3((unsigned)((n + 15) / 16)), dim3(256), 0, s, (u32x4 *)xs, ldk, out, x, w,
+                       wlen, len, eps, gemma, n);
     DITCH_TRY_HIP(hipGetLastError());
 }
 void launch_rmsnorm_split_mx(void *xm, int64_t ldst, float *out, const float *x, const float *w, int64_t wlen,

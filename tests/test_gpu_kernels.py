@@ -172,9 +172,8 @@ def test_rmsnorm_layernorm_softmax(dev, ref):
 
 @pytest.mark.parametrize("length", [512, 1024, 2048, 4096])
 def test_rmsnorm_rows_held_in_registers(dev, ref, length):
-    """Rows of 512-4096 columns take the wave-per-row kernel (the row held in
-    registers, one read): with and without a weight, gemma's (1 + w), and a
-    row count that leaves the last workgroup partly empty."""
+    """Rows of 512-4096 columns, held in registers: with and without a weight,
+    and gemma's (1 + w)."""
     rng = np.random.default_rng(length)
     x = (rng.standard_normal((7, length)) * 3).astype(np.float32)
     w = rng.standard_normal(length).astype(np.float32)

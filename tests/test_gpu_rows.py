@@ -1,0 +1,63 @@
+"""Row kernels and the few-token forward at the edges of their ranges, against
+the oracle (needs an MI355X)."""
+import numpy as np
+import pytest
+
+import model_gen as mg
+from ditch_amd import abi
+from ditch_amd.hip import Model
+from oracle.ref import RefModel
+
+pytestmark = pytest.mark.gpu
+
+
+# one 8-column piece, a wave's edge, more columns than a workgroup of 512, the
+# longest row of the row kernel; then the general kernel (longer, not of 8)
+@pytest.mark.parametrize("length", [8, 512, 520, 7168, 8192, 8200, 1020])
+@pytest.mark.parametrize("n", [1, 129])
+def test_rmsnorm_row_lengths(dev, ref, n, length):
+    rng = np.random.default_rng(length + n)
+    x = (rng.standard_normal((n, length)) * 3).astype(np.float32)
+    w = rng.standard_normal(length).astype(np.float32)
+    # sums of squares and products in f32, at most a few roundings a value
+    for weight, gemma in ((w, False), (w, True), (None, False)):
+        want = ref.rmsnorm_rows(x, weight, 1e-6, gemma=gemma)
+        got = dev.rmsnormRows(x, weight, 1e-6, gemma_style=gemma)
+        assert np.abs(got - want).max() <= 4e-6 * np.abs(want).max()
+
+
+def _check(gm, cm, lens, vocab, seed):
+    tokens, rows, last = mg.batch(len(lens), lens, vocab, seed=seed)
+    rg, lg = gm.forward(tokens, rows, capture_rows=last, logit_rows=last)
+    rc, lc = cm.forward(tokens, rows, capture_rows=last, logit_rows=last)
+    # two-term products (2^-18 an activation) and other summation orders
+    # through two layers: 1e-5 of the largest value, ten times that allowed
+    assert np.abs(lg - lc).max() <= 1e-4 * np.abs(lc).max()
+    assert np.abs(rg - rc).max() <= 1e-4 * np.abs(rc).max()
+
+
+# f32 rows up to 8 tokens, fragments above; one and two token blocks; the last
+# count of the few-token path and the first two of the tiled one
+LENS = [[1], [5, 3], [9], [7, 9], [17], [33], [63, 64], [128], [100, 30]]
+
+
+@pytest.mark.parametrize("fmt", ["bf16", "fp8", "mxfp4", "int4", "q8_0", "f32"])
+def test_forward_token_counts_match_oracle(dev, ref, fmt):
+    """Plain layers, then with deltas on o and down (whose inputs stay f32)."""
+    inter = 640 if fmt == "int4" else 672  # (int4 rows are whole 128-column groups)
+    spec = mg.dense(fmt, hidden=384, inter=inter, heads=6, kv_heads=2, head_dim=64, layers=2, vocab=640, seed=4)
+    gm, cm = Model(dev, spec), RefModel(spec)
+    rng = np.random.default_rng(5)
+    try:
+        for i, lens in enumerate(LENS):
+            _check(gm, cm, lens, 640, i)
+        for slot, k, rank, li in ((abi.SLOT["O"], 384, 3, 0), (abi.SLOT["DOWN"], inter, 2, 1)):
+            a = (rng.standard_normal((rank, k)) * 0.05).astype(np.float32)
+            b = (rng.standard_normal((384, rank)) * 0.05).astype(np.float32)
+            for m in (gm, cm):
+                m.set_delta(li, slot, -1, a, b)
+        for i, lens in enumerate(LENS):
+            _check(gm, cm, lens, 640, 20 + i)
+    finally:
+        gm.free()
+        cm.free()
