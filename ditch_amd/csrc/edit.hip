@@ -7,13 +7,15 @@
 // input-side ablation (abliterate.zig:234-261).
 //
 // Every pass over W runs on the resident (re-tiled, still quantised) weight:
-// row norms, W^T y for up to 16 vectors at a time, and the exact three-term
+// row norms, W^T y for all vectors in one launch, and the exact three-term
 // product W x for the q vectors of the SVD. The rest is q or k vectors of
-// the matrix's width: one workgroup orthonormalises them, one runs the
-// Jacobi eigen-solver of the q x q Gram matrix.
+// the matrix's width: up to 24 are orthonormalised over column chunks (wider
+// sets by one workgroup), one workgroup runs the Jacobi eigen-solver of the
+// q x q Gram matrix.
 #include <math.h>
 #include <string.h>
 
+#include <algorithm>
 #include <vector>
 
 #include "internal.h"
@@ -237,63 +239,256 @@ __global__ __launch_bounds__(1024) void edit_orth_reg_kernel(float *vecs, int64_
     }
 }
 
+// ---------------------------------------------------------------------------
+// Orthonormalisation of few vectors (q <= ED_GRAM_Q) in three short launches
+// over column chunks, instead of one workgroup's 2 q^2 dot products in a row
+// (10 vectors: 67 us at 896 columns and 100 at 4864, all of it barriers and
+// f64 latency). Gram-Schmidt needs only the inner products: a launch leaves
+// every chunk's part of the f64 Gram matrix, the next adds the parts, factors
+// the Gram matrix (each workgroup the same small Cholesky, whose rows are the
+// projections of Gram-Schmidt in f64), applies it to its own columns with one
+// rounding an element, and leaves the parts of the new Gram matrix; the third
+// does that pass again, which takes the orthogonality from eps * cond to eps
+// as the second Gram-Schmidt pass does. A vector that depends on the earlier
+// ones to f32 rounding (its remainder at most 1e-7 of it) or whose norm is at
+// most 1e-20 is zero and projects nothing; NaN and infinite vectors too.
+// The neighbours ride along: the operator's second half on the product the
+// chunk is read from (`scale`, `u`), the dot products the next half needs and
+// the row-scaled copy it multiplies (`pa`, `cy`).
+// 6 to 9 us a launch (latency: the parts, the factorisation, the columns); the
+// 28 orthonormalisations and their neighbours of an 896 x 4864 edit took 67 to
+// 100 us each and 12 to 20 us of neighbours.
+constexpr int ED_GRAM_Q = 24;  // vectors: LDS for a 256-column chunk and the parts
+constexpr int ED_GRAM_K = 8;   // directions of the neighbours
+struct OrthArgs {
+    float *v;  // [q][n], in place
+    int64_t n;
+    int q, k, chunk;
+    // before: v = v * scale[col] + sum_l (sum of dots_in)[j][l] u[l][col]
+    const float *scale, *u;
+    const double *dots_in;
+    int dots_parts;
+    const double *gram_in;  // [chunks][pairs]: orthonormalise by this Gram matrix
+    double *gram_out;       // parts of the resulting vectors' Gram matrix
+    // after: parts of dot(pa_l, v_j) [chunks][q k], cy = cs[col] v
+    const float *pa, *cs;
+    double *dots_out;
+    float *cy;
+    int store;
+};
+
+// row and column of the p-th entry of a lower triangle (p below 2^20)
+__device__ __forceinline__ void ed_pair(int p, int &i, int &j) {
+    i = (int)((__fsqrt_rn(8.f * p + 1.f) - 1.f) * 0.5f);
+    while (i * (i + 1) / 2 > p) i--;
+    while ((i + 1) * (i + 2) / 2 <= p) i++;
+    j = p - i * (i + 1) / 2;
+}
+
+__device__ __forceinline__ double ed_lane(double v, int lane) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                            __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+
+// QM: the vectors, rounded up to the instances below. A thread holds one
+// column of every vector; the Cholesky is done by each wave that holds
+// columns (lane i: row i), so its factors are scalars for the columns.
+template <int QM>
+__global__ __launch_bounds__(256) void edit_orth_chunk_kernel(OrthArgs a) {
+    extern __shared__ double ed_sh[];
+    const int q = a.q, k = a.k, ld = a.chunk + 1, pairs = q * (q + 1) / 2;
+    const int np = pairs > q * k ? pairs : q * k;
+    double *tmp = ed_sh;
+    float *xl = (float *)(tmp + 4 * np), *pr = xl + q * ld;  // [q][ld], [k][ld]
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int64_t n = a.n, c0 = (int64_t)blockIdx.x * a.chunk, col = c0 + tid;
+    const int nc = (int)(n - c0 < a.chunk ? n - c0 : a.chunk);
+    const bool in = tid < nc;
+    float x[QM];
+#pragma unroll
+    for (int j = 0; j < QM; j++) x[j] = in && j < q ? a.v[j * n + col] : 0.f;
+
+    // parts [chunks][count] added by four waves, then in wave order
+    auto add_parts = [&](const double *parts, int chunks, int count) {
+        for (int p = lane; p < count; p += 64) {
+            double r = 0.0;
+#pragma unroll 8
+            for (int b = wave; b < chunks; b += 4) r += parts[(int64_t)b * count + p];
+            tmp[wave * np + p] = r;
+        }
+        __syncthreads();
+    };
+    auto part = [&](int p) { return tmp[p] + tmp[np + p] + tmp[2 * np + p] + tmp[3 * np + p]; };
+
+    if (a.u) {
+        const float sc = a.scale && in ? a.scale[col] : 1.f;
+        add_parts(a.dots_in, a.dots_parts, q * k);
+        if (a.scale) {
+#pragma unroll
+            for (int j = 0; j < QM; j++) x[j] = __fmul_rn(x[j], sc);
+        }
+        for (int l = 0; l < k; l++) {
+            const float u = in ? a.u[l * n + col] : 0.f;
+#pragma unroll
+            for (int j = 0; j < QM; j++)
+                if (j < q) x[j] = __fadd_rn(x[j], __fmul_rn((float)part(j * k + l), u));
+        }
+        __syncthreads();
+    }
+    if (a.gram_in) {
+        add_parts(a.gram_in, (int)gridDim.x, pairs);
+        if (wave * 64 < nc) {
+            double row[QM], inv[QM];
+            const int i = lane < q ? lane : q - 1;
+#pragma unroll
+            for (int j = 0; j < QM; j++) row[j] = j <= i ? part(i * (i + 1) / 2 + j) : 0.0;
+            const double d0 = part(i * (i + 1) / 2 + i);
+#pragma unroll
+            for (int j = 0; j < QM; j++) {
+                inv[j] = 0.0;
+                if (j >= q) continue;
+                const double r = ed_lane(row[j], j);
+                const bool live = r > 1e-14 * ed_lane(d0, j) && r > 1e-40;
+                double y = __builtin_amdgcn_rsq(r);
+#pragma unroll
+                for (int it = 0; it < 2; it++) y = y * (1.5 - 0.5 * r * y * y);
+                inv[j] = live ? y : 0.0;
+                row[j] = live ? row[j] * y : 0.0;
+#pragma unroll
+                for (int c = j + 1; c < QM; c++)
+                    if (c < q) row[c] -= row[j] * ed_lane(row[j], c);
+            }
+            double xd[QM];
+#pragma unroll
+            for (int r = 0; r < QM; r++) {
+                xd[r] = 0.0;
+                if (r >= q) continue;
+                double acc = (double)x[r];
+#pragma unroll
+                for (int j = 0; j < r; j++) acc -= ed_lane(row[j], r) * xd[j];
+                x[r] = inv[r] > 0.0 ? (float)(acc * inv[r]) : 0.f;
+                xd[r] = (double)x[r];
+            }
+        }
+        __syncthreads();
+    }
+    if (in) {
+        const float cs = a.cy ? a.cs[col] : 0.f;
+#pragma unroll
+        for (int j = 0; j < QM; j++)
+            if (j < q) {
+                if (a.store) a.v[j * n + col] = x[j];
+                if (a.cy) a.cy[j * n + col] = __fmul_rn(cs, x[j]);
+                xl[j * ld + tid] = x[j];
+            }
+        if (a.pa)
+            for (int l = 0; l < k; l++) pr[l * ld + tid] = a.pa[l * n + col];
+    }
+    __syncthreads();
+    // dot products of LDS rows over the chunk: a pair a lane, a quarter of the
+    // columns a wave
+    auto dots = [&](int count, bool gram, double *out) {
+        for (int p = lane; p < count; p += 64) {
+            int i, j;
+            if (gram) ed_pair(p, i, j);
+            else i = p / k, j = q + p % k;  // (the rows of pr follow those of x)
+            double r = 0.0;
+#pragma unroll 8
+            for (int c = wave; c < nc; c += 4) r += (double)xl[i * ld + c] * (double)xl[j * ld + c];
+            tmp[wave * np + p] = r;
+        }
+        __syncthreads();
+        for (int p = tid; p < count; p += 256) out[(int64_t)blockIdx.x * count + p] = part(p);
+        __syncthreads();
+    };
+    if (a.pa) dots(q * k, false, a.dots_out);
+    if (a.gram_out) dots(pairs, true, a.gram_out);
+}
+
 // SVD widths up to ED_LDS_Q keep the Jacobi's two q x q matrices in LDS;
 // wider ones work on them in place in global memory.
 constexpr int ED_LDS_Q = 128;
 
 // abliterate.jacobiEigen (abliterate.zig:427-469): cyclic Jacobi in f32 on the
 // q x q matrix m (in place: its diagonal ends as the eigenvalues),
-// eigenvectors in the columns of vecs. One block; the rotation's updates
-// are spread over the block's threads in the reference's order.
+// eigenvectors in the columns of vecs. One block. A sweep takes its pivots in
+// rounds of n / 2 disjoint ones (a tournament: entry 0 stays, the others move
+// on by one), whose rotations touch different rows and columns: the angles of
+// a round together, then every column pair, then every row pair. One pivot at
+// a time, a rotation's division and square root chain (0.35 us) came 45 times
+// a sweep of 10 x 10; in rounds 9 times.
 template <bool LDS>
-__global__ __launch_bounds__(1024) void edit_jacobi_kernel(float *m_g, float *vecs_g, int n) {
+__global__ __launch_bounds__(1024) void edit_jacobi_kernel(float *m_g, float *vecs_g, float2 *rot_g, int n) {
     extern __shared__ float ed_dyn[];
-    __shared__ int stop;
+    __shared__ double sh[16];
     float *m = LDS ? ed_dyn : m_g, *vecs = LDS ? ed_dyn + n * n : vecs_g;
+    const int half = (n + 1) / 2, ring = 2 * half - 1;  // odd n: one pivot of a round has no partner
+    float2 *rot = LDS ? (float2 *)(ed_dyn + 2 * n * n) : rot_g;
     const int tid = threadIdx.x, nt = blockDim.x;
     for (int t = tid; t < n * n; t += nt) {
         if (LDS) m[t] = m_g[t];
         vecs[t] = (t / n == t % n) ? 1.f : 0.f;
     }
     __syncthreads();
+    // the pivots (p < q) of pair i of a round; false: none
+    auto pivot = [&](int round, int i, int &p, int &q) {
+        const int a = i ? 1 + (round + i) % ring : 0, b = 1 + (round + ring - i) % ring;
+        p = a < b ? a : b;
+        q = a < b ? b : a;
+        return q < n;
+    };
     for (int sweep = 0; sweep < 50; sweep++) {
-        if (tid == 0) {
-            double off = 0;
-            for (int i = 0; i < n; i++)
-                for (int j = 0; j < n; j++)
-                    if (i != j) off += (double)m[i * n + j] * (double)m[i * n + j];
-            stop = off < 1e-18;
+        double off = 0;
+        for (int t = tid; t < n * n; t += nt)
+            if (t / n != t % n) off += (double)m[t] * (double)m[t];
+        off = ed_block_sum(off, sh);
+        if (off < 1e-18) break;
+        for (int round = 0; round < ring; round++) {
+            __syncthreads();
+            for (int i = tid; i < half; i += nt) {
+                int p, q;
+                float2 r = make_float2(1.f, 0.f);
+                if (pivot(round, i, p, q)) {
+                    const float apq = m[p * n + q];
+                    if (!(fabsf(apq) < 1e-20f)) {
+                        const float app = m[p * n + p], aqq = m[q * n + q];
+                        const float theta = __fdiv_rn(__fsub_rn(aqq, app), __fmul_rn(2.0f, apq));
+                        const float sg = theta > 0.f ? 1.f : theta < 0.f ? -1.f : 0.f;
+                        const float t = __fdiv_rn(sg, __fadd_rn(fabsf(theta), __fsqrt_rn(__fadd_rn(__fmul_rn(theta, theta), 1.0f))));
+                        const float tf = theta == 0.f ? 1.0f : t;
+                        r.x = __fdiv_rn(1.0f, __fsqrt_rn(__fadd_rn(__fmul_rn(tf, tf), 1.0f)));
+                        r.y = __fmul_rn(tf, r.x);
+                    }
+                }
+                rot[i] = r;
+            }
+            __syncthreads();
+            for (int t = tid; t < n * half; t += nt) {
+                const int k = t % n, i = t / n;
+                int p, q;
+                if (!pivot(round, i, p, q)) continue;
+                const float cs = rot[i].x, sn = rot[i].y;
+                if (sn == 0.f && cs == 1.f) continue;
+                const float akp = m[k * n + p], akq = m[k * n + q];
+                m[k * n + p] = __fsub_rn(__fmul_rn(cs, akp), __fmul_rn(sn, akq));
+                m[k * n + q] = __fadd_rn(__fmul_rn(sn, akp), __fmul_rn(cs, akq));
+                const float vkp = vecs[k * n + p], vkq = vecs[k * n + q];
+                vecs[k * n + p] = __fsub_rn(__fmul_rn(cs, vkp), __fmul_rn(sn, vkq));
+                vecs[k * n + q] = __fadd_rn(__fmul_rn(sn, vkp), __fmul_rn(cs, vkq));
+            }
+            __syncthreads();
+            for (int t = tid; t < n * half; t += nt) {
+                const int k = t % n, i = t / n;
+                int p, q;
+                if (!pivot(round, i, p, q)) continue;
+                const float cs = rot[i].x, sn = rot[i].y;
+                if (sn == 0.f && cs == 1.f) continue;
+                const float apk = m[p * n + k], aqk = m[q * n + k];
+                m[p * n + k] = __fsub_rn(__fmul_rn(cs, apk), __fmul_rn(sn, aqk));
+                m[q * n + k] = __fadd_rn(__fmul_rn(sn, apk), __fmul_rn(cs, aqk));
+            }
         }
         __syncthreads();
-        if (stop) break;
-        for (int p = 0; p < n; p++)
-            for (int q = p + 1; q < n; q++) {
-                const float apq = m[p * n + q];
-                if (fabsf(apq) < 1e-20f) continue;
-                const float app = m[p * n + p], aqq = m[q * n + q];
-                const float theta = __fdiv_rn(__fsub_rn(aqq, app), __fmul_rn(2.0f, apq));
-                const float sg = theta > 0.f ? 1.f : theta < 0.f ? -1.f : 0.f;
-                const float t = __fdiv_rn(sg, __fadd_rn(fabsf(theta), __fsqrt_rn(__fadd_rn(__fmul_rn(theta, theta), 1.0f))));
-                const float tf = theta == 0.f ? 1.0f : t;
-                const float cs = __fdiv_rn(1.0f, __fsqrt_rn(__fadd_rn(__fmul_rn(tf, tf), 1.0f)));
-                const float sn = __fmul_rn(tf, cs);
-                __syncthreads();  // every thread has read the pivot before it changes
-                for (int k = tid; k < n; k += nt) {
-                    const float akp = m[k * n + p], akq = m[k * n + q];
-                    m[k * n + p] = __fsub_rn(__fmul_rn(cs, akp), __fmul_rn(sn, akq));
-                    m[k * n + q] = __fadd_rn(__fmul_rn(sn, akp), __fmul_rn(cs, akq));
-                    const float vkp = vecs[k * n + p], vkq = vecs[k * n + q];
-                    vecs[k * n + p] = __fsub_rn(__fmul_rn(cs, vkp), __fmul_rn(sn, vkq));
-                    vecs[k * n + q] = __fadd_rn(__fmul_rn(sn, vkp), __fmul_rn(cs, vkq));
-                }
-                __syncthreads();
-                for (int k = tid; k < n; k += nt) {
-                    const float apk = m[p * n + k], aqk = m[q * n + k];
-                    m[p * n + k] = __fsub_rn(__fmul_rn(cs, apk), __fmul_rn(sn, aqk));
-                    m[q * n + k] = __fadd_rn(__fmul_rn(sn, apk), __fmul_rn(cs, aqk));
-                }
-                __syncthreads();
-            }
     }
     __syncthreads();
     if (LDS)
@@ -305,42 +500,47 @@ __global__ __launch_bounds__(1024) void edit_jacobi_kernel(float *m_g, float *ve
 
 // The SVD's factors and the LoRA pair (abliterate.zig:514-547): eigenvalues
 // sorted descending (a stable sort), s_t = sqrt(max(lambda, 0)), u_t = Q e,
-// v_t = B^T e / s_t; a[t] = sqrt(s_t) v_t, b[i][t] = u_t[i] sqrt(s_t). One
-// block per output component t (rank of them).
+// v_t = B^T e / s_t; a[t] = sqrt(s_t) v_t, b[i][t] = u_t[i] sqrt(s_t). A
+// thread per row and column, a grid row per output component t (rank of them).
 __global__ __launch_bounds__(256) void edit_svd_out_kernel(float *a, float *b, const float *evals_m,
                                                            const float *evecs, const float *qy, const float *bt,
-                                                           int q, int64_t rows, int64_t cols, int64_t rank,
-                                                           int64_t ldb, int64_t b_off) {
-    extern __shared__ int order[];  // q entries
-    const int t = blockIdx.x;
-    if (threadIdx.x == 0) {
-        for (int i = 0; i < q; i++) order[i] = i;
-        for (int i = 1; i < q; i++) {
-            const int o = order[i];
-            int j = i;
-            while (j > 0 && evals_m[order[j - 1] * q + order[j - 1]] < evals_m[o * q + o]) {
-                order[j] = order[j - 1];
-                j--;
-            }
-            order[j] = o;
-        }
+                                                           int q, int64_t rows, int64_t cols, int64_t ldb,
+                                                           int64_t b_off) {
+    extern __shared__ float ed_dyn[];  // the q eigenvalues, then the q entries of the eigenvector
+    float *ev = ed_dyn, *e = ed_dyn;
+    __shared__ int src_s;
+    const int t = blockIdx.y;
+    for (int i = threadIdx.x; i < q; i += blockDim.x) ev[i] = evals_m[(int64_t)i * q + i];
+    if (threadIdx.x == 0) src_s = t;
+    __syncthreads();
+    // component t's eigenvalue: t are larger, or equal and before it
+    for (int i = threadIdx.x; i < q; i += blockDim.x) {
+        int above = 0;
+        for (int j = 0; j < q; j++) above += ev[j] > ev[i] || (ev[j] == ev[i] && j < i);
+        if (above == t) src_s = i;
     }
     __syncthreads();
-    const int src = order[t];
-    const float lambda = fmaxf(evals_m[src * q + src], 0.f);
+    const int src = src_s;
+    const float lambda = fmaxf(ev[src], 0.f);
+    __syncthreads();
+    for (int i = threadIdx.x; i < q; i += blockDim.x) e[i] = evecs[(int64_t)i * q + src];
+    __syncthreads();
     const float s = __fsqrt_rn(lambda);
     const float sq = __fsqrt_rn(fmaxf(s, 0.f));
     const float inv = s > 1e-12f ? __fdiv_rn(1.0f, s) : 0.f;
-    for (int64_t i = threadIdx.x; i < rows; i += blockDim.x) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < rows) {
         float u = 0.f;
-        for (int c = 0; c < q; c++) u = __fadd_rn(u, __fmul_rn(evecs[c * q + src], qy[c * rows + i]));
+#pragma unroll 4
+        for (int c = 0; c < q; c++) u = __fadd_rn(u, __fmul_rn(e[c], qy[c * rows + i]));
         b[i * ldb + b_off + t] = __fmul_rn(u, sq);
     }
-    for (int64_t j = threadIdx.x; j < cols; j += blockDim.x) {
+    if (i < cols) {
         float v = 0.f;
-        for (int c = 0; c < q; c++) v = __fadd_rn(v, __fmul_rn(evecs[c * q + src], bt[c * cols + j]));
+#pragma unroll 4
+        for (int c = 0; c < q; c++) v = __fadd_rn(v, __fmul_rn(e[c], bt[c * cols + i]));
         v = s > 1e-12f ? __fmul_rn(v, inv) : 0.f;
-        a[t * cols + j] = __fmul_rn(sq, v);
+        a[t * cols + i] = __fmul_rn(sq, v);
     }
 }
 
@@ -377,6 +577,7 @@ int64_t edit_rank(int64_t rows, int64_t cols, int64_t k, int mode, int64_t lora_
 
 struct EditWork {
     DevBuf v, norms, vn, a, bp, wa, gram, c, d, omega, qy, qx, cy, dots, bbt, evecs, xs, xa, wu;
+    DevBuf gram0, gram1, dpart0, dpart1, rot;
 };
 
 // b[i][0..r) = bp[i][0..r), b[i][r + j] = -lambda wu[j][i]  (abliterate.zig:252-257)
@@ -409,7 +610,54 @@ static void edit_matvecT(const TileView &w, float *out, const float *y, int64_t 
     launch_matvecT(out, w, y, q, s);
 }
 
-static void edit_orth(float *vecs, int64_t q, int64_t n, hipStream_t s) {
+// columns a workgroup: 64 up to 4096 (enough workgroups), at most 256
+static int orth_chunk(int64_t n) { return (int)(64 * std::min<int64_t>(4, (n + 4095) / 4096)); }
+static int64_t orth_chunks(int64_t n) { return (n + orth_chunk(n) - 1) / orth_chunk(n); }
+static bool orth_takes(int64_t q, int64_t k) { return q <= ED_GRAM_Q && k <= ED_GRAM_K; }
+
+static void launch_orth_chunk(OrthArgs a, hipStream_t s) {
+    a.chunk = orth_chunk(a.n);
+    const int64_t pairs = (int64_t)a.q * (a.q + 1) / 2, np = std::max<int64_t>(pairs, (int64_t)a.q * a.k);
+    const size_t lds = (size_t)(4 * np * 8 + (a.q + a.k) * (a.chunk + 1) * 4);
+    DITCH_CHECK(lds <= 65536, DITCH_INVALID_ARGUMENT, "edit: too many vectors for the chunked orthonormalisation");
+    const dim3 grid((unsigned)orth_chunks(a.n));
+    if (a.q <= 4) hipLaunchKernelGGL(edit_orth_chunk_kernel<4>, grid, dim3(256), lds, s, a);
+    else if (a.q <= 12) hipLaunchKernelGGL(edit_orth_chunk_kernel<12>, grid, dim3(256), lds, s, a);
+    else hipLaunchKernelGGL(edit_orth_chunk_kernel<24>, grid, dim3(256), lds, s, a);
+    DITCH_TRY_HIP(hipGetLastError());
+}
+
+// The three launches: `first` holds what is done before the first Gram matrix,
+// `last` what follows the second pass (v, n, q and k are first's).
+static void edit_orth_chunks(EditWork &W, OrthArgs first, OrthArgs last, hipStream_t s) {
+    const int64_t parts = orth_chunks(first.n) * first.q * (first.q + 1) / 2;
+    double *g0 = W.gram0.get<double>(parts), *g1 = W.gram1.get<double>(parts);
+    OrthArgs mid{};
+    mid.v = last.v = first.v;
+    mid.n = last.n = first.n;
+    mid.q = last.q = first.q;
+    mid.k = last.k = first.k;
+    first.gram_out = g0;
+    first.store = first.u != nullptr;
+    mid.gram_in = g0;
+    mid.gram_out = g1;
+    mid.store = 1;
+    last.gram_in = g1;
+    last.store = 1;
+    launch_orth_chunk(first, s);
+    launch_orth_chunk(mid, s);
+    launch_orth_chunk(last, s);
+}
+
+static void edit_orth(EditWork &W, float *vecs, int64_t q, int64_t n, hipStream_t s) {
+    if (orth_takes(q, 0)) {
+        OrthArgs a{};
+        a.v = vecs;
+        a.n = n;
+        a.q = (int)q;
+        edit_orth_chunks(W, a, OrthArgs{}, s);
+        return;
+    }
     const int64_t ept = (n + 1023) / 1024;
     if (ept <= 2)
         hipLaunchKernelGGL(edit_orth_reg_kernel<2>, dim3(1), dim3(1024), 0, s, vecs, q, n);
@@ -426,19 +674,21 @@ static void edit_orth(float *vecs, int64_t q, int64_t n, hipStream_t s) {
     DITCH_TRY_HIP(hipGetLastError());
 }
 
-static void edit_jacobi(float *m, float *vecs, int64_t q, hipStream_t s) {
+static void edit_jacobi(EditWork &W, float *m, float *vecs, int64_t q, hipStream_t s) {
     DITCH_CHECK(q <= 46340, DITCH_UNSUPPORTED, "edit: SVD width above 46340");
-    const dim3 block(q <= 256 ? 256 : 1024);
+    const int64_t items = q * ((q + 1) / 2);  // (row, pair) updates of a round
+    const dim3 block((unsigned)std::min<int64_t>(1024, (items + 63) / 64 * 64));
     if (q <= ED_LDS_Q) {
         static const bool attr = [] {
             return hipFuncSetAttribute((const void *)edit_jacobi_kernel<true>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       2 * ED_LDS_Q * ED_LDS_Q * 4) == hipSuccess;
+                                       2 * ED_LDS_Q * ED_LDS_Q * 4 + ED_LDS_Q * 8) == hipSuccess;
         }();
         DITCH_CHECK(attr, DITCH_DEVICE_FAILED, "edit: the Jacobi kernel's LDS size was refused");
-        hipLaunchKernelGGL(edit_jacobi_kernel<true>, dim3(1), block, (size_t)(2 * q * q * 4), s, m, vecs, (int)q);
+        hipLaunchKernelGGL(edit_jacobi_kernel<true>, dim3(1), block, (size_t)(2 * q * q * 4 + (q + 1) * 4), s, m, vecs,
+                           (float2 *)nullptr, (int)q);
     } else {
-        hipLaunchKernelGGL(edit_jacobi_kernel<false>, dim3(1), block, 0, s, m, vecs, (int)q);
+        hipLaunchKernelGGL(edit_jacobi_kernel<false>, dim3(1), block, 0, s, m, vecs, W.rot.get<float2>((q + 1) / 2), (int)q);
     }
     DITCH_TRY_HIP(hipGetLastError());
 }
@@ -520,20 +770,67 @@ void edit_delta_device(ditch_hip *h, const TileView &w, const float *hv, int64_t
                                    cols);
                 DITCH_TRY_HIP(hipGetLastError());
             };
-            apply(qy, omega);
-            edit_orth(qy, q, rows, s);
-            for (int it = 0; it < 6; it++) {
-                applyT(qx, qy);
-                edit_orth(qx, q, cols, s);
-                apply(qy, qx);
-                edit_orth(qy, q, rows, s);
+            if (orth_takes(q, k)) {
+                // the operator's halves with the second part of each in the
+                // orthonormalisation's launches
+                double *ax = W.dpart0.get<double>(orth_chunks(cols) * q * k);
+                double *dy = W.dpart1.get<double>(orth_chunks(rows) * q * k);
+                OrthArgs in{};  // ax = dot(a_l, omega_j)
+                in.v = omega;
+                in.n = cols;
+                in.q = (int)q;
+                in.k = (int)k;
+                in.pa = a;
+                in.dots_out = ax;
+                launch_orth_chunk(in, s);
+                for (int it = 0; it < 7; it++) {
+                    if (it) {
+                        edit_matvecT(w, qx, cy, q, s);
+                        OrthArgs f{}, l{};
+                        f.v = qx;
+                        f.n = cols;
+                        f.q = (int)q;
+                        f.k = (int)k;
+                        f.u = a;
+                        f.dots_in = dy;
+                        f.dots_parts = (int)orth_chunks(rows);
+                        l.pa = a;
+                        l.dots_out = ax;
+                        edit_orth_chunks(W, f, l, s);
+                    }
+                    edit_matmul(w, qy, it ? qx : omega, q, s, &W.xs);
+                    OrthArgs f{}, l{};
+                    f.v = qy;
+                    f.n = rows;
+                    f.q = (int)q;
+                    f.k = (int)k;
+                    f.scale = c;
+                    f.u = d;
+                    f.dots_in = ax;
+                    f.dots_parts = (int)orth_chunks(cols);
+                    l.pa = d;
+                    l.dots_out = dy;
+                    l.cs = c;
+                    l.cy = cy;
+                    edit_orth_chunks(W, f, l, s);
+                }
+            } else {
+                apply(qy, omega);
+                edit_orth(W, qy, q, rows, s);
+                for (int it = 0; it < 6; it++) {
+                    applyT(qx, qy);
+                    edit_orth(W, qx, q, cols, s);
+                    apply(qy, qx);
+                    edit_orth(W, qy, q, rows, s);
+                }
             }
             applyT(qx, qy);  // B^T = (Q^T D)^T
             float *bbt = W.bbt.get<float>(q * q), *evecs = W.evecs.get<float>(q * q);
             edit_dots(bbt, qx, q, qx, q, cols, s);
-            edit_jacobi(bbt, evecs, q, s);
-            hipLaunchKernelGGL(edit_svd_out_kernel, dim3((unsigned)r_out), dim3(256), (size_t)q * 4, s, A, Bp, bbt,
-                               evecs, qy, qx, (int)q, rows, cols, r_out, r_out, (int64_t)0);
+            edit_jacobi(W, bbt, evecs, q, s);
+            hipLaunchKernelGGL(edit_svd_out_kernel, dim3((unsigned)((std::max(rows, cols) + 255) / 256), (unsigned)r_out),
+                               dim3(256), (size_t)q * 4, s, A, Bp, bbt, evecs, qy, qx, (int)q, rows, cols, r_out,
+                               (int64_t)0);
             DITCH_TRY_HIP(hipGetLastError());
         }
         if (ablate) {
@@ -541,7 +838,7 @@ void edit_delta_device(ditch_hip *h, const TileView &w, const float *hv, int64_t
             // rank grows by k (abliterate.zig:234-261)
             float *u = A + r_out * cols;
             edit_matvecT(w, u, v, k, s);
-            edit_orth(u, k, cols, s);
+            edit_orth(W, u, k, cols, s);
             float *wu = W.wu.get<float>(k * rows);
             float *xa = W.xa.get<float>(k * r_out);
             edit_matmul(w, wu, u, k, s, &W.xs, A, Bp, (int)r_out, xa);

@@ -33,10 +33,9 @@ struct WtyArgs {
     const WtySeg *segs;     // device table, or NULL: the one segment `one`
     const int64_t *items;   // per workgroup: segment << 32 | unit (with segs)
     WtySeg one;
-    int64_t q0, q;          // directions q0 .. q0 + q (q <= the kernel's QB)
+    int64_t q;              // directions, QB of them a workgroup (blockIdx.y)
 };
 
-constexpr int WTY_WAVES = 4;
 constexpr int WTY_STEP = 4;  // row groups whose loads are in flight together
 
 
@@ -122,11 +121,11 @@ template <int TF, bool FAST> constexpr int wty_side_words() {
     else return 1;
 }
 
-template <int TF, int QB, bool FAST>
-__global__ __launch_bounds__(WTY_WAVES * 64) void wty_kernel(WtyArgs a) {
+template <int TF, int QB, bool FAST, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void wty_kernel(WtyArgs a) {
     constexpr int TL = Fmt<TF>::tiles, UK = 32 * TL, NV = 8 * TL;
     constexpr int NS = wty_side_words<TF, FAST>();
-    __shared__ float red[WTY_WAVES][QB][UK];
+    __shared__ float red[WAVES][QB][UK];
     int64_t unit;
     const WtySeg *sp = &a.one;
     if (a.segs) {
@@ -141,7 +140,7 @@ __global__ __launch_bounds__(WTY_WAVES * 64) void wty_kernel(WtyArgs a) {
     float *out = sp->out;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int r16 = lane & 15, kq = lane >> 4;
-    const int64_t groups = (w.rows + 15) / 16;
+    const int64_t groups = (w.rows + 15) / 16, q0 = (int64_t)blockIdx.y * QB;
     float acc[QB][NV];
 #pragma unroll
     for (int j = 0; j < QB; j++)
@@ -150,7 +149,7 @@ __global__ __launch_bounds__(WTY_WAVES * 64) void wty_kernel(WtyArgs a) {
 
     SideStep st{1u, 0};
     if constexpr (FAST) st = side_step<TF>(w);
-    for (int64_t g0 = (int64_t)wave * WTY_STEP; g0 < groups; g0 += WTY_WAVES * WTY_STEP) {
+    for (int64_t g0 = (int64_t)wave * WTY_STEP; g0 < groups; g0 += WAVES * WTY_STEP) {
         Raw raw[WTY_STEP];
         WtySide<TF> sd[WTY_STEP];
         uint32_t sw[WTY_STEP][NS];
@@ -170,7 +169,7 @@ __global__ __launch_bounds__(WTY_WAVES * 64) void wty_kernel(WtyArgs a) {
             }
 #pragma unroll
             for (int j = 0; j < QB; j++)
-                yv[i][j] = (g0 + i < groups && row < w.rows && j < a.q) ? y[(a.q0 + j) * w.rows + row] : 0.f;
+                yv[i][j] = (g0 + i < groups && row < w.rows && q0 + j < a.q) ? y[(q0 + j) * w.rows + row] : 0.f;
         }
 #pragma unroll
         for (int i = 0; i < WTY_STEP; i++) {
@@ -210,30 +209,45 @@ __global__ __launch_bounds__(WTY_WAVES * 64) void wty_kernel(WtyArgs a) {
             if (r16 == 0) red[wave][j][32 * (v / 8) + 8 * kq + (v % 8)] = s;
         }
     __syncthreads();
-    for (int i = threadIdx.x; i < QB * UK; i += WTY_WAVES * 64) {
+    for (int i = threadIdx.x; i < QB * UK; i += WAVES * 64) {
         const int j = i / UK, c = i % UK;
         const int64_t col = unit * UK + c;
-        if (j >= a.q || col >= w.cols) continue;
+        if (q0 + j >= a.q || col >= w.cols) continue;
         float s = red[0][j][c];
 #pragma unroll
-        for (int wv = 1; wv < WTY_WAVES; wv++) s = __fadd_rn(s, red[wv][j][c]);
-        out[(a.q0 + j) * w.cols + col] = s;
+        for (int wv = 1; wv < WAVES; wv++) s = __fadd_rn(s, red[wv][j][c]);
+        out[(q0 + j) * w.cols + col] = s;
     }
 }
 
-template <int TF, bool FAST>
+template <int TF, int QB, bool FAST, int WAVES>
 static void wty_launch_q(const WtyArgs &a, unsigned blocks, hipStream_t s) {
-    if (a.q == 1) hipLaunchKernelGGL((wty_kernel<TF, 1, FAST>), dim3(blocks), dim3(WTY_WAVES * 64), 0, s, a);
-    else if (a.q == 2) hipLaunchKernelGGL((wty_kernel<TF, 2, FAST>), dim3(blocks), dim3(WTY_WAVES * 64), 0, s, a);
-    else hipLaunchKernelGGL((wty_kernel<TF, 4, FAST>), dim3(blocks), dim3(WTY_WAVES * 64), 0, s, a);
+    const dim3 grid(blocks, (unsigned)((a.q + QB - 1) / QB));
+    hipLaunchKernelGGL((wty_kernel<TF, QB, FAST, WAVES>), grid, dim3(WAVES * 64), 0, s, a);
+}
+
+// All directions in one launch, QB of them a workgroup: more share a weight's
+// decode, fewer give more workgroups (a launch per four directions before).
+// us for 10 directions with QB = 1, 2, 4: bf16 896 x 4864 (152 column units)
+// 10.4, 8.4, 9.6; 896 x 896 (28) 5.7, 6.5, 8.5; FP8 4096 x 14336 (448) 147,
+// 100, 80; MXFP4 4096 x 14336 (112) 81, 66, 68, 4096 x 4096 (32) 41, 34, 45.
+// One direction of few units: 16 waves a workgroup, FP8 4096 x 4096 32 -> 21
+// us, bf16 896 x 896 5.8 -> 3.9 (with more directions their registers spill;
+// with enough workgroups 4 waves are better, 62 against 73 us for 1000 units).
+template <int TF, bool FAST>
+static void wty_launch_blocks(const WtyArgs &a, unsigned blocks, hipStream_t s) {
+    if (a.q == 1 && blocks < 512) wty_launch_q<TF, 1, FAST, 16>(a, blocks, s);
+    else if (a.q == 1) wty_launch_q<TF, 1, FAST, 4>(a, blocks, s);
+    else if (a.q == 2 || (int64_t)blocks * ((a.q + 3) / 4) < 512) wty_launch_q<TF, 2, FAST, 4>(a, blocks, s);
+    else wty_launch_q<TF, 4, FAST, 4>(a, blocks, s);
 }
 
 template <int TF>
 static void wty_launch_fast(const WtyArgs &a, bool fast, unsigned blocks, hipStream_t s) {
     if constexpr (wty_has_fast<TF>()) {
-        if (fast) return wty_launch_q<TF, true>(a, blocks, s);
+        if (fast) return wty_launch_blocks<TF, true>(a, blocks, s);
     }
-    wty_launch_q<TF, false>(a, blocks, s);
+    wty_launch_blocks<TF, false>(a, blocks, s);
 }
 
 // The kind of kernel a tensor takes: its tile format, and whether it takes
@@ -243,26 +257,23 @@ static int wty_kind(const TileView &w) {
     return w.tf * 2 + (fast ? 1 : 0);
 }
 
-// q directions in passes of at most 4 (the accumulators of one pass stay in
-// registers)
+// q directions of every workgroup's columns
 static void wty_launch(int kind, WtyArgs a, int64_t q, unsigned blocks, hipStream_t s) {
     const int tf = kind / 2;
     const bool fast = kind % 2;
-    for (int64_t q0 = 0; q0 < q; q0 += 4) {
-        a.q0 = q0;
-        a.q = q - q0 < 4 ? q - q0 : 4;
-        switch (tf) {
-        case TF_BF16: wty_launch_fast<TF_BF16>(a, fast, blocks, s); break;
-        case TF_F16: wty_launch_fast<TF_F16>(a, fast, blocks, s); break;
-        case TF_F32: wty_launch_fast<TF_F32>(a, fast, blocks, s); break;
-        case TF_Q8: wty_launch_fast<TF_Q8>(a, fast, blocks, s); break;
-        case TF_FP8: wty_launch_fast<TF_FP8>(a, fast, blocks, s); break;
-        case TF_MX4: wty_launch_fast<TF_MX4>(a, fast, blocks, s); break;
-        case TF_INT4: wty_launch_fast<TF_INT4>(a, fast, blocks, s); break;
-        default: throw Error{DITCH_UNSUPPORTED, "matvecTMulti: tile format"};
-        }
-        DITCH_TRY_HIP(hipGetLastError());
+    DITCH_CHECK(q <= 65535, DITCH_UNSUPPORTED, "matvecTMulti: more than 65535 vectors");
+    a.q = q;
+    switch (tf) {
+    case TF_BF16: wty_launch_fast<TF_BF16>(a, fast, blocks, s); break;
+    case TF_F16: wty_launch_fast<TF_F16>(a, fast, blocks, s); break;
+    case TF_F32: wty_launch_fast<TF_F32>(a, fast, blocks, s); break;
+    case TF_Q8: wty_launch_fast<TF_Q8>(a, fast, blocks, s); break;
+    case TF_FP8: wty_launch_fast<TF_FP8>(a, fast, blocks, s); break;
+    case TF_MX4: wty_launch_fast<TF_MX4>(a, fast, blocks, s); break;
+    case TF_INT4: wty_launch_fast<TF_INT4>(a, fast, blocks, s); break;
+    default: throw Error{DITCH_UNSUPPORTED, "matvecTMulti: tile format"};
     }
+    DITCH_TRY_HIP(hipGetLastError());
 }
 
 void launch_matvecT(float *out, const TileView &w, const float *y, int64_t q, hipStream_t s) {

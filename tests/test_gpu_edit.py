@@ -161,3 +161,51 @@ def test_model_edit_ex_then_forward(dev, ref, mode):
             check_parity(ref, rg, lg, rc, lc, f"edit_ex {mode} cache={cache}")
     finally:
         cm.free()
+
+
+# SVD widths q = 2 lora + 4 at the edges of the chunked orthonormalisation's
+# instances (12 | 14, 24 | 26), more directions than it takes beside it, and
+# widths around a chunk of 64 columns
+@pytest.mark.parametrize("rows,cols,k,lora", [(256, 320, 1, 4), (193, 4160, 2, 5), (129, 65, 1, 10), (128, 64, 1, 11),
+                                              (200, 300, 8, 8), (200, 300, 9, 9), (31, 40, 3, 1)])
+def test_full_edit_svd_widths_match_oracle(dev, ref, rows, cols, k, lora):
+    w = _weight("f32", rows, cols, rows + k)
+    rng = np.random.default_rng(rows + k)
+    v = orthonormal_rows(rng, k, rows)
+    ga, gb = dev.edit_delta_ex(w, v, 1.0, "full", lora_rank=lora, seed=5, ablate=lora == 4)
+    ca, cb = ref.edit_delta_ex(w, v, 1.0, MODES["full"], lora_rank=lora, seed=5, ablate=lora == 4)
+    assert ga.shape == ca.shape and gb.shape == cb.shape
+    gd = gb.astype(np.float64) @ ga.astype(np.float64)
+    cd = cb.astype(np.float64) @ ca.astype(np.float64)
+    # the randomised SVD's tail, as in the tests above
+    assert np.linalg.norm(gd - cd) <= 1e-2 * np.linalg.norm(cd)
+
+
+@pytest.mark.parametrize("rank", [0, 1, 3])
+def test_full_edit_of_a_rank_deficient_weight(dev, ref, rank):
+    """Fewer independent columns than SVD vectors: the dependent ones vanish
+    and the factors stay finite."""
+    rng = np.random.default_rng(rank)
+    rows, cols = 96, 130
+    w = (rng.standard_normal((rows, rank)) @ rng.standard_normal((rank, cols))).astype(np.float32) * 0.1
+    v = orthonormal_rows(rng, 1, rows)
+    ga, gb = dev.edit_delta_ex(HostWeight.f32(w), v, 1.0, "full", lora_rank=3, seed=2)
+    assert np.isfinite(ga).all() and np.isfinite(gb).all()
+    ca, cb = ref.edit_delta_ex(HostWeight.f32(w), v, 1.0, MODES["full"], lora_rank=3, seed=2)
+    gd = gb.astype(np.float64) @ ga.astype(np.float64)
+    cd = cb.astype(np.float64) @ ca.astype(np.float64)
+    # directions of rounding noise differ; they carry at most its 1e-6
+    assert np.linalg.norm(gd - cd) <= 1e-2 * np.linalg.norm(cd) + 1e-6 * np.linalg.norm(w)
+
+
+@pytest.mark.parametrize("fmt", ["bf16", "fp8", "mxfp4", "int4", "q8_0", "f32"])
+@pytest.mark.parametrize("k", [1, 2, 3, 9])
+def test_directions_of_one_launch_match_oracle(dev, ref, fmt, k):
+    """A = V^T W with one, two and four directions a workgroup; the last
+    workgroup's beyond k."""
+    w = _weight(fmt, 272, 640, k)
+    v = orthonormal_rows(np.random.default_rng(k), k, 272)
+    ga, gb = dev.edit_delta_ex(w, v, 1.0, "none")
+    ca, cb = ref.edit_delta_ex(w, v, 1.0, MODES["none"])
+    # f32 sums of 272 products in another order: 272 * 2^-24 of the largest
+    assert np.abs(ga - ca).max() <= 2e-5 * np.abs(ca).max() and np.array_equal(gb, cb)
