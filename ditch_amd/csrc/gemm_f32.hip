@@ -292,12 +292,35 @@ __global__ __launch_bounds__(64 * WG * WG * KS) void f32_tile_kernel(GemmParams 
     };
     const int common = U - (KS - 1) * nu;  // units that every slice has (the last one's)
     int s = 0;
-    for (; s + 4 <= common; s += 4) {  // no branch inside: every wait is a count
+    // sums of 512 columns are added to the total: as one chain over K the
+    // error against 64 bits was 2.1e-6 at 13312 columns, so 0.6e-6
+    floatx4 total[2][2];
+#pragma unroll
+    for (int m = 0; m < 2; m++)
+#pragma unroll
+        for (int i = 0; i < 2; i++) total[m][i] = floatx4{0.f, 0.f, 0.f, 0.f};
+    auto fold = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int m = 0; m < 2; m++)
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    total[m][i][r] = __fadd_rn(total[m][i][r], acc[m][i][r]);
+                    acc[m][i][r] = 0.f;
+                }
+    };
+    auto four = [&](int s) __attribute__((always_inline)) {  // no branch inside: every wait is a count
         step(s, even, odd, buf1, buf3, true);
         step(s + 1, odd, even, buf2, buf0, true);
         step(s + 2, even, odd, buf3, buf1, true);
         step(s + 3, odd, even, buf0, buf2, true);
+    };
+    for (; s + 16 <= common; s += 16) {
+        for (int b = 0; b < 16; b += 4) four(s + b);
+        fold();
     }
+    for (; s + 4 <= common; s += 4) four(s);
     for (; s < nu; s += 4) {
         step(s, even, odd, buf1, buf3, false);
         if (s + 1 < nu) step(s + 1, odd, even, buf2, buf0, false);
@@ -305,6 +328,12 @@ __global__ __launch_bounds__(64 * WG * WG * KS) void f32_tile_kernel(GemmParams 
         if (s + 3 < nu) step(s + 3, odd, even, buf0, buf2, false);
     }
     __builtin_amdgcn_s_waitcnt(0x70);  // vmcnt(0): no copy outlives its buffer
+#pragma unroll
+    for (int m = 0; m < 2; m++)
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) acc[m][i][r] = __fadd_rn(total[m][i][r], acc[m][i][r]);
 
     if constexpr (KS == 1) {
         const int64_t t0 = (int64_t)tm * (32 * WG) + wm * 32, r0 = (int64_t)tn * (32 * WG) + wn * 32;
