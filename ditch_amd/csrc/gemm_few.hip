@@ -478,6 +478,9 @@ void launch_tf(const FewCall &c) {
 // 37 / 37; MXFP4 14336 x 4096 on 96 37 / 47, 4096 x 4096 on 128 22 / 49. On
 // long rows the tiled product leaves most CUs without a tile: 4096 x 14336 on
 // 128 tokens FP8 52 / 57, INT4 55 / 60, Q8_0 51 / 167; bf16 on 64 49 / 51.
+// MXFP4 from 128 tokens on is three terms here (what the scaled MFMA holds):
+// 4096 x 4096 on 160 40 / 50, on 200 54 / 51, 1024 x 4096 on 255 24 / 50,
+// 4096 x 14336 on 160 117 / 146, on 200 175 / 146.
 bool few_gemm_takes(const TileView &w, int64_t n, bool exact) {
     if (!w.fast || n < 1 || n > 255 || w.cols < 4) return false;
     const bool bf16 = w.tf == TF_BF16, mx4 = w.tf == TF_MX4, q8 = w.tf == TF_Q8;
@@ -486,6 +489,7 @@ bool few_gemm_takes(const TileView &w, int64_t n, bool exact) {
     if (exact) return false;
     const double work = (double)n * w.rows * w.cols;
     const bool long_k = w.cols >= 8192 && w.rows <= 4096;
+    if (mx4 && w.mx && n >= 128) return work <= (long_k ? 9.4e9 : 2.7e9);
     if (mx4) return work <= (long_k ? 1.5e10 : 5.7e9);
     if (q8) return work <= (long_k ? 1.5e10 : n > 64 ? 4.4e9 : 2.6e9);
     return work <= (long_k ? (bf16 ? 3.8e9 : 7.6e9) : 2.6e9);

@@ -73,3 +73,22 @@ def test_non_finite_activations_stay_in_their_token(dev, ref, n):
     others = [i for i in range(n) if i not in (2, 4)]
     assert not np.isfinite(got[[2, 4]]).any()
     np.testing.assert_array_equal(got[others], clean[others])
+
+
+@pytest.mark.parametrize("n,rows,cols", [(128, 72, 640), (255, 40, 4096)])
+def test_mxfp4_from_128_tokens_keeps_the_scaled_product_s_precision(dev, ref, n, rows, cols):
+    """Three terms, as the fp6 terms of the scaled MFMA hold 18 bits: the error
+    against 64 bits is that of f32 sums (two terms: 2.5e-6)."""
+    rng = np.random.default_rng(n)
+    w = wg.make("mxfp4", rows, cols, rng)
+    x = rng.standard_normal((n, cols)).astype(np.float32)
+    t = dev.upload(w)
+    try:
+        bx, bo = hipmem.Buffer.from_array(x), hipmem.Buffer(n * rows * 4)
+        t.matmul_device(bo.ptr, bx.ptr, n)
+        dev.sync()
+        got = bo.download(np.float32, (n, rows)).astype(np.float64)
+    finally:
+        t.free()
+    want = x.astype(np.float64) @ dequant_f32(ref, w).astype(np.float64).T
+    assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want)
