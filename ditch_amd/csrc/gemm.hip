@@ -131,10 +131,22 @@ static void dispatch_tf(int tf, const GemmParams &p, int64_t max_rows, int64_t n
     DITCH_TRY_HIP(hipGetLastError());
 }
 
+// Where the GEMV beats the few-token product on f32 rows (us GEMV / few-token):
+// bf16 and Q8_0 from 9 tokens on, where the latter needs fragments (bf16 1024
+// x 4096 on 9 8.8 / 9.4, 14336 x 4096 on 16 29 / 31; Q8_0 14336 x 4096 on 9
+// 15.8 / 17.0, 1024 x 4096 9.9 / 9.4), and weights past the 256 MB cache: bf16
+// 89312 x 2048 on 5 59.3 / 63.2, Q8_0 128256 x 4096 on 4 91 / 96, on 8 119 / 112.
+static bool gemv_ahead(const TileView &w, int64_t n) {
+    const int64_t elements = w.rows * w.cols;
+    if (w.tf == TF_BF16) return n <= 16 && (n > 8 || elements > (1 << 27));
+    if (w.tf == TF_Q8) return n <= 16 && (n > 8 ? w.rows >= 4096 : n <= 4 && elements > (1 << 28));
+    return false;
+}
+
 void launch_matmul(const TileView &w, float *out, const float *x, int64_t n, const MatmulEpilogue &ep, hipStream_t s,
                    const int32_t *row_index, DevBuf *ws) {
     if (n <= 0 || w.rows <= 0) return;
-    if (few_gemm_takes(w, n, ep.exact != 0)) {
+    if (few_gemm_takes(w, n, ep.exact != 0) && !(ws && !ep.exact && gemv_ahead(w, n))) {
         // (three terms too where the product they stand in for is the scaled
         // MFMA's, whose fp6 terms hold 18 bits)
         const int xt = ep.exact || mx_gemm_takes(w, n) ? 3 : 2;

@@ -374,10 +374,7 @@ static void gemv_launch(const GemmParams &p, int64_t rows, unsigned nseg, bool l
         const int pp = (int)((p.n * UK / 2 + 63) / 64);
         const bool full = p.w.cols % UK == 0 && (p.ldx & 1) == 0 && ((uintptr_t)p.x & 7) == 0 && nseg == 1 &&
                           !p.row_index && (uint64_t)p.n * p.ldx * 4 < (1ull << 32);
-        // (bf16 and Q8_0 rows of that kind go to the few-token product)
-        constexpr bool CP = TF != TF_BF16 && TF != TF_Q8;
-        if constexpr (!CP) hipLaunchKernelGGL((gemv_kernel<TF, NT, XT, D, W, true>), grid, dim3(64 * W), 0, s, p);
-        else if (XT == 2 && full && pp == 1 && p.n == 1)
+        if (XT == 2 && full && pp == 1 && p.n == 1)
             hipLaunchKernelGGL((gemv_kernel<TF, NT, XT, D, W, true, 1, 1>), grid, dim3(64 * W), 0, s, p);
         else if (XT == 2 && full && pp == 1)
             hipLaunchKernelGGL((gemv_kernel<TF, NT, XT, D, W, true, 1>), grid, dim3(64 * W), 0, s, p);
