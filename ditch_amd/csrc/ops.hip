@@ -515,95 +515,127 @@ __global__ void softmax_kernel(float *x, int64_t len) {
     for (int64_t i = threadIdx.x; i < len; i += blockDim.x) xr[i] = __fmul_rn(xr[i], inv);
 }
 
-// log-softmax (tensor.zig:1203-1210): f32 max, f64 sum of exp, f32 x - lse.
 // log-softmax and KL over long rows (tensor.zig:1203-1210, scorers.zig:
-// 387-394), each row split into `S` chunks so that a few rows of a 128 k
-// vocabulary still spread over every CU. The arithmetic is the reference's:
-// the f32 row maximum m (exact in any order), then s = sum exp(f64(x - m))
-// in f64 with x - m taken in f32, lse = m + f32(log s), out = x - lse.
-//   pass 1  per chunk: its maximum                         -> part_m[row][S]
-//   pass 2  per chunk: m = max of the row's part_m, the chunk's f64 sum
-//                                                          -> part_s[row][S]
-//   pass 3  per chunk: s = the row's part_s added in chunk order, lse, and
-//           the chunk's outputs (log-probs, or the KL terms -> part_k)
-//   pass 4  (KL only) per row: part_k added in chunk order.
-struct RowSplit {
-    int64_t len, chunk;
-    int S;
-};
+// 387-394), each row in chunks of ROW_CHUNK so that a few rows of a 128 k
+// vocabulary still spread over every CU. As the reference: the f32 row
+// maximum m, s = sum exp(x - m) in f64, lse = m + f32(log s), out = x - lse.
+//   pass 1  per chunk, held in registers (one read): its maximum m_c and
+//           s_c = sum exp(x - m_c), the difference taken in f64
+//   pass 2  per chunk: s = sum s_c exp(m_c - m) over the row's chunks, lse,
+//           and the chunk's outputs (log-probs, or the KL terms -> part_k)
+//   pass 3  (KL only) per row: part_k added by a wave.
+// The chunking depends on the row's length alone, so a row has the same lse in
+// both functions and the KL of a row against its own log-probs is 0. Bound by
+// memory, then by the f64 exponentials: 64 rows of 151936, log-softmax and KL
+// 182 -> 77 us (the maximum had a pass of its own, and each workgroup added the
+// row's parts one after the other).
+constexpr int ROW_CHUNK = 2048;  // 256 threads x 8
 
-__global__ __launch_bounds__(256) void rowsplit_max_kernel(float *part_m, const float *x, RowSplit rs) {
-    __shared__ float sh[8];
-    const int64_t row = blockIdx.y, c = blockIdx.x;
-    const float *xr = x + row * rs.len;
-    const int64_t i0 = c * rs.chunk, i1 = i0 + rs.chunk < rs.len ? i0 + rs.chunk : rs.len;
-    float m = -INFINITY;
-    for (int64_t i = i0 + threadIdx.x; i < i1; i += blockDim.x) m = fmaxf(m, xr[i]);
-    m = block_max(m, sh);
-    if (threadIdx.x == 0) part_m[row * rs.S + c] = m;
+// element j of a thread's 8 (VEC: two float4 runs of the chunk)
+template <bool VEC> __device__ __forceinline__ int row_elem(int j) {
+    return VEC ? (j / 4) * 1024 + 4 * threadIdx.x + j % 4 : j * 256 + threadIdx.x;
+}
+template <bool VEC>
+__device__ __forceinline__ void row_load(float (&v)[8], const float *x, int count, float fill) {
+#pragma unroll
+    for (int j = 0; j < 8; j += VEC ? 4 : 1) {
+        const int e = row_elem<VEC>(j);
+        if constexpr (VEC) {
+            const float4 f = e < count ? *(const float4 *)(x + e) : make_float4(fill, fill, fill, fill);
+            v[j] = f.x; v[j + 1] = f.y; v[j + 2] = f.z; v[j + 3] = f.w;
+        } else {
+            v[j] = e < count ? x[e] : fill;
+        }
+    }
 }
 
-__device__ __forceinline__ float rowsplit_row_max(const float *part_m, int64_t row, int S) {
+template <bool VEC>
+__global__ __launch_bounds__(256) void rowpart_kernel(float *part_m, double *part_s, const float *x, int64_t len) {
+    __shared__ float shm[8];
+    __shared__ double shs[8];
+    const int64_t row = blockIdx.y, c = blockIdx.x, i0 = c * ROW_CHUNK;
+    const int count = (int)(len - i0 < ROW_CHUNK ? len - i0 : ROW_CHUNK);
+    float v[8];
+    row_load<VEC>(v, x + row * len + i0, count, -INFINITY);
     float m = -INFINITY;
-    for (int c = 0; c < S; c++) m = fmaxf(m, part_m[row * S + c]);
-    return m;
-}
-
-__global__ __launch_bounds__(256) void rowsplit_sum_kernel(double *part_s, const float *part_m, const float *x,
-                                                           RowSplit rs) {
-    __shared__ double sh[8];
-    const int64_t row = blockIdx.y, c = blockIdx.x;
-    const float m = rowsplit_row_max(part_m, row, rs.S);
-    const float *xr = x + row * rs.len;
-    const int64_t i0 = c * rs.chunk, i1 = i0 + rs.chunk < rs.len ? i0 + rs.chunk : rs.len;
+#pragma unroll
+    for (int j = 0; j < 8; j++) m = fmaxf(m, v[j]);
+    m = block_max(m, shm);
+    const double ref = m == -INFINITY ? 0.0 : (double)m;  // (a chunk of -inf adds 0, NaN stays)
     double acc = 0.0;
-    for (int64_t i = i0 + threadIdx.x; i < i1; i += blockDim.x) acc += exp((double)__fsub_rn(xr[i], m));
-    acc = block_sum_d(acc, sh);
-    if (threadIdx.x == 0) part_s[row * rs.S + c] = acc;
+#pragma unroll
+    for (int j = 0; j < 8; j++) acc += exp((double)v[j] - ref);  // (past the row: exp(-inf))
+    acc = block_sum_d(acc, shs);
+    if (threadIdx.x == 0) {
+        part_m[row * gridDim.x + c] = m;
+        part_s[row * gridDim.x + c] = acc;
+    }
 }
 
-__device__ __forceinline__ float rowsplit_lse(const double *part_s, const float *part_m, int64_t row, int S) {
-    const float m = rowsplit_row_max(part_m, row, S);
+// a row's lse from its S chunks, by every wave (the same sums in each)
+__device__ __forceinline__ float rowpart_lse(const double *part_s, const float *part_m, int64_t row, int S) {
+    const int lane = threadIdx.x & 63;
+    float m = -INFINITY;
+    for (int c = lane; c < S; c += 64) m = fmaxf(m, part_m[row * S + c]);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
     double s = 0.0;
-    for (int c = 0; c < S; c++) s += part_s[row * S + c];
+    for (int c = lane; c < S; c += 64) s += part_s[row * S + c] * exp((double)part_m[row * S + c] - (double)m);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
     return __fadd_rn(m, (float)log(s));
 }
 
-__global__ __launch_bounds__(256) void rowsplit_logsoftmax_kernel(float *out, const double *part_s,
-                                                                  const float *part_m, const float *x, RowSplit rs) {
-    const int64_t row = blockIdx.y, c = blockIdx.x;
-    const float lse = rowsplit_lse(part_s, part_m, row, rs.S);
-    const float *xr = x + row * rs.len;
-    float *o = out + row * rs.len;
-    const int64_t i0 = c * rs.chunk, i1 = i0 + rs.chunk < rs.len ? i0 + rs.chunk : rs.len;
-    for (int64_t i = i0 + threadIdx.x; i < i1; i += blockDim.x) o[i] = __fsub_rn(xr[i], lse);
+template <bool VEC>
+__global__ __launch_bounds__(256) void rowpart_logsoftmax_kernel(float *out, const double *part_s, const float *part_m,
+                                                                 const float *x, int64_t len) {
+    const int64_t row = blockIdx.y, c = blockIdx.x, i0 = c * ROW_CHUNK;
+    const int count = (int)(len - i0 < ROW_CHUNK ? len - i0 : ROW_CHUNK);
+    float v[8];
+    row_load<VEC>(v, x + row * len + i0, count, 0.f);
+    const float lse = rowpart_lse(part_s, part_m, row, gridDim.x);
+    float *o = out + row * len + i0;
+#pragma unroll
+    for (int j = 0; j < 8; j += VEC ? 4 : 1) {
+        const int e = row_elem<VEC>(j);
+        if (e >= count) continue;
+        if constexpr (VEC)
+            *(float4 *)(o + e) = make_float4(__fsub_rn(v[j], lse), __fsub_rn(v[j + 1], lse), __fsub_rn(v[j + 2], lse),
+                                             __fsub_rn(v[j + 3], lse));
+        else o[e] = __fsub_rn(v[j], lse);
+    }
 }
 
 // KL terms of one chunk: sum exp(lb) (lb - lt) in f64 with lt = t - lse
 // (scorers.zig:390-394)
-__global__ __launch_bounds__(256) void rowsplit_kl_kernel(double *part_k, const double *part_s, const float *part_m,
-                                                          const float *base, const float *trial, RowSplit rs) {
+template <bool VEC>
+__global__ __launch_bounds__(256) void rowpart_kl_kernel(double *part_k, const double *part_s, const float *part_m,
+                                                         const float *base, const float *trial, int64_t len) {
     __shared__ double sh[8];
-    const int64_t row = blockIdx.y, c = blockIdx.x;
-    const float lse = rowsplit_lse(part_s, part_m, row, rs.S);
-    const float *tr = trial + row * rs.len, *br = base + row * rs.len;
-    const int64_t i0 = c * rs.chunk, i1 = i0 + rs.chunk < rs.len ? i0 + rs.chunk : rs.len;
+    const int64_t row = blockIdx.y, c = blockIdx.x, i0 = c * ROW_CHUNK;
+    const int count = (int)(len - i0 < ROW_CHUNK ? len - i0 : ROW_CHUNK);
+    float b[8], t[8];
+    row_load<VEC>(b, base + row * len + i0, count, 0.f);
+    row_load<VEC>(t, trial + row * len + i0, count, 0.f);
+    const float lse = rowpart_lse(part_s, part_m, row, gridDim.x);
     double acc = 0.0;
-    for (int64_t i = i0 + threadIdx.x; i < i1; i += blockDim.x) {
-        const double lb = (double)br[i];
-        const double lt = (double)__fsub_rn(tr[i], lse);
-        acc += exp(lb) * (lb - lt);
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        const double lb = (double)b[j], lt = (double)__fsub_rn(t[j], lse), term = exp(lb) * (lb - lt);
+        if (row_elem<VEC>(j) < count) acc += term;
     }
     acc = block_sum_d(acc, sh);
-    if (threadIdx.x == 0) part_k[row * rs.S + c] = acc;
+    if (threadIdx.x == 0) part_k[row * gridDim.x + c] = acc;
 }
 
-__global__ void rowsplit_kl_total_kernel(double *kl, const double *part_k, int64_t n, int S) {
-    const int64_t row = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+__global__ void rowpart_kl_total_kernel(double *kl, const double *part_k, int64_t n, int S) {
+    const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= n) return;
     double s = 0.0;
-    for (int c = 0; c < S; c++) s += part_k[row * S + c];
-    kl[row] = s;
+    for (int c = threadIdx.x & 63; c < S; c += 64) s += part_k[row * S + c];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    if ((threadIdx.x & 63) == 0) kl[row] = s;
 }
 
 // out[i][j] = act(gate[i][j]) * up[i][j] (tensor.zig:1296-1337)
@@ -785,44 +817,34 @@ void launch_softmax_rows(float *x, int64_t n, int64_t len, hipStream_t s) {
     hipLaunchKernelGGL(softmax_kernel, dim3((unsigned)n), dim3(256), 0, s, x, len);
     DITCH_TRY_HIP(hipGetLastError());
 }
-// Chunks per row: enough workgroups to cover the CUs about twice, chunks
-// of at least 2048 elements.
-static RowSplit row_split(int64_t n, int64_t len) {
-    int64_t S = (512 + n - 1) / n;
-    const int64_t most = (len + 2047) / 2048;
-    S = S < most ? S : most;
-    S = S < 1 ? 1 : S;
-    RowSplit rs;
-    rs.len = len;
-    rs.chunk = (len + S - 1) / S;
-    rs.S = (int)((len + rs.chunk - 1) / rs.chunk);
-    return rs;
-}
-
-// part_m [n][S] f32, part_s [n][S] f64 (and part_k [n][S] f64 for KL) in `tmp`
-static void row_split_passes(const RowSplit &rs, const float *x, int64_t n, float *&pm, double *&ps, double **pk,
-                             hipStream_t s, DevBuf *tmp) {
-    const size_t cells = (size_t)n * rs.S;
-    double *d = tmp->get<double>(3 * cells);
-    ps = d;
-    if (pk) *pk = d + cells;
-    pm = (float *)(d + 2 * cells);
-    dim3 grid((unsigned)rs.S, (unsigned)n);
-    hipLaunchKernelGGL(rowsplit_max_kernel, grid, dim3(256), 0, s, pm, x, rs);
+// Pass 1 into `tmp`: s_c [n][S] f64, room for the KL parts, m_c [n][S] f32.
+// Rows of whole float4s at aligned addresses are read so.
+struct RowParts {
+    double *s, *k;
+    float *m;
+    dim3 grid;
+    bool vec;
+};
+static RowParts row_parts(const float *x, const void *other, int64_t n, int64_t len, hipStream_t s, DevBuf *tmp) {
+    const int64_t S = (len + ROW_CHUNK - 1) / ROW_CHUNK, cells = n * S;
+    RowParts r;
+    r.s = tmp->get<double>(3 * cells);
+    r.k = r.s + cells;
+    r.m = (float *)(r.k + cells);
+    r.grid = dim3((unsigned)S, (unsigned)n);
+    r.vec = len % 4 == 0 && (((uintptr_t)x | (uintptr_t)other) & 15) == 0;
+    if (r.vec) hipLaunchKernelGGL(rowpart_kernel<true>, r.grid, dim3(256), 0, s, r.m, r.s, x, len);
+    else hipLaunchKernelGGL(rowpart_kernel<false>, r.grid, dim3(256), 0, s, r.m, r.s, x, len);
     DITCH_TRY_HIP(hipGetLastError());
-    hipLaunchKernelGGL(rowsplit_sum_kernel, grid, dim3(256), 0, s, ps, pm, x, rs);
-    DITCH_TRY_HIP(hipGetLastError());
+    return r;
 }
 
 void launch_log_softmax_rows(float *out, const float *x, int64_t n, int64_t len, hipStream_t s, DevBuf *tmp) {
     if (n <= 0 || len <= 0) return;
     DITCH_CHECK(n <= 65535, DITCH_UNSUPPORTED, "log-softmax: more than 65535 rows in one call");
-    const RowSplit rs = row_split(n, len);
-    float *pm;
-    double *ps;
-    row_split_passes(rs, x, n, pm, ps, nullptr, s, tmp);
-    hipLaunchKernelGGL(rowsplit_logsoftmax_kernel, dim3((unsigned)rs.S, (unsigned)n), dim3(256), 0, s, out, ps, pm, x,
-                       rs);
+    const RowParts r = row_parts(x, out, n, len, s, tmp);
+    if (r.vec) hipLaunchKernelGGL(rowpart_logsoftmax_kernel<true>, r.grid, dim3(256), 0, s, out, r.s, r.m, x, len);
+    else hipLaunchKernelGGL(rowpart_logsoftmax_kernel<false>, r.grid, dim3(256), 0, s, out, r.s, r.m, x, len);
     DITCH_TRY_HIP(hipGetLastError());
 }
 void launch_kl_rows(double *kl, const float *base, const float *trial, int64_t n, int64_t vocab, hipStream_t s,
@@ -830,14 +852,12 @@ void launch_kl_rows(double *kl, const float *base, const float *trial, int64_t n
     if (n <= 0) return;
     DITCH_CHECK(n <= 65535, DITCH_UNSUPPORTED, "KL: more than 65535 rows in one call");
     DITCH_CHECK(vocab > 0, DITCH_INVALID_ARGUMENT, "KL: empty rows");
-    const RowSplit rs = row_split(n, vocab);
-    float *pm;
-    double *ps, *pk;
-    row_split_passes(rs, trial, n, pm, ps, &pk, s, tmp);
-    hipLaunchKernelGGL(rowsplit_kl_kernel, dim3((unsigned)rs.S, (unsigned)n), dim3(256), 0, s, pk, ps, pm, base, trial,
-                       rs);
+    const RowParts r = row_parts(trial, base, n, vocab, s, tmp);
+    if (r.vec) hipLaunchKernelGGL(rowpart_kl_kernel<true>, r.grid, dim3(256), 0, s, r.k, r.s, r.m, base, trial, vocab);
+    else hipLaunchKernelGGL(rowpart_kl_kernel<false>, r.grid, dim3(256), 0, s, r.k, r.s, r.m, base, trial, vocab);
     DITCH_TRY_HIP(hipGetLastError());
-    hipLaunchKernelGGL(rowsplit_kl_total_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, kl, pk, n, rs.S);
+    hipLaunchKernelGGL(rowpart_kl_total_kernel, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, s, kl, r.k, n,
+                       (int)r.grid.x);
     DITCH_TRY_HIP(hipGetLastError());
 }
 void launch_gated_act(uint32_t act, float *out, const float *gate, const float *up, int64_t n, int64_t len,

@@ -61,3 +61,23 @@ def test_forward_token_counts_match_oracle(dev, ref, fmt):
     finally:
         gm.free()
         cm.free()
+
+
+# one element, the edges of a 2048-element chunk, of the lanes that add 64
+# chunks, and rows that are not whole float4s
+@pytest.mark.parametrize("V", [1, 2047, 2048, 2052, 133120, 131073])
+def test_log_softmax_and_kl_row_lengths(dev, ref, V):
+    rng = np.random.default_rng(V)
+    x = (rng.standard_normal((3, V)) * 5).astype(np.float32)
+    x[1, : V // 2] = -np.inf  # whole chunks of masked logits
+    x[2, 0] = 80.0
+    lp = dev.logSoftmaxRows(x)
+    want = ref.log_softmax_rows(x)
+    fin = np.isfinite(want)
+    # one f32 rounding of lse and one of the difference, at most 100 large
+    assert np.array_equal(fin, np.isfinite(lp)) and np.abs(lp[fin] - want[fin]).max() <= 4 * 2.0**-24 * 128
+    # a row against its own log-probs; masked logits on both sides are NaN (0 * inf)
+    kl = dev.klRows(lp, x)
+    assert kl[0] == 0 and kl[2] == 0
+    if V > 1:
+        assert np.isnan(kl[1]) and np.isnan(ref.kl_rows(want, x)[1])
