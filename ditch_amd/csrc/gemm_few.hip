@@ -50,6 +50,12 @@ template <int MATS> struct FewParams {
     uint8_t *ys;
     int64_t ldk_y;
     uint32_t act;
+    // SEG: segment blockIdx.y's matrices and rows (mat[] unused)
+    const GroupSeg *segs, *segs_up;
+    const int32_t *row_index;
+    const float *delta_xa;
+    int delta_stride;
+    float *out;
 };
 
 // weight units and side words per row group of a 128-column step
@@ -87,8 +93,11 @@ __device__ __forceinline__ uint32_t next_term(float &a, float &b) {
 
 // GLU: mat[0] and mat[1] are gate and up; a workgroup takes OT row groups of
 // both, and its epilogue writes act(gate) * up of the summed tiles.
-template <int TF, int MT, int OT, int W, int XT, int NX, int MATS, bool GLU>
+// SEG: a segment (a routed expert) a blockIdx.y, up to NX of its rows gathered
+// by row_index (or consecutive), from f32 rows.
+template <int TF, int MT, int OT, int W, int XT, int NX, int MATS, bool GLU, bool SEG = false>
 __global__ __launch_bounds__(64 * W) void few_kernel(FewParams<MATS> p) {
+    static_assert(!SEG || (NX > 1 && MT == 1), "segments read f32 rows");
     constexpr int UPS = Few<TF>::UPS, NS = Few<TF>::NS;
     constexpr int NT = GLU ? 2 * OT : OT;  // row groups in registers
     typedef FewSlot<XT, NX> Slot;
@@ -112,13 +121,15 @@ __global__ __launch_bounds__(64 * W) void few_kernel(FewParams<MATS> p) {
         }
     }
     int mi = 0;
-    if constexpr (!GLU) {
+    if constexpr (!GLU && !SEG) {
 #pragma unroll
         for (int i = 0; i + 1 < MATS; i++) mi += rb >= p.end[i];
         if (mi) rb -= p.end[mi - 1];
     }
     const FewMat &mat = p.mat[mi];
-    const TileView &w = mat.w;
+    const GroupSeg *seg = SEG ? p.segs + blockIdx.y : nullptr;
+    const TileView &w = SEG ? seg->w : mat.w;
+    const int64_t n = SEG ? seg->cnt : p.n, off = SEG ? seg->off : 0;
     const int64_t groups = (w.rows + 15) / 16, g0 = (int64_t)rb * OT, units = w.units_k, K = w.cols;
     const int steps = (int)((units + UPS - 1) / UPS), per = (steps + W - 1) / W;
     const int s0 = wave * per < steps ? wave * per : steps, s1 = s0 + per < steps ? s0 + per : steps;
@@ -130,7 +141,7 @@ __global__ __launch_bounds__(64 * W) void few_kernel(FewParams<MATS> p) {
     if constexpr (TF == TF_FP8 || TF == TF_INT4) st = side_step<TF>(w);
 #pragma unroll
     for (int i = 0; i < NT; i++) {
-        const TileView &wi = GLU && i >= OT ? p.mat[MATS - 1].w : w;
+        const TileView &wi = GLU && i >= OT ? (SEG ? p.segs_up[blockIdx.y].w : p.mat[MATS - 1].w) : w;
         const int64_t g = g0 + i % OT < groups ? g0 + i % OT : groups - 1;
         wb[i] = wi.codes + g * units * 1024;
         if constexpr (NS > 0) sb[i] = wi.side + side_row(wi, g, lane);
@@ -151,6 +162,15 @@ __global__ __launch_bounds__(64 * W) void few_kernel(FewParams<MATS> p) {
         }
     }
 
+    const float *xr[SEG ? NX / 2 : 1];
+    if constexpr (SEG) {
+#pragma unroll
+        for (int m = 0; m < NX / 2; m++) {
+            const int64_t tok = 2 * m + (lane >> 5), r = off + (tok < n ? tok : n - 1);
+            xr[m] = p.x + (p.row_index ? (int64_t)p.row_index[r] : r) * p.ldx;
+        }
+    }
+
     typedef FewSet<TF, MT, NT, XT, NX> Set;
     auto fetch = [&](Set &v, int s) __attribute__((always_inline)) {
         if constexpr (NX == 1) {
@@ -161,7 +181,8 @@ __global__ __launch_bounds__(64 * W) void few_kernel(FewParams<MATS> p) {
 #pragma unroll
             for (int m = 0; m < NX / 2; m++) {
                 const int64_t tok = 2 * m + (lane >> 5);
-                v.xp[m] = gload<float4>(p.x + (tok < p.n ? tok : p.n - 1) * p.ldx + kc);
+                if constexpr (SEG) v.xp[m] = gload<float4>(xr[m] + kc);
+                else v.xp[m] = gload<float4>(p.x + (tok < n ? tok : n - 1) * p.ldx + kc);
             }
         }
 #pragma unroll
@@ -312,7 +333,7 @@ __global__ __launch_bounds__(64 * W) void few_kernel(FewParams<MATS> p) {
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
                     const int64_t tok = blk * 16 + 4 * kq + r;
-                    if (tok < p.n && row < w.rows) p.y[tok * w.rows + row] = v[r];
+                    if (tok < n && row < w.rows) p.y[(off + tok) * w.rows + row] = v[r];
                 }
             }
             if (p.ys) {
@@ -339,13 +360,21 @@ __global__ __launch_bounds__(64 * W) void few_kernel(FewParams<MATS> p) {
     }
     GemmParams e{};
     e.w.rows = w.rows;
-    e.out = mat.out;
-    e.n = p.n;
-    e.bias = mat.bias;
-    e.accumulate = mat.accumulate;
-    e.delta_b = mat.delta_b;
-    e.delta_xa = mat.delta_xa;
-    e.delta_rank = e.delta_stride = mat.delta_rank;
+    e.n = n;
+    if constexpr (SEG) {
+        e.out = p.out + off * w.rows;
+        e.delta_b = seg->delta_b;
+        e.delta_xa = p.delta_xa + off * p.delta_stride;
+        e.delta_rank = seg->delta_rank;
+        e.delta_stride = p.delta_stride;
+    } else {
+        e.out = mat.out;
+        e.bias = mat.bias;
+        e.accumulate = mat.accumulate;
+        e.delta_b = mat.delta_b;
+        e.delta_xa = mat.delta_xa;
+        e.delta_rank = e.delta_stride = mat.delta_rank;
+    }
     for (int q = wave; q < MT * NT; q += W) {
         floatx4 v[1][1] = {{total(q)}};
         const int64_t tok[1] = {((int64_t)tb * MT + q / NT) * 16 + 4 * kq}, row[1] = {(g0 + q % NT) * 16 + c16};
@@ -467,6 +496,31 @@ void launch_tf(const FewCall &c) {
     }
 }
 
+// 16 rows and four K slices a workgroup: the segments fill the CUs
+template <int TF, int NX, bool GLU>
+void launch_segs_nx(const FewParams<1> &q, int64_t groups, unsigned nseg, hipStream_t s) {
+    hipLaunchKernelGGL((few_kernel<TF, 1, 1, 4, 2, NX, 1, GLU, true>), dim3((unsigned)groups, nseg), dim3(256), 0, s, q);
+}
+template <int TF, bool GLU>
+void launch_segs(const FewParams<1> &q, int64_t groups, unsigned nseg, int64_t max_cnt, hipStream_t s) {
+    if (max_cnt <= 2) launch_segs_nx<TF, 2, GLU>(q, groups, nseg, s);
+    else if (max_cnt <= 4) launch_segs_nx<TF, 4, GLU>(q, groups, nseg, s);
+    else launch_segs_nx<TF, 8, GLU>(q, groups, nseg, s);
+}
+template <bool GLU>
+void launch_segs_tf(int tf, const FewParams<1> &q, int64_t rows, unsigned nseg, int64_t max_cnt, hipStream_t s) {
+    const int64_t groups = (rows + 15) / 16;
+    switch (tf) {
+    case TF_BF16: launch_segs<TF_BF16, GLU>(q, groups, nseg, max_cnt, s); break;
+    case TF_Q8: launch_segs<TF_Q8, GLU>(q, groups, nseg, max_cnt, s); break;
+    case TF_FP8: launch_segs<TF_FP8, GLU>(q, groups, nseg, max_cnt, s); break;
+    case TF_MX4: launch_segs<TF_MX4, GLU>(q, groups, nseg, max_cnt, s); break;
+    case TF_INT4: launch_segs<TF_INT4, GLU>(q, groups, nseg, max_cnt, s); break;
+    default: throw Error{DITCH_UNSUPPORTED, "few-token segments: format"};
+    }
+    DITCH_TRY_HIP(hipGetLastError());
+}
+
 }  // namespace
 
 // Up to 32 tokens for every shape; above that while the product is small
@@ -550,6 +604,46 @@ void launch_few_glu(const TileView &gate, const TileView &up, uint32_t act, floa
     default: throw Error{DITCH_UNSUPPORTED, "few-token gate/up: format"};
     }
     DITCH_TRY_HIP(hipGetLastError());
+}
+
+bool few_grouped_takes(const GroupSeg *segs, unsigned nseg, int64_t max_cnt) {
+    if (nseg < 1 || nseg > 65535 || max_cnt > 8) return false;
+    const TileView &f = segs[0].w;
+    for (unsigned i = 0; i < nseg; i++) {
+        const TileView &w = segs[i].w;
+        if (segs[i].cnt < 1 || segs[i].cnt > max_cnt || !few_gemm_takes(w, segs[i].cnt, false) || w.cols % 4 != 0 ||
+            w.tf != f.tf || w.rows != f.rows || w.cols != f.cols)
+            return false;
+    }
+    return true;
+}
+
+void launch_few_grouped(const GroupSeg *d_segs, const TileView &shape, unsigned nseg, int64_t max_cnt, float *out,
+                        const float *x, const float *delta_xa, int delta_stride, hipStream_t s) {
+    FewParams<1> q{};
+    q.segs = d_segs;
+    q.x = x;
+    q.ldx = shape.cols;
+    q.out = out;
+    q.delta_xa = delta_xa;
+    q.delta_stride = delta_stride;
+    q.tblocks = 1;
+    launch_segs_tf<false>(shape.tf, q, shape.rows, nseg, max_cnt, s);
+}
+
+void launch_few_glu_grouped(const GroupSeg *d_gate, const GroupSeg *d_up, const TileView &shape, unsigned nseg,
+                            int64_t max_cnt, uint32_t act, float *y, const float *x, const int32_t *row_index,
+                            hipStream_t s) {
+    FewParams<1> q{};
+    q.segs = d_gate;
+    q.segs_up = d_up;
+    q.x = x;
+    q.ldx = shape.cols;
+    q.row_index = row_index;
+    q.y = y;
+    q.act = act;
+    q.tblocks = 1;
+    launch_segs_tf<true>(shape.tf, q, shape.rows, nseg, max_cnt, s);
 }
 
 }  // namespace ditch

@@ -1308,7 +1308,16 @@ static void moe_forward(ditch_hip_model *m, Layer &L, float *x, const float *h, 
         const bool fused = tile_grouped_takes(sg.data(), nseg, max_cnt) && tile_grouped_takes(sd.data(), nseg, max_cnt) &&
                            tile_glu_takes(vg, su[0].w, 128);
         const void *dfr = nullptr;
-        if (fused) {
+        // up to 8 rows an expert (decode steps): the few-token kernel, as above
+        // with f32 rows (2 layers of 128 experts of 2048 x 768 INT4, 4 rows:
+        // 63 + 63 + 5 us for gate, up and SwiGLU and 73 for down with the GEMV, 23
+        // and 12 here)
+        const bool few = !fused && few_grouped_takes(sg.data(), nseg, max_cnt) && few_grouped_takes(su.data(), nseg, max_cnt) &&
+                         few_grouped_takes(sd.data(), nseg, max_cnt) && sg[0].w.tf == su[0].w.tf &&
+                         sg[0].w.rows == su[0].w.rows;
+        if (few) {
+            launch_few_glu_grouped(dsegs, dsegs + nseg, vg, nseg, max_cnt, 0, gate, h, pair_token, s);
+        } else if (fused) {
             const int64_t ldk_d = split_k_tiles(vd);
             void *fr = m->acts.get<uint8_t>(split_bytes_ldk(grouped_blocks(sg.data(), nseg) * 16, ldk_d, 2));
             // a chunk of at least n pairs: the n token rows split once and gathered
@@ -1338,6 +1347,8 @@ static void moe_forward(ditch_hip_model *m, Layer &L, float *x, const float *h, 
         if (dfr)
             launch_tile_gemm_grouped(dsegs + 2 * nseg, sd.data(), nseg, eo, hidden, nullptr, inter, nullptr, dxa, max_rank,
                                      &m->xsplit, &m->gmeta, s, dfr);
+        else if (few)
+            launch_few_grouped(dsegs + 2 * nseg, vd, nseg, max_cnt, eo, gate, dxa, max_rank, s);
         else
             launch_matmul_grouped(dsegs + 2 * nseg, sd.data(), nseg, vd.tf, hidden, inter, max_cnt, eo, gate, nullptr,
                                   dxa, max_rank, s, &m->xsplit, &m->gmeta);
