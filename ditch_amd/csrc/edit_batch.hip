@@ -15,6 +15,7 @@
 // launch, and the result does not depend on timing. Like the reference, a
 // row whose y is 0 contributes nothing (0 times a non-finite weight
 // included).
+#include <algorithm>
 #include <map>
 
 #include "gemm_common.h"
@@ -33,7 +34,7 @@ struct WtyArgs {
     const WtySeg *segs;     // device table, or NULL: the one segment `one`
     const int64_t *items;   // per workgroup: segment << 32 | unit (with segs)
     WtySeg one;
-    int64_t q;              // directions, QB of them a workgroup (blockIdx.y)
+    int64_t q0, q;          // directions q0 .. q, QB of them a workgroup (blockIdx.y)
 };
 
 constexpr int WTY_STEP = 4;  // row groups whose loads are in flight together
@@ -140,7 +141,7 @@ __global__ __launch_bounds__(WAVES * 64) void wty_kernel(WtyArgs a) {
     float *out = sp->out;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int r16 = lane & 15, kq = lane >> 4;
-    const int64_t groups = (w.rows + 15) / 16, q0 = (int64_t)blockIdx.y * QB;
+    const int64_t groups = (w.rows + 15) / 16, q0 = a.q0 + (int64_t)blockIdx.y * QB;
     float acc[QB][NV];
 #pragma unroll
     for (int j = 0; j < QB; j++)
@@ -222,7 +223,7 @@ __global__ __launch_bounds__(WAVES * 64) void wty_kernel(WtyArgs a) {
 
 template <int TF, int QB, bool FAST, int WAVES>
 static void wty_launch_q(const WtyArgs &a, unsigned blocks, hipStream_t s) {
-    const dim3 grid(blocks, (unsigned)((a.q + QB - 1) / QB));
+    const dim3 grid(blocks, (unsigned)((a.q - a.q0 + QB - 1) / QB));
     hipLaunchKernelGGL((wty_kernel<TF, QB, FAST, WAVES>), grid, dim3(WAVES * 64), 0, s, a);
 }
 
@@ -261,19 +262,21 @@ static int wty_kind(const TileView &w) {
 static void wty_launch(int kind, WtyArgs a, int64_t q, unsigned blocks, hipStream_t s) {
     const int tf = kind / 2;
     const bool fast = kind % 2;
-    DITCH_CHECK(q <= 65535, DITCH_UNSUPPORTED, "matvecTMulti: more than 65535 vectors");
-    a.q = q;
-    switch (tf) {
-    case TF_BF16: wty_launch_fast<TF_BF16>(a, fast, blocks, s); break;
-    case TF_F16: wty_launch_fast<TF_F16>(a, fast, blocks, s); break;
-    case TF_F32: wty_launch_fast<TF_F32>(a, fast, blocks, s); break;
-    case TF_Q8: wty_launch_fast<TF_Q8>(a, fast, blocks, s); break;
-    case TF_FP8: wty_launch_fast<TF_FP8>(a, fast, blocks, s); break;
-    case TF_MX4: wty_launch_fast<TF_MX4>(a, fast, blocks, s); break;
-    case TF_INT4: wty_launch_fast<TF_INT4>(a, fast, blocks, s); break;
-    default: throw Error{DITCH_UNSUPPORTED, "matvecTMulti: tile format"};
+    for (int64_t q0 = 0; q0 < q; q0 += 65532) {  // (a grid's rows)
+        a.q0 = q0;
+        a.q = std::min<int64_t>(q, q0 + 65532);
+        switch (tf) {
+        case TF_BF16: wty_launch_fast<TF_BF16>(a, fast, blocks, s); break;
+        case TF_F16: wty_launch_fast<TF_F16>(a, fast, blocks, s); break;
+        case TF_F32: wty_launch_fast<TF_F32>(a, fast, blocks, s); break;
+        case TF_Q8: wty_launch_fast<TF_Q8>(a, fast, blocks, s); break;
+        case TF_FP8: wty_launch_fast<TF_FP8>(a, fast, blocks, s); break;
+        case TF_MX4: wty_launch_fast<TF_MX4>(a, fast, blocks, s); break;
+        case TF_INT4: wty_launch_fast<TF_INT4>(a, fast, blocks, s); break;
+        default: throw Error{DITCH_UNSUPPORTED, "matvecTMulti: tile format"};
+        }
+        DITCH_TRY_HIP(hipGetLastError());
     }
-    DITCH_TRY_HIP(hipGetLastError());
 }
 
 void launch_matvecT(float *out, const TileView &w, const float *y, int64_t q, hipStream_t s) {

@@ -93,8 +93,8 @@ __device__ __forceinline__ uint32_t next_term(float &a, float &b) {
 
 // GLU: mat[0] and mat[1] are gate and up; a workgroup takes OT row groups of
 // both, and its epilogue writes act(gate) * up of the summed tiles.
-// SEG: a segment (a routed expert) a blockIdx.y, up to NX of its rows gathered
-// by row_index (or consecutive), from f32 rows.
+// SEG: a segment (a routed expert) a blockIdx.y, NX of its rows a blockIdx.z,
+// gathered by row_index (or consecutive), from f32 rows.
 template <int TF, int MT, int OT, int W, int XT, int NX, int MATS, bool GLU, bool SEG = false>
 __global__ __launch_bounds__(64 * W) void few_kernel(FewParams<MATS> p) {
     static_assert(!SEG || (NX > 1 && MT == 1), "segments read f32 rows");
@@ -129,7 +129,9 @@ __global__ __launch_bounds__(64 * W) void few_kernel(FewParams<MATS> p) {
     const FewMat &mat = p.mat[mi];
     const GroupSeg *seg = SEG ? p.segs + blockIdx.y : nullptr;
     const TileView &w = SEG ? seg->w : mat.w;
-    const int64_t n = SEG ? seg->cnt : p.n, off = SEG ? seg->off : 0;
+    const int64_t first = SEG ? (int64_t)blockIdx.z * NX : 0;  // of the segment's rows
+    const int64_t n = SEG ? (seg->cnt - first < NX ? seg->cnt - first : NX) : p.n, off = SEG ? seg->off + first : 0;
+    if (SEG && n <= 0) return;
     const int64_t groups = (w.rows + 15) / 16, g0 = (int64_t)rb * OT, units = w.units_k, K = w.cols;
     const int steps = (int)((units + UPS - 1) / UPS), per = (steps + W - 1) / W;
     const int s0 = wave * per < steps ? wave * per : steps, s1 = s0 + per < steps ? s0 + per : steps;
@@ -498,14 +500,15 @@ void launch_tf(const FewCall &c) {
 
 // 16 rows and four K slices a workgroup: the segments fill the CUs
 template <int TF, int NX, bool GLU>
-void launch_segs_nx(const FewParams<1> &q, int64_t groups, unsigned nseg, hipStream_t s) {
-    hipLaunchKernelGGL((few_kernel<TF, 1, 1, 4, 2, NX, 1, GLU, true>), dim3((unsigned)groups, nseg), dim3(256), 0, s, q);
+void launch_segs_nx(const FewParams<1> &q, int64_t groups, unsigned nseg, int64_t max_cnt, hipStream_t s) {
+    hipLaunchKernelGGL((few_kernel<TF, 1, 1, 4, 2, NX, 1, GLU, true>), dim3((unsigned)groups, nseg, (unsigned)((max_cnt + NX - 1) / NX)),
+                       dim3(256), 0, s, q);
 }
 template <int TF, bool GLU>
 void launch_segs(const FewParams<1> &q, int64_t groups, unsigned nseg, int64_t max_cnt, hipStream_t s) {
-    if (max_cnt <= 2) launch_segs_nx<TF, 2, GLU>(q, groups, nseg, s);
-    else if (max_cnt <= 4) launch_segs_nx<TF, 4, GLU>(q, groups, nseg, s);
-    else launch_segs_nx<TF, 8, GLU>(q, groups, nseg, s);
+    if (max_cnt <= 2) launch_segs_nx<TF, 2, GLU>(q, groups, nseg, max_cnt, s);
+    else if (max_cnt <= 4) launch_segs_nx<TF, 4, GLU>(q, groups, nseg, max_cnt, s);
+    else launch_segs_nx<TF, 8, GLU>(q, groups, nseg, max_cnt, s);
 }
 template <bool GLU>
 void launch_segs_tf(int tf, const FewParams<1> &q, int64_t rows, unsigned nseg, int64_t max_cnt, hipStream_t s) {
@@ -606,12 +609,22 @@ void launch_few_glu(const TileView &gate, const TileView &up, uint32_t act, floa
     DITCH_TRY_HIP(hipGetLastError());
 }
 
+// Experts of up to 8 rows, or of up to 32 where most have at most 8 (a chunk of
+// 8 rows reads the weights again, from L2): us for gate/up and down of 128
+// experts of 2048 x 768, here against the GEMV (20 tokens) and the tiled
+// products: INT4 20 tokens 44 + 29 / 190 + 73, FP8 36 tokens 53 + 41 / 61 + 50,
+// INT4 64 tokens (86 experts used, 1.3 chunks each) 87 + 61 / 119 + 55.
 bool few_grouped_takes(const GroupSeg *segs, unsigned nseg, int64_t max_cnt) {
-    if (nseg < 1 || nseg > 65535 || max_cnt > 8) return false;
+    if (nseg < 1 || nseg > 65535 || max_cnt > 32) return false;
     const TileView &f = segs[0].w;
+    if (max_cnt > 8) {
+        int64_t chunks = 0;
+        for (unsigned i = 0; i < nseg; i++) chunks += (segs[i].cnt + 7) / 8;
+        if (2 * chunks > 3 * (int64_t)nseg) return false;
+    }
     for (unsigned i = 0; i < nseg; i++) {
         const TileView &w = segs[i].w;
-        if (segs[i].cnt < 1 || segs[i].cnt > max_cnt || !few_gemm_takes(w, segs[i].cnt, false) || w.cols % 4 != 0 ||
+        if (segs[i].cnt < 1 || segs[i].cnt > max_cnt || !few_gemm_takes(w, 1, false) || w.cols % 4 != 0 ||
             w.tf != f.tf || w.rows != f.rows || w.cols != f.cols)
             return false;
     }

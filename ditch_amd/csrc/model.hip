@@ -1303,18 +1303,18 @@ static void moe_forward(ditch_hip_model *m, Layer &L, float *x, const float *h, 
         DITCH_TRY_HIP(hipMemcpyAsync(dsegs + nseg, su.data(), nseg * sizeof(GroupSeg), hipMemcpyHostToDevice, s));
         DITCH_TRY_HIP(hipMemcpyAsync(dsegs + 2 * nseg, sd.data(), nseg * sizeof(GroupSeg), hipMemcpyHostToDevice, s));
         const TileView &vg = sg[0].w, &vd = sd[0].w;
-        // gate, up and SwiGLU in one tiled product whose epilogue writes the
-        // down product's fragments (f32 rows too when a down delta needs them)
-        const bool fused = tile_grouped_takes(sg.data(), nseg, max_cnt) && tile_grouped_takes(sd.data(), nseg, max_cnt) &&
-                           tile_glu_takes(vg, su[0].w, 128);
-        const void *dfr = nullptr;
-        // up to 8 rows an expert (decode steps): the few-token kernel, as above
-        // with f32 rows (2 layers of 128 experts of 2048 x 768 INT4, 4 rows:
+        // few rows an expert (decode steps, short prompts): the few-token kernel,
+        // the gate/up result as f32 rows (2 layers of 128 experts of 2048 x 768 INT4, 4 rows:
         // 63 + 63 + 5 us for gate, up and SwiGLU and 73 for down with the GEMV, 23
         // and 12 here)
-        const bool few = !fused && few_grouped_takes(sg.data(), nseg, max_cnt) && few_grouped_takes(su.data(), nseg, max_cnt) &&
+        const bool few = few_grouped_takes(sg.data(), nseg, max_cnt) && few_grouped_takes(su.data(), nseg, max_cnt) &&
                          few_grouped_takes(sd.data(), nseg, max_cnt) && sg[0].w.tf == su[0].w.tf &&
                          sg[0].w.rows == su[0].w.rows;
+        // gate, up and SwiGLU in one tiled product whose epilogue writes the
+        // down product's fragments (f32 rows too when a down delta needs them)
+        const bool fused = !few && tile_grouped_takes(sg.data(), nseg, max_cnt) && tile_grouped_takes(sd.data(), nseg, max_cnt) &&
+                           tile_glu_takes(vg, su[0].w, 128);
+        const void *dfr = nullptr;
         if (few) {
             launch_few_glu_grouped(dsegs, dsegs + nseg, vg, nseg, max_cnt, 0, gate, h, pair_token, s);
         } else if (fused) {

@@ -83,17 +83,17 @@ def test_log_softmax_and_kl_row_lengths(dev, ref, V):
         assert np.isnan(kl[1]) and np.isnan(ref.kl_rows(want, x)[1])
 
 
-# one to eight rows an expert (instances of 2, 4 and 8 rows), nine (the GEMV),
-# with and without deltas on the experts' down projections
-@pytest.mark.parametrize("fmt", ["bf16", "fp8", "mxfp4", "int4", "q8_0"])
-def test_few_rows_an_expert_match_oracle(dev, ref, fmt):
-    spec = mg.moe(fmt, layers=1, experts=4, top_k=4, seed=13)
+# one to eight rows an expert (instances of 2, 4 and 8 rows), nine (two chunks
+# each: the GEMV), chunks of unequal experts, with and without deltas on the experts' down projections
+@pytest.mark.parametrize("fmt,experts", [("bf16", 4), ("fp8", 4), ("mxfp4", 4), ("int4", 4), ("q8_0", 4), ("int4", 12)])
+def test_few_rows_an_expert_match_oracle(dev, ref, fmt, experts):
+    spec = mg.moe(fmt, layers=1, experts=experts, top_k=4, seed=13)
     c = spec.config
     gm, cm = Model(dev, spec), RefModel(spec)
     rng = np.random.default_rng(6)
     try:
         for i in range(2):
-            for j, lens in enumerate([[1], [2], [3], [5], [3, 5], [9]]):  # top_k = experts: every row at each
+            for j, lens in enumerate([[1], [2], [3], [5], [3, 5], [9], [13, 6]]):  # (4 experts: every row at each)
                 _check(gm, cm, lens, c["vocab"], 10 * i + j)
             for e in (0, 3):
                 a = (rng.standard_normal((e + 1, c["moe_inter"])) * 0.05).astype(np.float32)
