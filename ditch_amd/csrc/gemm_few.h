@@ -34,11 +34,13 @@ bool few_glu_takes(const TileView &gate, const TileView &up, int64_t n);
 void launch_few_glu(const TileView &gate, const TileView &up, uint32_t act, float *y, void *ys, int64_t ldk_y,
                     const float *x, int64_t ldx, const void *xs, int64_t ldk, int64_t n, hipStream_t s);
 
-// Routed experts of up to 8 rows each (16-byte aligned f32 rows of whole
-// float4s), every expert one format and shape: the gate/up product with its
-// activation into y [pair][rows], the rows gathered by row_index, and the down
-// product from consecutive rows, deltas added (delta_xa [pair][stride]).
+// Routed experts of few rows each (16-byte aligned f32 rows of whole float4s),
+// every expert one format and shape: the gate/up product with its activation
+// into y [pair][rows], the rows gathered by row_index, and the down product
+// from consecutive rows, deltas added (delta_xa [pair][stride]). An expert's
+// gate and up share their scale layout (few_glu_takes); experts may differ.
 bool few_grouped_takes(const GroupSeg *segs, unsigned nseg, int64_t max_cnt);
+bool few_glu_grouped_takes(const GroupSeg *gate, const GroupSeg *up, unsigned nseg, int64_t max_cnt);
 void launch_few_glu_grouped(const GroupSeg *d_gate, const GroupSeg *d_up, const TileView &shape, unsigned nseg,
                             int64_t max_cnt, uint32_t act, float *y, const float *x, const int32_t *row_index,
                             hipStream_t s);

@@ -583,7 +583,8 @@ void launch_few_gemm(const FewMat *mats, int nmat, const float *x, int64_t ldx, 
 bool few_glu_takes(const TileView &gate, const TileView &up, int64_t n) {
     return gate.tf == up.tf && gate.rows == up.rows && gate.cols == up.cols && gate.units_k == up.units_k &&
            few_gemm_takes(gate, n, false) && few_gemm_takes(up, n, false) &&
-           gate.scale_type == up.scale_type && gate.group == up.group && gate.block_cols == up.block_cols;
+           gate.scale_type == up.scale_type && gate.group == up.group && gate.block_cols == up.block_cols &&
+           gate.side_cols == up.side_cols;
 }
 
 void launch_few_glu(const TileView &gate, const TileView &up, uint32_t act, float *y, void *ys, int64_t ldk_y,
@@ -628,6 +629,14 @@ bool few_grouped_takes(const GroupSeg *segs, unsigned nseg, int64_t max_cnt) {
             w.tf != f.tf || w.rows != f.rows || w.cols != f.cols)
             return false;
     }
+    return true;
+}
+
+// (an expert's up is decoded by its gate's scale layout)
+bool few_glu_grouped_takes(const GroupSeg *gate, const GroupSeg *up, unsigned nseg, int64_t max_cnt) {
+    if (!few_grouped_takes(gate, nseg, max_cnt)) return false;
+    for (unsigned i = 0; i < nseg; i++)
+        if (!few_glu_takes(gate[i].w, up[i].w, 1)) return false;
     return true;
 }
 

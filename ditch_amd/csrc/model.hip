@@ -1307,9 +1307,8 @@ static void moe_forward(ditch_hip_model *m, Layer &L, float *x, const float *h, 
         // the gate/up result as f32 rows (2 layers of 128 experts of 2048 x 768 INT4, 4 rows:
         // 63 + 63 + 5 us for gate, up and SwiGLU and 73 for down with the GEMV, 23
         // and 12 here)
-        const bool few = few_grouped_takes(sg.data(), nseg, max_cnt) && few_grouped_takes(su.data(), nseg, max_cnt) &&
-                         few_grouped_takes(sd.data(), nseg, max_cnt) && sg[0].w.tf == su[0].w.tf &&
-                         sg[0].w.rows == su[0].w.rows;
+        const bool few = few_glu_grouped_takes(sg.data(), su.data(), nseg, max_cnt) &&
+                         few_grouped_takes(sd.data(), nseg, max_cnt);
         // gate, up and SwiGLU in one tiled product whose epilogue writes the
         // down product's fragments (f32 rows too when a down delta needs them)
         const bool fused = !few && tile_grouped_takes(sg.data(), nseg, max_cnt) && tile_grouped_takes(sd.data(), nseg, max_cnt) &&

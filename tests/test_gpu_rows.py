@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 import model_gen as mg
+import weights_gen as wg
 from ditch_amd import abi
 from ditch_amd.hip import Model
 from oracle.ref import RefModel
@@ -100,6 +101,40 @@ def test_few_rows_an_expert_match_oracle(dev, ref, fmt, experts):
                 b = (rng.standard_normal((c["hidden"], e + 1)) * 0.05).astype(np.float32)
                 for m in (gm, cm):
                     m.set_delta(0, abi.SLOT["EXPERT_DOWN"], e, a, b)
+    finally:
+        gm.free()
+        cm.free()
+
+
+# an expert's gate and up need not share their scale layout: other group widths, scale types and block widths,
+# in every expert or in one that is not the first
+LAYOUTS = {
+    "int4_groups": ("int4", dict(group=64), dict(group=128)),
+    "int4_groups_up_finer": ("int4", dict(group=128), dict(group=64)),
+    "int4_scale_types": ("int4", dict(scale_kind="f16"), dict(scale_kind="bf16")),
+    "fp8_blocks": ("fp8", dict(block=(128, 64)), dict(block=(128, 128))),
+}
+
+
+def _mixed_experts(layout, which, seed):
+    fmt, gate, up = LAYOUTS[layout]
+    make = wg.int_random if fmt == "int4" else wg.fp8_random
+    spec = mg.moe(fmt, layers=1, experts=4, top_k=4, seed=seed)
+    c, rng = spec.config, np.random.default_rng(seed)
+    for e in range(4):
+        spec.set("EXPERT_GATE", make(c["moe_inter"], c["hidden"], rng, **gate), 0, e)
+        spec.set("EXPERT_UP", make(c["moe_inter"], c["hidden"], rng, **(up if which in ("all", e) else gate)), 0, e)
+    return spec
+
+
+@pytest.mark.parametrize("which", ["all", 2])
+@pytest.mark.parametrize("layout", list(LAYOUTS))
+def test_experts_of_unequal_scale_layouts_match_oracle(dev, ref, layout, which):
+    spec = _mixed_experts(layout, which, 21)
+    gm, cm = Model(dev, spec), RefModel(spec)
+    try:
+        for j, lens in enumerate([[1], [5], [9]]):  # (every row at each expert)
+            _check(gm, cm, lens, spec.config["vocab"], 30 + j)
     finally:
         gm.free()
         cm.free()
