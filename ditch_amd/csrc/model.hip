@@ -1311,8 +1311,9 @@ static void moe_forward(ditch_hip_model *m, Layer &L, float *x, const float *h, 
                          few_grouped_takes(sd.data(), nseg, max_cnt);
         // gate, up and SwiGLU in one tiled product whose epilogue writes the
         // down product's fragments (f32 rows too when a down delta needs them)
-        const bool fused = !few && tile_grouped_takes(sg.data(), nseg, max_cnt) && tile_grouped_takes(sd.data(), nseg, max_cnt) &&
-                           tile_glu_takes(vg, su[0].w, 128);
+        // (every expert's up is decoded by its gate's scale layout)
+        bool fused = !few && tile_grouped_takes(sg.data(), nseg, max_cnt) && tile_grouped_takes(sd.data(), nseg, max_cnt);
+        for (unsigned i = 0; fused && i < nseg; i++) fused = tile_glu_takes(sg[i].w, su[i].w, 128);
         const void *dfr = nullptr;
         if (few) {
             launch_few_glu_grouped(dsegs, dsegs + nseg, vg, nseg, max_cnt, 0, gate, h, pair_token, s);

@@ -133,7 +133,8 @@ def test_experts_of_unequal_scale_layouts_match_oracle(dev, ref, layout, which):
     spec = _mixed_experts(layout, which, 21)
     gm, cm = Model(dev, spec), RefModel(spec)
     try:
-        for j, lens in enumerate([[1], [5], [9]]):  # (every row at each expert)
+        # (every row at each expert; 40 rows take the tiled products)
+        for j, lens in enumerate([[1], [5], [9], [40]]):
             _check(gm, cm, lens, spec.config["vocab"], 30 + j)
     finally:
         gm.free()
