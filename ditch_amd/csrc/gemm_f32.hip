@@ -171,7 +171,7 @@ __global__ __launch_bounds__(256) void f32_gemm_kernel(GemmParams p, int tiles_m
 // the fp32 matrix cores; 4864 x 896 on 1024 tokens 104 -> 79 us.
 typedef __attribute__((address_space(3))) void lds_void;
 
-template <int TF, int WG, int KS>
+template <int TF, int WG, int KS, int SPAN>
 __global__ __launch_bounds__(64 * WG * WG * KS) void f32_tile_kernel(GemmParams p, int tiles_m, int tiles) {
     constexpr int NWS = WG * WG, NW = NWS * KS;       // waves of a slice, of the workgroup
     constexpr int AP = 4 * WG;                        // 1 KiB activation pieces of a slice's unit
@@ -188,7 +188,8 @@ __global__ __launch_bounds__(64 * WG * WG * KS) void f32_tile_kernel(GemmParams 
     const int tm = tile % tiles_m, tn = tile / tiles_m;
     const TileView &w = p.w;
     const int U = (int)w.units_k, groups = (int)((w.rows + 15) / 16);
-    const int nu = (U + KS - 1) / KS, u0 = ks * nu, u1 = u0 + nu < U ? u0 + nu : U;  // u0 >= u1: an empty slice
+    // (slices of U / KS units or one more, in nu steps each)
+    const int nu = (U + KS - 1) / KS, u0 = U * ks / KS, u1 = U * (ks + 1) / KS;
 
     // sources of this wave's copies at unit 0 (tokens and rows past the end
     // repeat the last one: their outputs are not stored)
@@ -290,10 +291,9 @@ __global__ __launch_bounds__(64 * WG * WG * KS) void f32_tile_kernel(GemmParams 
         copy(u0 + s + 3, cbuf);    // into the buffer of stage s - 1
         if (own || u0 + s < u1) products(cur);
     };
-    const int common = U - (KS - 1) * nu;  // units that every slice has (the last one's)
+    const int common = U / KS;  // units that every slice has
     int s = 0;
-    // sums of 512 columns are added to the total: as one chain over K the
-    // error against 64 bits was 2.1e-6 at 13312 columns, so 0.42e-6
+    // sums of SPAN units are added to the total (launch_staged)
     floatx4 total[2][2];
 #pragma unroll
     for (int m = 0; m < 2; m++)
@@ -313,17 +313,23 @@ __global__ __launch_bounds__(64 * WG * WG * KS) void f32_tile_kernel(GemmParams 
     auto four = [&](int s) __attribute__((always_inline)) {  // no branch inside: every wait is a count
         step(s, even, odd, buf1, buf3, true);
         step(s + 1, odd, even, buf2, buf0, true);
+        if constexpr (SPAN == 2) fold();
         step(s + 2, even, odd, buf3, buf1, true);
         step(s + 3, odd, even, buf0, buf2, true);
     };
-    for (; s + 16 <= common; s += 16) {
-        for (int b = 0; b < 16; b += 4) four(s + b);
-        fold();
+    if constexpr (SPAN > 4)
+        for (; s + SPAN <= common; s += SPAN) {
+            for (int b = 0; b < SPAN; b += 4) four(s + b);
+            fold();
+        }
+    for (; s + 4 <= common; s += 4) {
+        four(s);
+        if constexpr (SPAN <= 4) fold();
     }
-    for (; s + 4 <= common; s += 4) four(s);
     for (; s < nu; s += 4) {
         step(s, even, odd, buf1, buf3, false);
         if (s + 1 < nu) step(s + 1, odd, even, buf2, buf0, false);
+        if constexpr (SPAN == 2) fold();
         if (s + 2 < nu) step(s + 2, even, odd, buf3, buf1, false);
         if (s + 3 < nu) step(s + 3, odd, even, buf0, buf2, false);
     }
@@ -367,10 +373,23 @@ __global__ __launch_bounds__(64 * WG * WG * KS) void f32_tile_kernel(GemmParams 
     }
 }
 
+// A sum is at most a quarter of K, and 512 columns: no K's error against 64
+// bits is then above that of the register-staged kernel's four slices of one
+// chain each (13312 columns: 1.03e-6 there, 0.40e-6 here, 2.1e-6 in one chain;
+// 896 columns on 1024 tokens: 2.7e-7 there, 2.1e-7 here, 3.8e-7 in two chains).
+// Four slices need no shorter sums for it; with fewer, 128 columns from 512 on
+// and 64 below.
 template <int TF, int WG, int KS>
 void launch_tiles(const GemmParams &p, int tiles_m, int64_t tiles, hipStream_t s) {
-    hipLaunchKernelGGL((f32_tile_kernel<TF, WG, KS>), dim3((unsigned)tiles), dim3(64 * WG * WG * KS), 0, s, p,
-                       tiles_m, (int)tiles);
+    const dim3 grid((unsigned)tiles), block(64 * WG * WG * KS);
+    if constexpr (KS < 4) {
+        if (p.w.units_k < 64) {
+            if (p.w.units_k < 16) hipLaunchKernelGGL((f32_tile_kernel<TF, WG, KS, 2>), grid, block, 0, s, p, tiles_m, (int)tiles);
+            else hipLaunchKernelGGL((f32_tile_kernel<TF, WG, KS, 4>), grid, block, 0, s, p, tiles_m, (int)tiles);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((f32_tile_kernel<TF, WG, KS, 16>), grid, block, 0, s, p, tiles_m, (int)tiles);
 }
 
 // 64 x 64 tiles in one slice (0.85 of the fp32 matrix rate over full rounds of
