@@ -180,6 +180,17 @@ int32_t ditch_hip_sync(ditch_hip *h) {
     return guarded(h, [&] { DITCH_TRY_HIP(hipStreamSynchronize(h->stream)); });
 }
 
+// The scratch of a product of n tokens on s. From 17 to 31 tokens a product
+// shares none with calls on other streams and holds none under capture (a
+// replay would use it after it has grown): only the context's own stream,
+// outside a capture, has fragments.
+static DevBuf *product_scratch(ditch_hip *h, uint64_t n, hipStream_t s) {
+    if (n < 17 || n > 31) return &h->split;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (s == h->stream) DITCH_TRY_HIP(hipStreamIsCapturing(s, &cap));
+    return s == h->stream && cap == hipStreamCaptureStatusNone ? &h->few : nullptr;
+}
+
 // ---------------------------------------------------------------------------
 // VTable operations, host memory
 
@@ -194,7 +205,7 @@ int32_t ditch_hip_matmulT(ditch_hip *h, float *out, const float *x, uint64_t n, 
         h2d(dx.p, x, n * w->cols * 4, s);
         MatmulEpilogue ep;
         ep.exact = 1;
-        launch_matmul(t->v, dout.as<float>(), dx.as<float>(), (int64_t)n, ep, s, nullptr, &h->split);
+        launch_matmul(t->v, dout.as<float>(), dx.as<float>(), (int64_t)n, ep, s, nullptr, product_scratch(h, n, s));
         d2h(out, dout.p, n * w->rows * 4, s);
         DITCH_TRY_HIP(hipStreamSynchronize(s));
     });
@@ -399,7 +410,8 @@ int32_t ditch_hip_matmulT_device(ditch_hip *h, float *d_out, uint64_t out_bytes,
         MatmulEpilogue ep;
         ep.bias = d_bias;
         ep.accumulate = accumulate;
-        launch_matmul(w->v, d_out, d_x, (int64_t)n, ep, stream ? (hipStream_t)stream : h->stream, nullptr, &h->split);
+        hipStream_t s = stream ? (hipStream_t)stream : h->stream;
+        launch_matmul(w->v, d_out, d_x, (int64_t)n, ep, s, nullptr, product_scratch(h, n, s));
     });
 }
 

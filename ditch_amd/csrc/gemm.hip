@@ -150,7 +150,7 @@ void launch_matmul(const TileView &w, float *out, const float *x, int64_t n, con
         // (three terms too where the product they stand in for is the scaled
         // MFMA's, whose fp6 terms hold 18 bits)
         const int xt = ep.exact || mx_gemm_takes(w, n) ? 3 : 2;
-        const bool rows = !row_index && few_reads_rows(w, n, x, w.cols);
+        const bool rows = (n <= 8 || !ws) && !row_index && few_reads_rows(w, n, x, w.cols);
         const size_t xb = rows ? 0 : split_bytes_ldk(n, few_ldk(w), xt);
         // (fragments past a borrowed scratch: the products below need less)
         if (rows || (ws && !(ws->borrowed && xb > ws->bytes))) {

@@ -18,7 +18,7 @@ struct FewMat {
 bool few_gemm_takes(const TileView &w, int64_t n, bool exact);
 // k tiles of its fragments: whole 128-column steps (split_ldk)
 inline int64_t few_ldk(const TileView &w) { return split_ldk(w.cols); }
-// Whether it reads n f32 rows at x itself (no fragments).
+// Whether it can read n f32 rows at x itself (no fragments).
 bool few_reads_rows(const TileView &w, int64_t n, const float *x, int64_t ldx);
 // Products of 1 to 3 matrices of one format and K over the same activations,
 // in one launch: from f32 rows x (few_reads_rows) or, with x NULL, from

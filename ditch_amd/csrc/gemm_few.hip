@@ -21,7 +21,9 @@
 //     FP8 and 29 us for MXFP4 at 4096 x 4096 on one token;
 //   - up to 8 tokens (NX) each wave splits its slice of the f32 rows into bf16
 //     terms itself, in its own LDS slot; more tokens come as fragments
-//     (split_kernel's layout), which producers write directly;
+//     (split_kernel's layout), which producers write directly, or, where the
+//     caller has no scratch for them, in chunks of 8 (24 tokens: 0.6 to 0.9 of
+//     the fragments' time below 4 M weights, 1.2 to 1.9 of it at 14336 x 4096);
 //   - one launch may hold up to three matrices over the same activations.
 //
 // Measured, us a call with its split (before: the GEMV up to 16 tokens, the
@@ -109,7 +111,7 @@ __global__ __launch_bounds__(64 * W) void few_kernel(FewParams<MATS> p) {
     // turn, so the token blocks of a row block are 8 apart (one XCD reads the
     // row block's weights once from memory and then from its L2)
     int rb = blockIdx.x, tb = 0;
-    if (NX == 0 && p.tblocks > 1) {
+    if (!SEG && p.tblocks > 1) {
         const int nb = p.end[MATS - 1], full = nb / 8 * 8 * p.tblocks, L = blockIdx.x;
         if (L < full) {
             tb = L / 8 % p.tblocks;
@@ -129,9 +131,11 @@ __global__ __launch_bounds__(64 * W) void few_kernel(FewParams<MATS> p) {
     const FewMat &mat = p.mat[mi];
     const GroupSeg *seg = SEG ? p.segs + blockIdx.y : nullptr;
     const TileView &w = SEG ? seg->w : mat.w;
-    const int64_t first = SEG ? (int64_t)blockIdx.z * NX : 0;  // of the segment's rows
-    const int64_t n = SEG ? (seg->cnt - first < NX ? seg->cnt - first : NX) : p.n, off = SEG ? seg->off + first : 0;
+    // f32 rows: NX of the segment's or of the call's tokens
+    const int64_t all = SEG ? seg->cnt : p.n, first = SEG ? (int64_t)blockIdx.z * NX : NX ? (int64_t)tb * NX : 0;
+    const int64_t n = NX && all - first > NX ? NX : all - first, off = (SEG ? seg->off : 0) + first;
     if (SEG && n <= 0) return;
+    if constexpr (NX > 0) tb = 0;  // (outputs count from row off)
     const int64_t groups = (w.rows + 15) / 16, g0 = (int64_t)rb * OT, units = w.units_k, K = w.cols;
     const int steps = (int)((units + UPS - 1) / UPS), per = (steps + W - 1) / W;
     const int s0 = wave * per < steps ? wave * per : steps, s1 = s0 + per < steps ? s0 + per : steps;
@@ -184,7 +188,7 @@ __global__ __launch_bounds__(64 * W) void few_kernel(FewParams<MATS> p) {
             for (int m = 0; m < NX / 2; m++) {
                 const int64_t tok = 2 * m + (lane >> 5);
                 if constexpr (SEG) v.xp[m] = gload<float4>(xr[m] + kc);
-                else v.xp[m] = gload<float4>(p.x + (tok < n ? tok : n - 1) * p.ldx + kc);
+                else v.xp[m] = gload<float4>(p.x + (off + (tok < n ? tok : n - 1)) * p.ldx + kc);
             }
         }
 #pragma unroll
@@ -370,11 +374,11 @@ __global__ __launch_bounds__(64 * W) void few_kernel(FewParams<MATS> p) {
         e.delta_rank = seg->delta_rank;
         e.delta_stride = p.delta_stride;
     } else {
-        e.out = mat.out;
+        e.out = mat.out + off * w.rows;
         e.bias = mat.bias;
         e.accumulate = mat.accumulate;
         e.delta_b = mat.delta_b;
-        e.delta_xa = mat.delta_xa;
+        e.delta_xa = mat.delta_xa + off * mat.delta_rank;
         e.delta_rank = e.delta_stride = mat.delta_rank;
     }
     for (int q = wave; q < MT * NT; q += W) {
@@ -413,7 +417,7 @@ void launch_mats(const FewCall &c) {
     p.ys = (uint8_t *)c.ys;
     p.ldk_y = c.ldk_y;
     p.act = c.act;
-    p.tblocks = NX ? 1 : (int)((c.n + 16 * MT - 1) / (16 * MT));
+    p.tblocks = NX ? (int)((c.n + NX - 1) / NX) : (int)((c.n + 16 * MT - 1) / (16 * MT));
     p.x = c.x;
     p.xs = (const uint8_t *)c.xs;
     p.n = c.n;
@@ -478,7 +482,7 @@ void launch_tf(const FewCall &c) {
         if (c.n == 1) launch_rows<TF, XT, 1>(c, groups, steps);
         else if (c.n == 2) launch_rows<TF, XT, 2>(c, groups, steps);
         else if (c.n <= 4) launch_rows<TF, XT, 4>(c, groups, steps);
-        else launch_rows<TF, XT, 8>(c, groups, steps);
+        else launch_rows<TF, XT, 8>(c, groups * ((c.n + 7) / 8), steps);
         return;
     }
     // Few row groups x token blocks: eight K slices over 16 rows (1024 x 4096
@@ -553,7 +557,7 @@ bool few_gemm_takes(const TileView &w, int64_t n, bool exact) {
 }
 
 bool few_reads_rows(const TileView &w, int64_t n, const float *x, int64_t ldx) {
-    return n <= 8 && w.cols % 4 == 0 && ldx % 4 == 0 && ((uintptr_t)x & 15) == 0;
+    return n <= 32 && w.cols % 4 == 0 && ldx % 4 == 0 && ((uintptr_t)x & 15) == 0;
 }
 
 void launch_few_gemm(const FewMat *mats, int nmat, const float *x, int64_t ldx, const void *xs, int64_t ldk, int64_t n,
@@ -591,7 +595,7 @@ void launch_few_glu(const TileView &gate, const TileView &up, uint32_t act, floa
                     const float *x, int64_t ldx, const void *xs, int64_t ldk, int64_t n, hipStream_t s) {
     DITCH_CHECK(few_glu_takes(gate, up, n) && (y || ys) && (!ys || (gate.rows % 128 == 0 && ldk_y * 32 >= gate.rows)),
                 DITCH_INVALID_ARGUMENT, "few-token gate/up: shapes or outputs");
-    DITCH_CHECK(x ? few_reads_rows(gate, n, x, ldx) : xs && ldk >= few_ldk(gate), DITCH_INVALID_ARGUMENT,
+    DITCH_CHECK(x ? n <= 8 && few_reads_rows(gate, n, x, ldx) : xs && ldk >= few_ldk(gate), DITCH_INVALID_ARGUMENT,
                 "few-token gate/up: activations not in a form it reads");
     const FewMat mats[2] = {FewMat{gate, nullptr, nullptr, nullptr, nullptr, 0, 0}, FewMat{up, nullptr, nullptr, nullptr, nullptr, 0, 0}};
     FewCall c{mats, 2, x, ldx, xs, ldk, n, s};

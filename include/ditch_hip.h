@@ -225,7 +225,12 @@ int32_t ditch_hip_tensor_dequant(ditch_hip *h, void *d_out, uint64_t out_bytes,
  * `accumulate` != 0 adds into d_out (the residual add of model.zig:4944).
  * `out_bytes` / `x_bytes` are the buffers' lengths (the `out` and `x`
  * slices of compute.zig:100); shorter than n * rows * 4 / n * cols * 4 is
- * refused before anything is launched.                                     */
+ * refused before anything is launched. Products of 9 to 16 and of 32 and
+ * more tokens share the context's scratch, which grows with the largest of
+ * them: those on different streams need an order between them (events, or
+ * ditch_hip_matmulT_device_noalloc). Products of up to 8 and of 17 to 31
+ * tokens share nothing with calls on other streams, and neither allocate nor
+ * hold scratch on a stream other than the context's or under capture.      */
 int32_t ditch_hip_matmulT_device(ditch_hip *h, float *d_out, uint64_t out_bytes,
                                  const float *d_x, uint64_t x_bytes,
                                  uint64_t n, const ditch_hip_tensor *w,

@@ -4,6 +4,8 @@ from fragments, K of less than one 128-column step, of partial units and steps
 and of K slices of unequal length, rows that leave a row group and a row block
 part empty, the grids on both sides of each tile choice, and the last token
 count it takes."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -92,3 +94,109 @@ def test_mxfp4_from_128_tokens_keeps_the_scaled_product_s_precision(dev, ref, n,
         t.free()
     want = x.astype(np.float64) @ dequant_f32(ref, w).astype(np.float64).T
     assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want)
+
+
+def _stream(lib):
+    s = ctypes.c_void_p()
+    assert lib.hipStreamCreateWithFlags(ctypes.byref(s), 1) == 0  # non-blocking, default priority
+    return s
+
+
+@pytest.mark.parametrize("kind,n,rows,cols", [("bf16", 17, 50, 132), ("fp8", 24, 8208, 320), ("mxfp4", 25, 4096, 256),
+                                              ("int4", 31, 130, 2240), ("q8_0", 20, 33, 1056), ("bf16", 18, 40, 30)])
+def test_chunks_of_rows_on_another_stream(dev, ref, kind, n, rows, cols):
+    """17 to 31 tokens without scratch: chunks of 8 rows (the last one of any
+    size), or the register-staged product where rows are not whole float4s."""
+    rng = np.random.default_rng(n + rows + cols)
+    w = wg.make(kind, rows, cols, rng)
+    x = rng.standard_normal((n, cols)).astype(np.float32)
+    bias = rng.standard_normal(rows).astype(np.float32)
+    prior = rng.standard_normal((n, rows)).astype(np.float32)
+    lib = hipmem.hip()
+    s, t = _stream(lib), dev.upload(w)
+    try:
+        bx, bb, bo = (hipmem.Buffer.from_array(a) for a in (x, bias, prior))
+        t.matmul_device(bo.ptr, bx.ptr, n, d_bias=bb.ptr, accumulate=True, stream=s.value)
+        assert lib.hipStreamSynchronize(s) == 0
+        got = bo.download(np.float32, (n, rows))
+    finally:
+        t.free()
+        lib.hipStreamDestroy(s)
+    want = prior.astype(np.float64) + ref.matmulT(x, w).astype(np.float64) + bias
+    bound = split_bound("bf16", x, dequant_f32(ref, w))
+    assert (np.abs(got - want) <= TOL_MATMUL["atol"] + TOL_MATMUL["rtol"] * np.abs(want) + bound).all()
+
+
+def test_products_of_17_to_31_tokens_on_two_streams(dev, ref):
+    """No order between the streams and the context's own: every output is
+    that of the call alone."""
+    rng = np.random.default_rng(8)
+    lib = hipmem.hip()
+    streams = [_stream(lib).value, _stream(lib).value, None]
+    t = [dev.upload(wg.make("fp8", 2048, 1024, rng)), dev.upload(wg.make("int4", 1024, 4096, rng))]
+    try:
+        jobs = []
+        for i in range(24):
+            w, n = t[i % 2], (17, 24, 31)[i // 2 % 3]
+            bx = hipmem.Buffer.from_array(rng.standard_normal((n, w.cols)).astype(np.float32))
+            outs = [hipmem.Buffer(n * w.rows * 4) for _ in range(2)]
+            jobs.append((w, n, bx, outs, streams[i % 3]))
+        for alone in (False, True):
+            for w, n, bx, outs, s in jobs:
+                w.matmul_device(outs[alone].ptr, bx.ptr, n, stream=s)
+                if alone:
+                    hipmem.synchronize()
+            hipmem.synchronize()
+        for w, n, bx, outs, s in jobs:
+            a, b = (o.download(np.float32, (n, w.rows)) for o in outs)
+            np.testing.assert_array_equal(a, b)
+    finally:
+        for w in t:
+            w.free()
+        for s in streams[:2]:
+            lib.hipStreamDestroy(s)
+
+
+@pytest.mark.parametrize("own", [False, True])
+def test_product_of_24_tokens_captured_without_a_warm_up(dev, own):
+    """On another stream and on the context's own: nothing is allocated under
+    the capture, and a larger product afterwards leaves the graph's replays."""
+    lib = hipmem.hip()
+    P = ctypes.c_void_p
+    for name, args in {"hipStreamBeginCapture": [P, ctypes.c_int], "hipStreamEndCapture": [P, ctypes.POINTER(P)],
+                       "hipGraphInstantiate": [ctypes.POINTER(P), P, P, P, ctypes.c_size_t],
+                       "hipGraphLaunch": [P, P], "hipGraphExecDestroy": [P], "hipGraphDestroy": [P]}.items():
+        getattr(lib, name).argtypes = args
+        getattr(lib, name).restype = ctypes.c_int
+    rng = np.random.default_rng(9)
+    n, rows, cols = 24, 512, 2048
+    t, big = dev.upload(wg.make("fp8", rows, cols, rng)), dev.upload(wg.make("fp8", 64, 16384, rng))
+    made = None if own else _stream(lib)
+    stream = P(dev.stream) if own else made
+    graph, ge = P(), P()
+    try:
+        bx, bo, want = hipmem.Buffer(n * cols * 4), hipmem.Buffer(n * rows * 4), hipmem.Buffer(n * rows * 4)
+        bb, ob = hipmem.Buffer.from_array(np.ones((31, 16384), np.float32)), hipmem.Buffer(31 * 64 * 4)
+        assert lib.hipStreamBeginCapture(stream, 0) == 0  # hipStreamCaptureModeGlobal
+        t.matmul_device(bo.ptr, bx.ptr, n, stream=stream.value)
+        assert lib.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
+        assert lib.hipGraphInstantiate(ctypes.byref(ge), graph, None, None, 0) == 0
+        for _ in range(3):
+            bx.upload(rng.standard_normal((n, cols)).astype(np.float32))
+            big.matmul_device(ob.ptr, bb.ptr, 31)
+            t.matmul_device(want.ptr, bx.ptr, n)
+            hipmem.synchronize()
+            assert lib.hipGraphLaunch(ge, stream) == 0
+            hipmem.synchronize()
+            a, b = bo.download(np.float32, (n, rows)), want.download(np.float32, (n, rows))
+            # the same products, summed in another order: f32 rounding only
+            assert np.abs(a - b).max() <= 1e-5 * np.abs(b).max()
+    finally:
+        if ge.value:
+            lib.hipGraphExecDestroy(ge)
+        if graph.value:
+            lib.hipGraphDestroy(graph)
+        if made:
+            lib.hipStreamDestroy(made)
+        t.free()
+        big.free()
