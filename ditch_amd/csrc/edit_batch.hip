@@ -37,7 +37,8 @@ struct WtyArgs {
     int64_t q0, q;          // directions q0 .. q, QB of them a workgroup (blockIdx.y)
 };
 
-constexpr int WTY_STEP = 4;  // row groups whose loads are in flight together
+constexpr int WTY_WAVES = 4;  // (they set the order of the sums)
+constexpr int WTY_STEP = 4;   // row groups whose loads are in flight together
 
 
 // Side data of one (row, unit): the Q8 / MXFP4 scale word, or the FP8 /
@@ -122,11 +123,11 @@ template <int TF, bool FAST> constexpr int wty_side_words() {
     else return 1;
 }
 
-template <int TF, int QB, bool FAST, int WAVES>
-__global__ __launch_bounds__(WAVES * 64) void wty_kernel(WtyArgs a) {
+template <int TF, int QB, bool FAST>
+__global__ __launch_bounds__(WTY_WAVES * 64) void wty_kernel(WtyArgs a) {
     constexpr int TL = Fmt<TF>::tiles, UK = 32 * TL, NV = 8 * TL;
     constexpr int NS = wty_side_words<TF, FAST>();
-    __shared__ float red[WAVES][QB][UK];
+    __shared__ float red[WTY_WAVES][QB][UK];
     int64_t unit;
     const WtySeg *sp = &a.one;
     if (a.segs) {
@@ -150,7 +151,7 @@ __global__ __launch_bounds__(WAVES * 64) void wty_kernel(WtyArgs a) {
 
     SideStep st{1u, 0};
     if constexpr (FAST) st = side_step<TF>(w);
-    for (int64_t g0 = (int64_t)wave * WTY_STEP; g0 < groups; g0 += WAVES * WTY_STEP) {
+    for (int64_t g0 = (int64_t)wave * WTY_STEP; g0 < groups; g0 += WTY_WAVES * WTY_STEP) {
         Raw raw[WTY_STEP];
         WtySide<TF> sd[WTY_STEP];
         uint32_t sw[WTY_STEP][NS];
@@ -210,21 +211,21 @@ __global__ __launch_bounds__(WAVES * 64) void wty_kernel(WtyArgs a) {
             if (r16 == 0) red[wave][j][32 * (v / 8) + 8 * kq + (v % 8)] = s;
         }
     __syncthreads();
-    for (int i = threadIdx.x; i < QB * UK; i += WAVES * 64) {
+    for (int i = threadIdx.x; i < QB * UK; i += WTY_WAVES * 64) {
         const int j = i / UK, c = i % UK;
         const int64_t col = unit * UK + c;
         if (q0 + j >= a.q || col >= w.cols) continue;
         float s = red[0][j][c];
 #pragma unroll
-        for (int wv = 1; wv < WAVES; wv++) s = __fadd_rn(s, red[wv][j][c]);
+        for (int wv = 1; wv < WTY_WAVES; wv++) s = __fadd_rn(s, red[wv][j][c]);
         out[(q0 + j) * w.cols + col] = s;
     }
 }
 
-template <int TF, int QB, bool FAST, int WAVES>
+template <int TF, int QB, bool FAST>
 static void wty_launch_q(const WtyArgs &a, unsigned blocks, hipStream_t s) {
     const dim3 grid(blocks, (unsigned)((a.q - a.q0 + QB - 1) / QB));
-    hipLaunchKernelGGL((wty_kernel<TF, QB, FAST, WAVES>), grid, dim3(WAVES * 64), 0, s, a);
+    hipLaunchKernelGGL((wty_kernel<TF, QB, FAST>), grid, dim3(WTY_WAVES * 64), 0, s, a);
 }
 
 // All directions in one launch, QB of them a workgroup: more share a weight's
@@ -232,15 +233,16 @@ static void wty_launch_q(const WtyArgs &a, unsigned blocks, hipStream_t s) {
 // us for 10 directions with QB = 1, 2, 4: bf16 896 x 4864 (152 column units)
 // 10.4, 8.4, 9.6; 896 x 896 (28) 5.7, 6.5, 8.5; FP8 4096 x 14336 (448) 147,
 // 100, 80; MXFP4 4096 x 14336 (112) 81, 66, 68, 4096 x 4096 (32) 41, 34, 45.
-// One direction of few units: 16 waves a workgroup, FP8 4096 x 4096 32 -> 21
-// us, bf16 896 x 896 5.8 -> 3.9 (with more directions their registers spill;
-// with enough workgroups 4 waves are better, 62 against 73 us for 1000 units).
+// Four waves whatever the launch holds: their number sets the order of the
+// sums, and an edit's deltas have the same bits alone and in a batch. (One
+// direction with 16 waves: FP8 4096 x 4096 alone 32 -> 20 us, but six of it
+// with 4096 x 14336 124 -> 141, Q8_0 896 x 896 and 896 x 4864 of 12 layers
+// 22 -> 32.)
 template <int TF, bool FAST>
 static void wty_launch_blocks(const WtyArgs &a, unsigned blocks, hipStream_t s) {
-    if (a.q == 1 && blocks < 512) wty_launch_q<TF, 1, FAST, 16>(a, blocks, s);
-    else if (a.q == 1) wty_launch_q<TF, 1, FAST, 4>(a, blocks, s);
-    else if (a.q == 2 || (int64_t)blocks * ((a.q + 3) / 4) < 512) wty_launch_q<TF, 2, FAST, 4>(a, blocks, s);
-    else wty_launch_q<TF, 4, FAST, 4>(a, blocks, s);
+    if (a.q == 1) wty_launch_q<TF, 1, FAST>(a, blocks, s);
+    else if (a.q == 2 || (int64_t)blocks * ((a.q + 3) / 4) < 512) wty_launch_q<TF, 2, FAST>(a, blocks, s);
+    else wty_launch_q<TF, 4, FAST>(a, blocks, s);
 }
 
 template <int TF>

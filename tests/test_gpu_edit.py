@@ -209,3 +209,27 @@ def test_directions_of_one_launch_match_oracle(dev, ref, fmt, k):
     ca, cb = ref.edit_delta_ex(w, v, 1.0, MODES["none"])
     # f32 sums of 272 products in another order: 272 * 2^-24 of the largest
     assert np.abs(ga - ca).max() <= 2e-5 * np.abs(ca).max() and np.array_equal(gb, cb)
+
+
+@pytest.mark.parametrize("fmt", ["bf16", "fp8", "q8_0"])
+@pytest.mark.parametrize("k", [1, 5])
+def test_a_delta_has_the_same_bits_alone_and_in_a_batch(dev, fmt, k):
+    """Batches of more than 512 column units, each matrix of far fewer: the
+    forward after them is that after an edit per matrix, bit for bit."""
+    inter = {"bf16": 4096, "fp8": 8192, "q8_0": 8192}[fmt]
+    spec = mg.dense(fmt, hidden=128, inter=inter, layers=5, heads=2, kv_heads=2, head_dim=64, vocab=256, seed=k)
+    rng = np.random.default_rng(k)
+    targets = [(li, abi.SLOT["DOWN"], -1, orthonormal_rows(rng, k, 128), 0.7) for li in range(5)]
+    tokens, rows, last = mg.batch(2, [3, 9], 256, seed=2)
+    gm = Model(dev, spec)
+    try:
+        gm.edit_batch(targets, k)
+        want = gm.forward(tokens, rows, capture_rows=last, logit_rows=last)
+        gm.reset_deltas()
+        for t in targets:
+            gm.edit(*t)
+        got = gm.forward(tokens, rows, capture_rows=last, logit_rows=last)
+    finally:
+        gm.free()
+    for a, b in zip(got, want):
+        np.testing.assert_array_equal(a, b)
