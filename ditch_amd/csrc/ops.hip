@@ -524,8 +524,9 @@ __global__ void softmax_kernel(float *x, int64_t len) {
 //   pass 2  per chunk: s = sum s_c exp(m_c - m) over the row's chunks, lse,
 //           and the chunk's outputs (log-probs, or the KL terms -> part_k)
 //   pass 3  (KL only) per row: part_k added by a wave.
-// The chunking depends on the row's length alone, so a row has the same lse in
-// both functions and the KL of a row against its own log-probs is 0. Bound by
+// The chunking and the order of pass 1's sums depend on the row's length alone
+// (not on the buffers' alignment), so a row has the same lse in both functions
+// and the KL of a row against its own log-probs is 0. Bound by
 // memory, then by the f64 exponentials: 64 rows of 151936, log-softmax and KL
 // 182 -> 77 us (the maximum had a pass of its own, and each workgroup added the
 // row's parts one after the other).
@@ -557,6 +558,14 @@ __global__ __launch_bounds__(256) void rowpart_kernel(float *part_m, double *par
     const int count = (int)(len - i0 < ROW_CHUNK ? len - i0 : ROW_CHUNK);
     float v[8];
     row_load<VEC>(v, x + row * len + i0, count, -INFINITY);
+    if constexpr (!VEC) {  // to the elements that a thread has of aligned rows
+        __shared__ float4 turn[ROW_CHUNK / 4];
+#pragma unroll
+        for (int j = 0; j < 8; j++) ((float *)turn)[row_elem<false>(j)] = v[j];
+        __syncthreads();
+        const float4 a = turn[threadIdx.x], b = turn[256 + threadIdx.x];
+        v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+    }
     float m = -INFINITY;
 #pragma unroll
     for (int j = 0; j < 8; j++) m = fmaxf(m, v[j]);

@@ -1,11 +1,13 @@
 """Row kernels and the few-token forward at the edges of their ranges, against
 the oracle (needs an MI355X)."""
+import ctypes
+
 import numpy as np
 import pytest
 
 import model_gen as mg
 import weights_gen as wg
-from ditch_amd import abi
+from ditch_amd import abi, hipmem
 from ditch_amd.hip import Model
 from oracle.ref import RefModel
 
@@ -82,6 +84,22 @@ def test_log_softmax_and_kl_row_lengths(dev, ref, V):
     assert kl[0] == 0 and kl[2] == 0
     if V > 1:
         assert np.isnan(kl[1]) and np.isnan(ref.kl_rows(want, x)[1])
+
+
+# one buffer off 16-byte alignment (read element by element), rows of whole float4s or not
+@pytest.mark.parametrize("V", [5000, 4099])
+@pytest.mark.parametrize("off", [(0, 0, 4), (0, 4, 0), (4, 0, 0), (4, 4, 4)])
+def test_kl_against_own_log_probs_is_zero_at_any_alignment(dev, V, off):
+    x = (np.random.default_rng(V).standard_normal((3, V)) * 5).astype(np.float32)
+    bufs = [hipmem.Buffer(x.nbytes + 16) for _ in range(3)]  # the logits, their log-softmax, the logits for KL
+    at = [ctypes.c_void_p(b.ptr.value + o) for b, o in zip(bufs, off)]
+    for i in (0, 2):
+        bufs[i].upload(np.concatenate([np.zeros(off[i] // 4, np.float32), x.reshape(-1)]))
+    kl = hipmem.Buffer(3 * 8)
+    dev.logSoftmaxRows_device(at[1], at[0], 3, V)
+    dev.klRows_device(kl.ptr, at[1], at[2], 3, V)
+    dev.sync()
+    assert (kl.download(np.float64, (3,)) == 0).all()
 
 
 # one to eight rows an expert (instances of 2, 4 and 8 rows), nine (two chunks
