@@ -16,6 +16,9 @@ struct FewMat {
 // Whether the few-token product takes w on n tokens, from f32 rows or from
 // fragments (split_kernel's layout, few_ldk(K) k tiles).
 bool few_gemm_takes(const TileView &w, int64_t n, bool exact);
+// Estimated us of the product that runs otherwise, 33 to 255 tokens
+// (gemm_tile.hip).
+double large_gemm_us(const TileView &w, int64_t n);
 // k tiles of its fragments: whole 128-column steps (split_ldk)
 inline int64_t few_ldk(const TileView &w) { return split_ldk(w.cols); }
 // Whether it can read n f32 rows at x itself (no fragments).

@@ -473,6 +473,23 @@ void launch_rows(const FewCall &c, int64_t groups, int64_t steps) {
     else launch_cfg<TF, 1, 1, 4, XT, NX>(c);
 }
 
+// The tile of a product from fragments: token blocks x row groups.
+// Few row groups x token blocks: eight K slices over 16 rows (1024 x 4096
+// on 16 tokens: FP8 8.6 us, 10.3 with four over 32). Otherwise every
+// weight decoded feeds MT token blocks and every activation word NT row
+// groups; the larger tiles pay once the grid still fills the CUs (4096 x
+// 4096: MXFP4 on 48 tokens 13.0 us with 2 x 2, 15.0 with 1 x 2; on 96
+// tokens 19.1 with 2 x 4, 20.7; 14336 x 4096 on 16 tokens 15.4 with 1 x 2,
+// 19.6 with 2 x 2; FP8 on 128 tokens 55 us with 2 x 2, 66 with 2 x 4).
+// Three-term products hold half as many again.
+enum FewTile { FT_1x1, FT_1x2, FT_2x2, FT_2x4 };
+FewTile few_tile(int tf, int xt, int64_t groups, int64_t steps, int64_t tb) {
+    const int64_t units = groups * tb;
+    if (units <= 256 && steps > 16) return FT_1x1;
+    if (xt == 3 || tb == 1 || units < 640) return FT_1x2;
+    return units < 1536 || tf == TF_FP8 ? FT_2x2 : FT_2x4;
+}
+
 template <int TF, int XT>
 void launch_tf(const FewCall &c) {
     int64_t groups = 0;
@@ -485,20 +502,15 @@ void launch_tf(const FewCall &c) {
         else launch_rows<TF, XT, 8>(c, groups * ((c.n + 7) / 8), steps);
         return;
     }
-    // Few row groups x token blocks: eight K slices over 16 rows (1024 x 4096
-    // on 16 tokens: FP8 8.6 us, 10.3 with four over 32). Otherwise every
-    // weight decoded feeds MT token blocks and every activation word NT row
-    // groups; the larger tiles pay once the grid still fills the CUs (4096 x
-    // 4096: MXFP4 on 48 tokens 13.0 us with 2 x 2, 15.0 with 1 x 2; on 96
-    // tokens 19.1 with 2 x 4, 20.7; 14336 x 4096 on 16 tokens 15.4 with 1 x 2,
-    // 19.6 with 2 x 2). Three-term products hold half as many again.
-    const int64_t units = groups * tb;
-    if (units <= 256 && steps > 16) launch_cfg<TF, 1, 1, 8, XT, 0>(c);
-    else if (XT == 3 || tb == 1 || units < 640) launch_cfg<TF, 1, 2, 4, XT, 0>(c);
-    else if constexpr (XT == 2) {
-        // (FP8 on 128 tokens: 14336 x 4096 55 us with 2 x 2, 66 with 2 x 4)
-        if (units < 1536 || TF == TF_FP8) launch_cfg<TF, 2, 2, 4, XT, 0>(c);
-        else if constexpr (TF != TF_FP8) launch_cfg<TF, 2, 4, 4, XT, 0>(c);
+    switch (few_tile(TF, XT, groups, steps, tb)) {
+    case FT_1x1: launch_cfg<TF, 1, 1, 8, XT, 0>(c); break;
+    case FT_1x2: launch_cfg<TF, 1, 2, 4, XT, 0>(c); break;
+    case FT_2x2:
+        if constexpr (XT == 2) launch_cfg<TF, 2, 2, 4, XT, 0>(c);
+        break;
+    case FT_2x4:
+        if constexpr (XT == 2 && TF != TF_FP8) launch_cfg<TF, 2, 4, 4, XT, 0>(c);
+        break;
     }
 }
 
@@ -530,30 +542,41 @@ void launch_segs_tf(int tf, const FewParams<1> &q, int64_t rows, unsigned nseg, 
 
 }  // namespace
 
-// Up to 32 tokens for every shape; above that while the product is small
-// enough that the tiled and scaled-MFMA products, which multiply at twice the
-// rate and more, lose to their split-K passes and idle CUs. The lines, in
-// tokens x rows x columns, lie where the two measured the same (us here /
-// there): bf16 4096 x 4096 on 128 tokens 22 / 26, on 256 34 / 32, 14336 x
-// 4096 on 32 33 / 42, on 48 49 / 44; INT4 4096 x 4096 on 128 23 / 32, on 256
-// 37 / 37; MXFP4 14336 x 4096 on 96 37 / 47, 4096 x 4096 on 128 22 / 49. On
-// long rows the tiled product leaves most CUs without a tile: 4096 x 14336 on
-// 128 tokens FP8 52 / 57, INT4 55 / 60, Q8_0 51 / 167; bf16 on 64 49 / 51.
-// MXFP4 from 128 tokens on is three terms here (what the scaled MFMA holds):
-// 4096 x 4096 on 160 40 / 50, on 200 54 / 51, 1024 x 4096 on 255 24 / 50,
-// 4096 x 14336 on 160 117 / 146, on 200 175 / 146.
+// A call's time by its rounds of 256 workgroups, each an epilogue and a chain
+// over K: us a round, and a round and 1024 columns by tile, fitted to 3 900
+// calls of 33 to 255 tokens on 80 shapes of 256 to 32768 rows and 256 to 16384
+// columns (median error 6 %, MXFP4 from 128 tokens on with three terms).
+static double few_us(const TileView &w, int64_t n, int xt) {
+    struct Cost {
+        double round, k[4];
+    };
+    static constexpr Cost bf16{1.6, {1.2, 1.36, 1.9, 3.65}}, q8{2.2, {1.2, 1.2, 1.9, 3.35}}, fp8{0.7, {1.0, 1.3, 1.8, 0}},
+        mx4{0.3, {1.0, 1.1, 1.65, 2.45}}, mx4x3{0, {1.6, 1.56, 0, 0}}, int4{0.9, {1.15, 1.6, 2.07, 3.6}};
+    static constexpr int MT[4] = {1, 1, 2, 2}, NT[4] = {1, 2, 2, 4};
+    const Cost &c = w.tf == TF_BF16 ? bf16 : w.tf == TF_Q8 ? q8 : w.tf == TF_FP8 ? fp8 : w.tf == TF_INT4 ? int4
+                    : xt == 3 ? mx4x3 : mx4;
+    const int64_t groups = (w.rows + 15) / 16, tb = (n + 15) / 16;
+    const FewTile t = few_tile(w.tf, xt, groups, (w.cols + 127) / 128, tb);
+    const int64_t wgs = ((groups + NT[t] - 1) / NT[t]) * ((tb + MT[t] - 1) / MT[t]), rounds = (wgs + 255) / 256;
+    return 5.8 - c.round + rounds * (c.round + c.k[t] * w.cols / 1024.0);
+}
+
+// Up to 32 tokens for every shape; above that where it is ahead of the tiled,
+// scaled-MFMA or mid-batch product by the two estimates. Those multiply at
+// twice the rate and more but leave CUs idle or pass partial sums through
+// memory on few tokens, so this kernel wins while its grid is one round of the
+// CUs, and loses from two (long K) to five (short K) rounds on. us here /
+// there: bf16 4096 x 4096 on 128 tokens (one round) 20 / 25, on 160 (two) 34 /
+// 34; 16384 x 256 on 64 (two) 9.8 / 11.4, on 255 (eight) 27 / 14; 1024 x 14336
+// on 255 (two) 38 / 44, 4112 x 8192 on 48 (two) 36 / 29; INT4 16384 x 256 on
+// 160 (five) 16.1 / 16.6. Of 5 850 calls on 90 shapes eleven are 7 to 15 %
+// behind the product that runs otherwise (by lines in tokens x rows x columns
+// alone 300 of 3 700 were, up to 2.2 times).
 bool few_gemm_takes(const TileView &w, int64_t n, bool exact) {
     if (!w.fast || n < 1 || n > 255 || w.cols < 4) return false;
-    const bool bf16 = w.tf == TF_BF16, mx4 = w.tf == TF_MX4, q8 = w.tf == TF_Q8;
-    if (!bf16 && !mx4 && !q8 && w.tf != TF_FP8 && w.tf != TF_INT4) return false;
+    if (w.tf != TF_BF16 && w.tf != TF_MX4 && w.tf != TF_Q8 && w.tf != TF_FP8 && w.tf != TF_INT4) return false;
     if (n <= 32) return true;
-    if (exact) return false;
-    const double work = (double)n * w.rows * w.cols;
-    const bool long_k = w.cols >= 8192 && w.rows <= 4096;
-    if (mx4 && w.mx && n >= 128) return work <= (long_k ? 9.4e9 : 2.7e9);
-    if (mx4) return work <= (long_k ? 1.5e10 : 5.7e9);
-    if (q8) return work <= (long_k ? 1.5e10 : n > 64 ? 4.4e9 : 2.6e9);
-    return work <= (long_k ? (bf16 ? 3.8e9 : 7.6e9) : 2.6e9);
+    return !exact && few_us(w, n, mx_gemm_takes(w, n) ? 3 : 2) <= 1.02 * large_gemm_us(w, n);
 }
 
 bool few_reads_rows(const TileView &w, int64_t n, const float *x, int64_t ldx) {

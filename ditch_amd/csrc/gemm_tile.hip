@@ -30,6 +30,7 @@
 #include <type_traits>
 
 #include "gemm_common.h"
+#include "gemm_few.h"
 #include "gemm_wide.h"
 #include "tile_decode.h"
 
@@ -1710,6 +1711,25 @@ void launch_tile_glu(const TileView &gate, const TileView &up, uint32_t act, flo
     p.ldo = gate.rows;
     p.n = n;
     launch_tile_any<true>(p, 2, s);
+}
+
+// Fitted like few_us (gemm_few.hip): rounds of one workgroup a CU, each a chain
+// over its K part; partial sums written and added.
+double large_gemm_us(const TileView &w, int64_t n) {
+    const double k = w.cols / 1024.0;
+    auto rounds = [](int64_t wgs) { return (double)((wgs + 255) / 256); };
+    if (mx_gemm_takes(w, n)) {  // launch_mx
+        const int64_t tn = (w.rows + 511) / 512, t96 = (n + 95) / 96 * tn;
+        return rounds(t96 >= 256 ? t96 : (n + 63) / 64 * tn) * (10.7 + 9.7 * k);
+    }
+    if (wide_gemm_takes(w, n, 2, split_k_tiles(w))) {
+        const double r = rounds((w.rows + 63) / 64);
+        return n <= 64 ? 7.6 + 4.0 * r * k : n <= 128 ? 8.6 + 11.2 * r * k : 9.8 + 13.6 * r * k;
+    }
+    const int bn = 64 * tile_wgn(w.tf, 2), ks = tile_ksplit_of(w, n, 2);
+    const double part = w.tf == TF_BF16 ? 17 : w.tf == TF_Q8 ? 31 : w.tf == TF_FP8 ? 23 : w.tf == TF_INT4 ? 24 : 17;
+    return (w.tf == TF_BF16 ? 7 : 9) + rounds((n + 63) / 64 * ((w.rows + bn - 1) / bn) * ks) * part * k / ks +
+           (ks > 1 ? 3 + 1.9e-6 * ks * n * w.rows : 0);
 }
 
 // ---------------------------------------------------------------------------
