@@ -1,8 +1,12 @@
 """Products on f32 / f16 weights above 16 tokens (csrc/gemm_f32.hip) at the
-edges of the staged tiles: each tile and slice count of the dispatch, K of one
-unit (slices without any) and of slices of unequal length, ragged rows and
-tokens, rows that are not whole units, and a gathered non-finite activation
-that must stay in its token."""
+edges of the staged tiles: each tile and slice count of the dispatch and each
+span of its sums, ragged rows and tokens, K of one unit (slices without any),
+of slices of unequal length and of whole spans with a remainder, rows that are
+not whole units, and a gathered non-finite activation that must stay in its
+token."""
+import os
+import re
+
 import numpy as np
 import pytest
 
@@ -13,10 +17,43 @@ from test_gpu_kernels import TOL_MATMUL, close, dequant_f32
 pytestmark = pytest.mark.gpu
 
 
+# The kernel that each case runs, as <waves a side, K slices, units a sum>
+# (None: rows that are not whole units, the register-staged kernel)
+CASES = {
+    (17, 33, 32): (1, 4, 16), (40, 130, 160): (1, 4, 16), (100, 1000, 96): (1, 4, 16),
+    (1100, 950, 96): (1, 4, 16), (1090, 1030, 32): (1, 4, 16),
+    (40, 130, 2208): (1, 4, 16),  # 69 units: slices of 17 and 18, a whole sum and a remainder
+    (1024, 896, 160): (2, 2, 2), (1000, 885, 32): (2, 2, 2),  # (one unit: a slice without any)
+    (1000, 885, 1056): (2, 2, 4), (1000, 885, 2144): (2, 2, 16),  # 33 units: 16 and 17; 67: 33 and 34
+    (1030, 1310, 32): (2, 1, 2), (1030, 1310, 288): (2, 1, 2), (1030, 1310, 544): (2, 1, 4),
+    (1030, 1310, 2144): (2, 1, 16),
+    (50, 70, 72): None,
+}
+
+
+def _instance(n, rows, cols):
+    """launch_staged's choice, with the constants that its source has."""
+    path = os.path.join(os.path.dirname(__file__), "..", "ditch_amd", "csrc", "gemm_f32.hip")
+    with open(path) as f:
+        src = f.read()
+    one, two, small = map(float, re.search(r"\* 4 / ([\d.]+) : 4 / ([\d.]+);\n.*?/ 256\) / ([\d.]+);", src).groups())
+    whole, quarter = map(int, re.search(r"units_k < (\d+)\) \{\n +if \(p\.w\.units_k < (\d+)\)", src).groups())
+    if cols % 32:
+        return None
+
+    def tiles(side):
+        return -(-n // side) * -(-rows // side)
+
+    big = -(-tiles(64) // 256) * 4 / one if tiles(64) > 256 else 4 / two
+    wg, ks = (1, 4) if -(-tiles(32) // 256) / small < big else (2, 1) if tiles(64) > 256 else (2, 2)
+    units = cols // 32
+    return wg, ks, 16 if ks == 4 or units >= whole else 4 if units >= quarter else 2
+
+
 @pytest.mark.parametrize("kind", ["f32", "f16"])
-@pytest.mark.parametrize("n,rows,cols", [(17, 33, 32), (40, 130, 160), (100, 1000, 96), (1024, 896, 160),
-                                         (1100, 950, 96), (1090, 1030, 32), (50, 70, 72)])
+@pytest.mark.parametrize("n,rows,cols", list(CASES))
 def test_float_tiles(dev, ref, kind, n, rows, cols):
+    assert _instance(n, rows, cols) == CASES[n, rows, cols]
     rng = np.random.default_rng(n + rows + cols)
     w = wg.float_random(kind, rows, cols, rng)
     x = rng.standard_normal((n, cols)).astype(np.float32)

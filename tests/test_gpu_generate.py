@@ -196,10 +196,11 @@ def test_cache_chunked_prefill_equals_one_shot(dev, ref):
     assert np.abs(lg - lc).max() <= 1e-3 * np.abs(lc).max()
 
 
-# Attention of few rows (a workgroup per row and KV head): query groups of 7
-# (one pass of 8), 10 (8 + 2), 3 and 1, MLA's 192/128 head; decode rows at
-# the first and last position of a 1024-position cache, on both sides of the
-# wave counts' edges, and more rows than 127 (one a prompt).
+# Attention of few rows (a workgroup per row, KV head and up to 2 or 4 of its
+# query heads): query groups of 7 (2 + 2 + 2 + 1), 10 (4 + 4 + 2, from 256
+# workgroups on), 3 (2 + 1) and 1, MLA's 192/128 head; decode rows at the first
+# and last position of a 1024-position cache, on both sides of the wave
+# counts' edges, and more rows than 127 (one a prompt).
 ROW_ATTN = {
     "gqa7_hd64": (dict(heads=7, kv_heads=1, head_dim=64), [1, 33, 128, 90]),
     "gqa10_hd64_129_prompts": (dict(heads=10, kv_heads=1, head_dim=64), [1, 2, 3] * 43),

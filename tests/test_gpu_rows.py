@@ -44,10 +44,11 @@ def _check(gm, cm, lens, vocab, seed):
 LENS = [[1], [5, 3], [9], [7, 9], [17], [33], [63, 64], [128], [100, 30]]
 
 
-@pytest.mark.parametrize("fmt", ["bf16", "fp8", "mxfp4", "int4", "q8_0", "f32"])
-def test_forward_token_counts_match_oracle(dev, ref, fmt):
+# (gate and up in one launch: above 8 tokens where their rows are a multiple of 128; int4 rows are whole 128-column groups)
+@pytest.mark.parametrize("fmt,inter", [(f, i) for f in ("bf16", "fp8", "mxfp4", "int4", "q8_0", "f32") for i in (640, 672)
+                                       if f != "int4" or i == 640])
+def test_forward_token_counts_match_oracle(dev, ref, fmt, inter):
     """Plain layers, then with deltas on o and down (whose inputs stay f32)."""
-    inter = 640 if fmt == "int4" else 672  # (int4 rows are whole 128-column groups)
     spec = mg.dense(fmt, hidden=384, inter=inter, heads=6, kv_heads=2, head_dim=64, layers=2, vocab=640, seed=4)
     gm, cm = Model(dev, spec), RefModel(spec)
     rng = np.random.default_rng(5)
@@ -61,6 +62,34 @@ def test_forward_token_counts_match_oracle(dev, ref, fmt):
                 m.set_delta(li, slot, -1, a, b)
         for i, lens in enumerate(LENS):
             _check(gm, cm, lens, 640, 20 + i)
+    finally:
+        gm.free()
+        cm.free()
+
+
+# Gate and up in one launch (launch_glu): a layer on each side of its lines, by the 16-row groups of both matrices (rows
+# / 8), the 128-column steps and, from fragments, the 16-token blocks. The waves K is split over, from f32 rows and
+# from fragments, and the token blocks x row groups of a matrix a workgroup has there
+GLU_SHAPES = {
+    "8_waves_rows_and_fragments": (2176, 256, [[3], [9], [16]]),  # 32 groups, 17 steps, one block: 8; 8, 1 x 1
+    "8_waves_rows_last_step_half": (1088, 640, [[1], [2], [4], [5, 3], [13]]),  # 80 groups, 9 steps: 8; 4, 1 x 1
+    "4_waves_wide_rows": (1152, 4096, [[1], [6], [11]]),  # 512 groups, 9 steps: 4; 4, 1 x 1
+    "two_blocks": (128, 4096, [[17], [20, 12]]),  # 512 groups x 2 blocks: 4, 2 x 1
+    "two_blocks_of_two_groups": (128, 12288, [[17], [20, 12]]),  # 1536 groups x 2 blocks: 4, 2 x 2 (FP8: 2 x 1)
+}
+
+
+@pytest.mark.parametrize("fmt", ["bf16", "fp8", "mxfp4", "int4", "q8_0"])
+@pytest.mark.parametrize("shape", list(GLU_SHAPES))
+def test_gate_up_of_few_tokens_matches_oracle(dev, ref, fmt, shape):
+    hidden, inter, lens = GLU_SHAPES[shape]
+    if fmt == "int4":
+        hidden = -(-hidden // 128) * 128  # (whole 128-column groups)
+    spec = mg.dense(fmt, hidden=hidden, inter=inter, heads=2, kv_heads=1, head_dim=64, layers=1, vocab=256, seed=3)
+    gm, cm = Model(dev, spec), RefModel(spec)
+    try:
+        for i, prompts in enumerate(lens):
+            _check(gm, cm, prompts, 256, 40 + i)
     finally:
         gm.free()
         cm.free()
