@@ -180,12 +180,12 @@ int32_t ditch_hip_sync(ditch_hip *h) {
     return guarded(h, [&] { DITCH_TRY_HIP(hipStreamSynchronize(h->stream)); });
 }
 
-// The scratch of a product of n tokens on s. From 17 to 31 tokens a product
-// shares none with calls on other streams and holds none under capture (a
-// replay would use it after it has grown): only the context's own stream,
+// The scratch of a product of n tokens on s. Up to 8 tokens and from 17 to 31 a
+// product shares none with calls on other streams and holds none under capture
+// (a replay would use it after it has grown): only the context's own stream,
 // outside a capture, has fragments.
 static DevBuf *product_scratch(ditch_hip *h, uint64_t n, hipStream_t s) {
-    if (n < 17 || n > 31) return &h->split;
+    if (n > 8 && (n < 17 || n > 31)) return &h->split;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (s == h->stream) DITCH_TRY_HIP(hipStreamIsCapturing(s, &cap));
     return s == h->stream && cap == hipStreamCaptureStatusNone ? &h->few : nullptr;

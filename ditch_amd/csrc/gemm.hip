@@ -146,7 +146,7 @@ static bool gemv_ahead(const TileView &w, int64_t n) {
 void launch_matmul(const TileView &w, float *out, const float *x, int64_t n, const MatmulEpilogue &ep, hipStream_t s,
                    const int32_t *row_index, DevBuf *ws) {
     if (n <= 0 || w.rows <= 0) return;
-    if (few_gemm_takes(w, n, ep.exact != 0) && !(ws && !ep.exact && gemv_ahead(w, n))) {
+    if (few_gemm_takes(w, n, ep.exact != 0) && !((ws || n <= 8) && !ep.exact && gemv_ahead(w, n))) {
         // (three terms too where the product they stand in for is the scaled
         // MFMA's, whose fp6 terms hold 18 bits)
         const int xt = ep.exact || mx_gemm_takes(w, n) ? 3 : 2;

@@ -178,7 +178,8 @@ struct ditch_hip {
     int cu_count = 0;
     // activation fragments of the tiled GEMM for the context's own products
     ditch::DevBuf split;
-    // those of 17 to 31 tokens on the context's stream, which orders their uses
+    // those of up to 8 and of 17 to 31 tokens on the context's stream, which
+    // orders their uses
     ditch::DevBuf few;
     // per-chunk partials of the row-split log-softmax / KL
     ditch::DevBuf rowred;

@@ -103,10 +103,12 @@ def _stream(lib):
 
 
 @pytest.mark.parametrize("kind,n,rows,cols", [("bf16", 17, 50, 132), ("fp8", 24, 8208, 320), ("mxfp4", 25, 4096, 256),
-                                              ("int4", 31, 130, 2240), ("q8_0", 20, 33, 1056), ("bf16", 18, 40, 30)])
+                                              ("int4", 31, 130, 2240), ("q8_0", 20, 33, 1056), ("bf16", 18, 40, 30),
+                                              ("fp8", 5, 50, 131), ("bf16", 8, 33, 4099)])
 def test_chunks_of_rows_on_another_stream(dev, ref, kind, n, rows, cols):
     """17 to 31 tokens without scratch: chunks of 8 rows (the last one of any
-    size), or the register-staged product where rows are not whole float4s."""
+    size), or the register-staged product where rows are not whole float4s.
+    Up to 8 tokens of such rows: the GEMV."""
     rng = np.random.default_rng(n + rows + cols)
     w = wg.make(kind, rows, cols, rng)
     x = rng.standard_normal((n, cols)).astype(np.float32)
@@ -127,17 +129,20 @@ def test_chunks_of_rows_on_another_stream(dev, ref, kind, n, rows, cols):
     assert (np.abs(got - want) <= TOL_MATMUL["atol"] + TOL_MATMUL["rtol"] * np.abs(want) + bound).all()
 
 
-def test_products_of_17_to_31_tokens_on_two_streams(dev, ref):
-    """No order between the streams and the context's own: every output is
-    that of the call alone."""
+@pytest.mark.parametrize("counts,kinds", [((17, 24, 31), (("fp8", 2048, 1024), ("int4", 1024, 4096))),
+                                          ((1, 5, 8), (("fp8", 2048, 1026), ("bf16", 512, 4102)))])
+def test_products_without_shared_scratch_on_two_streams(dev, ref, counts, kinds):
+    """17 to 31 tokens, and up to 8 whose rows are not whole float4s. No order
+    between the streams and the context's own: every output is that of the
+    call alone."""
     rng = np.random.default_rng(8)
     lib = hipmem.hip()
     streams = [_stream(lib).value, _stream(lib).value, None]
-    t = [dev.upload(wg.make("fp8", 2048, 1024, rng)), dev.upload(wg.make("int4", 1024, 4096, rng))]
+    t = [dev.upload(wg.make(*kind, rng)) for kind in kinds]
     try:
         jobs = []
         for i in range(24):
-            w, n = t[i % 2], (17, 24, 31)[i // 2 % 3]
+            w, n = t[i % 2], counts[i // 2 % 3]
             bx = hipmem.Buffer.from_array(rng.standard_normal((n, w.cols)).astype(np.float32))
             outs = [hipmem.Buffer(n * w.rows * 4) for _ in range(2)]
             jobs.append((w, n, bx, outs, streams[i % 3]))
@@ -157,8 +162,9 @@ def test_products_of_17_to_31_tokens_on_two_streams(dev, ref):
             lib.hipStreamDestroy(s)
 
 
+@pytest.mark.parametrize("n,cols", [(24, 2048), (6, 2050)])
 @pytest.mark.parametrize("own", [False, True])
-def test_product_of_24_tokens_captured_without_a_warm_up(dev, own):
+def test_product_captured_without_a_warm_up(dev, own, n, cols):
     """On another stream and on the context's own: nothing is allocated under
     the capture, and a larger product afterwards leaves the graph's replays."""
     lib = hipmem.hip()
@@ -169,7 +175,7 @@ def test_product_of_24_tokens_captured_without_a_warm_up(dev, own):
         getattr(lib, name).argtypes = args
         getattr(lib, name).restype = ctypes.c_int
     rng = np.random.default_rng(9)
-    n, rows, cols = 24, 512, 2048
+    rows = 512
     t, big = dev.upload(wg.make("fp8", rows, cols, rng)), dev.upload(wg.make("fp8", 64, 16384, rng))
     made = None if own else _stream(lib)
     stream = P(dev.stream) if own else made
