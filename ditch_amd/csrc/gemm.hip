@@ -136,9 +136,12 @@ static void dispatch_tf(int tf, const GemmParams &p, int64_t max_rows, int64_t n
 // x 4096 on 9 8.8 / 9.4, 14336 x 4096 on 16 29 / 31; Q8_0 14336 x 4096 on 9
 // 15.8 / 17.0, 1024 x 4096 9.9 / 9.4), and weights past the 256 MB cache: bf16
 // 89312 x 2048 on 5 59.3 / 63.2, Q8_0 128256 x 4096 on 4 91 / 96, on 8 119 / 112.
-static bool gemv_ahead(const TileView &w, int64_t n) {
+// Up to 8 tokens bf16 also where the rows cannot be read as float4s (`rows`)
+// and K is short: 896 x 450 on 2 4.6 / 7.5, 4096 x 898 on 8 5.2 / 7.6, 65536 x
+// 898 on 1 20.4 / 23.4; 4096 x 2050 6.8 / 7.2, 1024 x 4099 12.4 / 8.5.
+static bool gemv_ahead(const TileView &w, int64_t n, bool rows) {
     const int64_t elements = w.rows * w.cols;
-    if (w.tf == TF_BF16) return n <= 16 && (n > 8 || elements > (1 << 27));
+    if (w.tf == TF_BF16) return n <= 16 && (n > 8 || elements > (1 << 27) || (!rows && w.cols < 4096));
     if (w.tf == TF_Q8) return n <= 16 && (n > 8 ? w.rows >= 4096 : n <= 4 && elements > (1 << 28));
     return false;
 }
@@ -146,11 +149,12 @@ static bool gemv_ahead(const TileView &w, int64_t n) {
 void launch_matmul(const TileView &w, float *out, const float *x, int64_t n, const MatmulEpilogue &ep, hipStream_t s,
                    const int32_t *row_index, DevBuf *ws) {
     if (n <= 0 || w.rows <= 0) return;
-    if (few_gemm_takes(w, n, ep.exact != 0) && !((ws || n <= 8) && !ep.exact && gemv_ahead(w, n))) {
+    const bool float4s = !row_index && few_reads_rows(w, n, x, w.cols);
+    if (few_gemm_takes(w, n, ep.exact != 0) && !((ws || n <= 8) && !ep.exact && gemv_ahead(w, n, float4s))) {
         // (three terms too where the product they stand in for is the scaled
         // MFMA's, whose fp6 terms hold 18 bits)
         const int xt = ep.exact || mx_gemm_takes(w, n) ? 3 : 2;
-        const bool rows = (n <= 8 || !ws) && !row_index && few_reads_rows(w, n, x, w.cols);
+        const bool rows = (n <= 8 || !ws) && float4s;
         const size_t xb = rows ? 0 : split_bytes_ldk(n, few_ldk(w), xt);
         // (fragments past a borrowed scratch: the products below need less)
         if (rows || (ws && !(ws->borrowed && xb > ws->bytes))) {
