@@ -154,7 +154,12 @@ void launch_matmul(const TileView &w, float *out, const float *x, int64_t n, con
         // (three terms too where the product they stand in for is the scaled
         // MFMA's, whose fp6 terms hold 18 bits)
         const int xt = ep.exact || mx_gemm_takes(w, n) ? 3 : 2;
-        const bool rows = (n <= 8 || !ws) && float4s;
+        // (from 17 tokens on chunks of 8 rows where the weights are few: one launch,
+        // 64 x 32 on 24 tokens bf16 5.2 us, 7.6 with fragments and 5.0 with the
+        // register-staged product; 4096 x 1024 bf16 6.1 / 7.7, INT4 7.0 / 7.3; 4096 x
+        // 2048 8.1 / 8.5 and 10.1 / 8.7)
+        const bool chunks = n > 16 && w.rows * w.cols <= (1 << 22);
+        const bool rows = (n <= 8 || chunks || !ws) && float4s;
         const size_t xb = rows ? 0 : split_bytes_ldk(n, few_ldk(w), xt);
         // (fragments past a borrowed scratch: the products below need less)
         if (rows || (ws && !(ws->borrowed && xb > ws->bytes))) {

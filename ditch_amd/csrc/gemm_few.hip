@@ -22,8 +22,9 @@
 //   - up to 8 tokens (NX) each wave splits its slice of the f32 rows into bf16
 //     terms itself, in its own LDS slot; more tokens come as fragments
 //     (split_kernel's layout), which producers write directly, or, where the
-//     caller has no scratch for them, in chunks of 8 (24 tokens: 0.6 to 0.9 of
-//     the fragments' time below 4 M weights, 1.2 to 1.9 of it at 14336 x 4096);
+//     caller has no scratch for them or there are few weights, in chunks of 8 (24
+//     tokens: 0.6 to 0.9 of the fragments' time below 4 M weights, 1.2 to 1.9 of
+//     it at 14336 x 4096);
 //   - one launch may hold up to three matrices over the same activations.
 //
 // Measured, us a call with its split (before: the GEMV up to 16 tokens, the

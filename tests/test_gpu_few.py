@@ -26,6 +26,8 @@ CASES = [
     ("int4", 1, 130, 192), ("int4", 4, 72, 4224), ("int4", 8, 16, 128), ("int4", 10, 260, 2240),
     ("int4", 48, 4000, 256), ("int4", 130, 72, 1024),
     ("q8_0", 2, 8208, 96), ("q8_0", 6, 70, 4128), ("q8_0", 15, 33, 1056), ("q8_0", 64, 3080, 64), ("q8_0", 129, 40, 416),
+    # 17 to 31 tokens: chunks of rows up to 2^22 weights, fragments above
+    ("fp8", 31, 4096, 1024), ("bf16", 24, 4100, 1028), ("mxfp4", 31, 2080, 2080), ("int4", 17, 4112, 1152),
     # odd rows of up to 8 tokens on both sides of the GEMV's line
     ("bf16", 5, 40, 4094), ("bf16", 5, 40, 4098), ("fp8", 3, 40, 30),
 ]
