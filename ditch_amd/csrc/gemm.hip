@@ -149,8 +149,14 @@ static bool gemv_ahead(const TileView &w, int64_t n, bool rows) {
 void launch_matmul(const TileView &w, float *out, const float *x, int64_t n, const MatmulEpilogue &ep, hipStream_t s,
                    const int32_t *row_index, DevBuf *ws) {
     if (n <= 0 || w.rows <= 0) return;
+    // without scratch from 17 tokens on, the tallest weights by the register-staged
+    // product: chunks read them once each (us chunks / there, 24 tokens: bf16
+    // 131072 x 896 67 / 48, 98304 x 2048 123 / 102, 65536 x 1024 40 / 44 and on 31
+    // 50 / 43, 65536 x 2048 68 / 79; Q8_0 131072 x 896 72 / 57)
+    const bool staged = !ws && n > 16 && (w.tf == TF_BF16 || w.tf == TF_Q8) && w.rows >= 65536 &&
+                        (w.rows >= 98304 || w.cols <= 1024);
     const bool float4s = !row_index && few_reads_rows(w, n, x, w.cols);
-    if (few_gemm_takes(w, n, ep.exact != 0) && !((ws || n <= 8) && !ep.exact && gemv_ahead(w, n, float4s))) {
+    if (few_gemm_takes(w, n, ep.exact != 0) && !staged && !((ws || n <= 8) && !ep.exact && gemv_ahead(w, n, float4s))) {
         // (three terms too where the product they stand in for is the scaled
         // MFMA's, whose fp6 terms hold 18 bits)
         const int xt = ep.exact || mx_gemm_takes(w, n) ? 3 : 2;

@@ -562,21 +562,28 @@ static double few_us(const TileView &w, int64_t n, int xt) {
     return 5.8 - c.round + rounds * (c.round + c.k[t] * w.cols / 1024.0);
 }
 
-// Up to 32 tokens for every shape; above that where it is ahead of the tiled,
-// scaled-MFMA or mid-batch product by the two estimates. Those multiply at
-// twice the rate and more but leave CUs idle or pass partial sums through
-// memory on few tokens, so this kernel wins while its grid is one round of the
-// CUs, and loses from two (long K) to five (short K) rounds on. us here /
-// there: bf16 4096 x 4096 on 128 tokens (one round) 20 / 25, on 160 (two) 34 /
-// 34; 16384 x 256 on 64 (two) 9.8 / 11.4, on 255 (eight) 27 / 14; 1024 x 14336
-// on 255 (two) 38 / 44, 4112 x 8192 on 48 (two) 36 / 29; INT4 16384 x 256 on
-// 160 (five) 16.1 / 16.6. Of 5 850 calls on 90 shapes eleven are 7 to 15 %
-// behind the product that runs otherwise (by lines in tokens x rows x columns
-// alone 300 of 3 700 were, up to 2.2 times).
+// Up to 32 tokens every shape but the tallest from 17 on, whose many rounds'
+// epilogues outweigh a short K. us here / there, 17 to 31 tokens: bf16 65536 x
+// 256 17 / 12, 131072 x 512 41 / 30, 65536 x 512 24 / 25, 65536 x 896 33 / 39;
+// Q8_0 131072 x 256 32 / 20, 131072 x 512 39 / 36. 32 tokens, bf16: 65536 x 896
+// 34 / 26, 65536 x 4096 136 / 112, 32768 x 896 21 / 23.
+// Above 32 where it is ahead of the tiled, scaled-MFMA or mid-batch product by
+// the two estimates. Those multiply at twice the rate and more but leave CUs
+// idle or pass partial sums through memory on few tokens, so this kernel wins
+// while its grid is one round of the CUs, and loses from two (long K) to five
+// (short K) rounds on. us here / there: bf16 4096 x 4096 on 128 tokens (one
+// round) 20 / 25, on 160 (two) 34 / 34; 16384 x 256 on 64 (two) 9.8 / 11.4, on
+// 255 (eight) 27 / 14; 1024 x 14336 on 255 (two) 38 / 44, 4112 x 8192 on 48
+// (two) 36 / 29; INT4 16384 x 256 on 160 (five) 16.1 / 16.6. Of 5 850 calls on
+// 90 shapes eleven are 7 to 15 % behind the product that runs otherwise (by
+// lines in tokens x rows x columns alone 300 of 3 700 were, up to 2.2 times).
 bool few_gemm_takes(const TileView &w, int64_t n, bool exact) {
     if (!w.fast || n < 1 || n > 255 || w.cols < 4) return false;
     if (w.tf != TF_BF16 && w.tf != TF_MX4 && w.tf != TF_Q8 && w.tf != TF_FP8 && w.tf != TF_INT4) return false;
-    if (n <= 32) return true;
+    if (n <= 32) {
+        if (exact || n <= 16 || w.rows < 65536) return true;
+        return w.tf == TF_BF16 ? n < 32 && w.cols > 512 : w.tf != TF_Q8 || w.cols > 256;
+    }
     return !exact && few_us(w, n, mx_gemm_takes(w, n) ? 3 : 2) <= 1.02 * large_gemm_us(w, n);
 }
 

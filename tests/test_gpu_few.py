@@ -30,6 +30,9 @@ CASES = [
     ("fp8", 31, 4096, 1024), ("bf16", 24, 4100, 1028), ("mxfp4", 31, 2080, 2080), ("int4", 17, 4112, 1152),
     # odd rows of up to 8 tokens on both sides of the GEMV's line
     ("bf16", 5, 40, 4094), ("bf16", 5, 40, 4098), ("fp8", 3, 40, 30),
+    # the tallest weights from 17 tokens on: the products that ran before
+    ("bf16", 24, 65540, 64), ("bf16", 32, 65540, 96), ("bf16", 17, 65540, 516), ("q8_0", 20, 65540, 64),
+    ("q8_0", 32, 65540, 64), ("int4", 31, 65540, 128),
 ]
 
 
@@ -108,10 +111,12 @@ def _stream(lib):
 
 @pytest.mark.parametrize("kind,n,rows,cols", [("bf16", 17, 50, 132), ("fp8", 24, 8208, 320), ("mxfp4", 25, 4096, 256),
                                               ("int4", 31, 130, 2240), ("q8_0", 20, 33, 1056), ("bf16", 18, 40, 30),
-                                              ("fp8", 5, 50, 131), ("bf16", 8, 33, 4099)])
+                                              ("fp8", 5, 50, 131), ("bf16", 8, 33, 4099),
+                                              ("bf16", 20, 65540, 64), ("q8_0", 31, 98304, 64), ("bf16", 17, 65540, 1028)])
 def test_chunks_of_rows_on_another_stream(dev, ref, kind, n, rows, cols):
     """17 to 31 tokens without scratch: chunks of 8 rows (the last one of any
-    size), or the register-staged product where rows are not whole float4s.
+    size), or the register-staged product where rows are not whole float4s or the
+    weights are the tallest.
     Up to 8 tokens of such rows: the GEMV."""
     rng = np.random.default_rng(n + rows + cols)
     w = wg.make(kind, rows, cols, rng)
