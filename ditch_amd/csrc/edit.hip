@@ -255,9 +255,9 @@ __global__ __launch_bounds__(1024) void edit_orth_reg_kernel(float *vecs, int64_
 // The neighbours ride along: the operator's second half on the product the
 // chunk is read from (`scale`, `u`), the dot products the next half needs and
 // the row-scaled copy it multiplies (`pa`, `cy`).
-// 6 to 9 us a launch (latency: the parts, the factorisation, the columns); the
-// 28 orthonormalisations and their neighbours of an 896 x 4864 edit took 67 to
-// 100 us each and 12 to 20 us of neighbours.
+// 6 to 9 us a launch (latency: the parts, the factorisation, the columns); each
+// of the 13 orthonormalisations of an 896 x 4864 edit took 67 to 100 us, and 12
+// to 20 us of neighbours.
 constexpr int ED_GRAM_Q = 24;  // vectors: LDS for a 256-column chunk and the parts
 constexpr int ED_GRAM_K = 8;   // directions of the neighbours
 struct OrthArgs {
@@ -403,6 +403,90 @@ __global__ __launch_bounds__(256) void edit_orth_chunk_kernel(OrthArgs a) {
     };
     if (a.pa) dots(q * k, false, a.dots_out);
     if (a.gram_out) dots(pairs, true, a.gram_out);
+}
+
+// The same two passes by one workgroup, the vectors in registers: up to Q of
+// at most 1024 EPT columns (an input-side ablation's, which have no neighbours).
+// Bound by the launch and four barriers; three launches and their gaps took
+// longer than the vector-by-vector kernels above, us an ablated edit with these,
+// the three launches and here: 256 columns 2 directions 58 / 69 / 64, 3072
+// columns 2 and 4 64 / 73 / 63 and 83 / 74 / 73; from 14336 columns on equal.
+template <int Q, int EPT>
+__global__ __launch_bounds__(1024) void edit_orth_small_kernel(float *v, int q, int64_t n) {
+    constexpr int P = Q * (Q + 1) / 2;
+    __shared__ double parts[16][P], gram[P];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    float x[Q][EPT];
+#pragma unroll
+    for (int i = 0; i < Q; i++)
+#pragma unroll
+        for (int m = 0; m < EPT; m++) {
+            const int64_t t = (int64_t)m * 1024 + tid;
+            x[i][m] = i < q && t < n ? v[i * n + t] : 0.f;
+        }
+    for (int pass = 0; pass < 2; pass++) {
+#pragma unroll
+        for (int i = 0; i < Q; i++)
+#pragma unroll
+            for (int j = 0; j <= i; j++) {
+                if (i >= q) continue;
+                double r = 0.0;
+#pragma unroll
+                for (int m = 0; m < EPT; m++) r += (double)x[i][m] * (double)x[j][m];
+                r = ed_wave_total(r);
+                if (lane == 0) parts[wave][i * (i + 1) / 2 + j] = r;
+            }
+        __syncthreads();
+        if (tid < q * (q + 1) / 2) {
+            double r = 0.0;
+#pragma unroll
+            for (int w = 0; w < 16; w++) r += parts[w][tid];
+            gram[tid] = r;
+        }
+        __syncthreads();
+        double l[Q][Q], inv[Q];  // the Cholesky factor, as edit_orth_chunk_kernel's
+#pragma unroll
+        for (int j = 0; j < Q; j++) {
+            inv[j] = 0.0;
+            if (j >= q) continue;
+            const double d = gram[j * (j + 1) / 2 + j];
+            double r = d;
+#pragma unroll
+            for (int c = 0; c < j; c++) r -= l[j][c] * l[j][c];
+            double y = __builtin_amdgcn_rsq(r);
+#pragma unroll
+            for (int it = 0; it < 2; it++) y = y * (1.5 - 0.5 * r * y * y);
+            inv[j] = r > 1e-14 * d && r > 1e-40 ? y : 0.0;
+#pragma unroll
+            for (int i = j + 1; i < Q; i++) {
+                if (i >= q) continue;
+                double g = gram[i * (i + 1) / 2 + j];
+#pragma unroll
+                for (int c = 0; c < j; c++) g -= l[i][c] * l[j][c];
+                l[i][j] = inv[j] > 0.0 ? g * y : 0.0;
+            }
+        }
+#pragma unroll
+        for (int m = 0; m < EPT; m++) {
+            double xd[Q];
+#pragma unroll
+            for (int i = 0; i < Q; i++) {
+                if (i >= q) continue;
+                double acc = (double)x[i][m];
+#pragma unroll
+                for (int j = 0; j < i; j++) acc -= l[i][j] * xd[j];
+                x[i][m] = inv[i] > 0.0 ? (float)(acc * inv[i]) : 0.f;
+                xd[i] = (double)x[i][m];
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < Q; i++)
+#pragma unroll
+        for (int m = 0; m < EPT; m++) {
+            const int64_t t = (int64_t)m * 1024 + tid;
+            if (i < q && t < n) v[i * n + t] = x[i][m];
+        }
 }
 
 // SVD widths up to ED_LDS_Q keep the Jacobi's two q x q matrices in LDS;
@@ -650,6 +734,13 @@ static void edit_orth_chunks(EditWork &W, OrthArgs first, OrthArgs last, hipStre
 }
 
 static void edit_orth(EditWork &W, float *vecs, int64_t q, int64_t n, hipStream_t s) {
+    if ((q <= 4 && n <= 4096) || (q <= 2 && n <= 8192)) {
+        if (n <= 1024) hipLaunchKernelGGL((edit_orth_small_kernel<4, 1>), dim3(1), dim3(1024), 0, s, vecs, (int)q, n);
+        else if (n <= 4096) hipLaunchKernelGGL((edit_orth_small_kernel<4, 4>), dim3(1), dim3(1024), 0, s, vecs, (int)q, n);
+        else hipLaunchKernelGGL((edit_orth_small_kernel<2, 8>), dim3(1), dim3(1024), 0, s, vecs, (int)q, n);
+        DITCH_TRY_HIP(hipGetLastError());
+        return;
+    }
     if (orth_takes(q, 0)) {
         OrthArgs a{};
         a.v = vecs;

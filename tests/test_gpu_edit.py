@@ -93,6 +93,37 @@ def test_device_edit_matches_oracle(dev, ref, fmt, rows, cols, k, mode, ablate):
         assert np.linalg.norm(dstar - gd) <= 1.10 * best + 1e-6 * np.linalg.norm(dstar)
 
 
+# the input side's U = orth(W^T V): one workgroup of 1, 4 and 8 columns a thread (up to 4, 4 and 2 vectors), three
+# launches past them
+@pytest.mark.parametrize("cols,k", [(30, 1), (1024, 4), (1026, 2), (4096, 4), (4096, 5), (4100, 1), (4100, 3), (8192, 2),
+                                    (8194, 2)])
+def test_input_side_directions_are_orthonormal(dev, ref, cols, k):
+    rng = np.random.default_rng(cols + k)
+    w = HostWeight.f32((rng.standard_normal((96, cols)) * 0.02).astype(np.float32))
+    v = orthonormal_rows(rng, k, 96)
+    a, _ = dev.edit_delta_ex(w, v, 1.0, "none", ablate=True)
+    u = a[k:].astype(np.float64)
+    want = v.astype(np.float64) @ ref.dequant(w).astype(np.float64)
+    for i in range(k):
+        for j in range(i):
+            want[i] -= (want[i] @ want[j]) * want[j]
+        want[i] /= np.linalg.norm(want[i])
+    # one rounding an element; f32 sums over 96 rows (at most 96 * 2^-24 of the norm, nearly orthogonal vectors)
+    assert np.abs(u @ u.T - np.eye(k)).max() <= 2.0**-22
+    assert np.linalg.norm(u - want, axis=1).max() <= 96 * 2.0**-24 * 2
+
+
+def test_input_side_direction_that_repeats_is_zero(dev):
+    rng = np.random.default_rng(3)
+    w = HostWeight.f32((rng.standard_normal((64, 700)) * 0.02).astype(np.float32))
+    v = orthonormal_rows(rng, 3, 64)
+    v[1] = v[0]
+    a, b = dev.edit_delta_ex(w, v, 1.0, "none", ablate=True)
+    u = a[3:].astype(np.float64)
+    assert (u[1] == 0).all() and np.abs(u[[0, 2]] @ u[[0, 2]].T - np.eye(2)).max() <= 2.0**-22
+    assert np.isfinite(a).all() and np.isfinite(b).all()
+
+
 WIDE = [("f32", 300, 400, 2, "full", 40), ("bf16", 320, 400, 3, "full", 70), ("int4", 384, 512, 20, "pre", 3),
         ("fp8", 384, 1024, 24, "none", 3)]
 
