@@ -649,7 +649,7 @@ bool attention_mfma_takes(int64_t hd, int64_t vd, int64_t groups) {
 // another on a workgroup per KV head: 116 us for 16 prompts of 32 to 96 keys
 // (2 KV heads of 64), 69 us for one row of 500 keys (8 KV heads of 128).
 // Here a row's keys and values are read once, straight into registers, by
-// 4 to 16 waves with several rows of the cache in flight each: 5 and 9 us.
+// 4 to 16 waves with several rows of the cache in flight each: 6 and 12 us.
 // What bounds it is that read (3.4 TB/s over 48 rows of 300 to 900 keys; one
 // CU's loads for a single row) and two barriers.
 //

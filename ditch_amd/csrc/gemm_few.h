@@ -16,6 +16,11 @@ struct FewMat {
 // Whether the few-token product takes w on n tokens, from f32 rows or from
 // fragments (split_kernel's layout, few_ldk(K) k tiles).
 bool few_gemm_takes(const TileView &w, int64_t n, bool exact);
+// Whether it takes several matrices of one format and K in one launch, over
+// fragments that their producer writes, instead of a product and a split each
+// (and saved_us of other work).
+constexpr double FEW_SPLIT_US = 3;
+bool few_launch_takes(const TileView *const *w, int count, int64_t n, double saved_us);
 // Estimated us of the product that runs otherwise, 33 to 255 tokens
 // (gemm_tile.hip).
 double large_gemm_us(const TileView &w, int64_t n);

@@ -547,7 +547,7 @@ void launch_segs_tf(int tf, const FewParams<1> &q, int64_t rows, unsigned nseg, 
 // over K: us a round, and a round and 1024 columns by tile, fitted to 3 900
 // calls of 33 to 255 tokens on 80 shapes of 256 to 32768 rows and 256 to 16384
 // columns (median error 6 %, MXFP4 from 128 tokens on with three terms).
-static double few_us(const TileView &w, int64_t n, int xt) {
+static double few_us(const TileView &w, int64_t rows, int64_t n, int xt) {
     struct Cost {
         double round, k[4];
     };
@@ -556,7 +556,7 @@ static double few_us(const TileView &w, int64_t n, int xt) {
     static constexpr int MT[4] = {1, 1, 2, 2}, NT[4] = {1, 2, 2, 4};
     const Cost &c = w.tf == TF_BF16 ? bf16 : w.tf == TF_Q8 ? q8 : w.tf == TF_FP8 ? fp8 : w.tf == TF_INT4 ? int4
                     : xt == 3 ? mx4x3 : mx4;
-    const int64_t groups = (w.rows + 15) / 16, tb = (n + 15) / 16;
+    const int64_t groups = (rows + 15) / 16, tb = (n + 15) / 16;
     const FewTile t = few_tile(w.tf, xt, groups, (w.cols + 127) / 128, tb);
     const int64_t wgs = ((groups + NT[t] - 1) / NT[t]) * ((tb + MT[t] - 1) / MT[t]), rounds = (wgs + 255) / 256;
     return 5.8 - c.round + rounds * (c.round + c.k[t] * w.cols / 1024.0);
@@ -577,14 +577,34 @@ static double few_us(const TileView &w, int64_t n, int xt) {
 // (two) 36 / 29; INT4 16384 x 256 on 160 (five) 16.1 / 16.6. Of 5 850 calls on
 // 90 shapes eleven are 7 to 15 % behind the product that runs otherwise (by
 // lines in tokens x rows x columns alone 300 of 3 700 were, up to 2.2 times).
+static bool few_form(const TileView &w, int64_t n) {
+    return w.fast && n >= 1 && n <= 255 && w.cols >= 4 &&
+           (w.tf == TF_BF16 || w.tf == TF_MX4 || w.tf == TF_Q8 || w.tf == TF_FP8 || w.tf == TF_INT4);
+}
 bool few_gemm_takes(const TileView &w, int64_t n, bool exact) {
-    if (!w.fast || n < 1 || n > 255 || w.cols < 4) return false;
-    if (w.tf != TF_BF16 && w.tf != TF_MX4 && w.tf != TF_Q8 && w.tf != TF_FP8 && w.tf != TF_INT4) return false;
+    if (!few_form(w, n)) return false;
     if (n <= 32) {
         if (exact || n <= 16 || w.rows < 65536) return true;
         return w.tf == TF_BF16 ? n < 32 && w.cols > 512 : w.tf != TF_Q8 || w.cols > 256;
     }
-    return !exact && few_us(w, n, mx_gemm_takes(w, n) ? 3 : 2) <= 1.02 * large_gemm_us(w, n);
+    return !exact && few_us(w, w.rows, n, mx_gemm_takes(w, n) ? 3 : 2) <= 1.02 * large_gemm_us(w, n);
+}
+
+// Several matrices in one launch share its rounds and its fragments, which their
+// producer writes: above 32 tokens one estimate for all of them against the sum
+// of theirs and what the launch saves besides. Matrix by matrix, some went one
+// way and some the other: two layers of 896 x 4864 Q8_0 on 40 tokens 104 us with
+// all here, 133 mixed; of 4096 x 14336 bf16 350 and 402.
+bool few_launch_takes(const TileView *const *w, int count, int64_t n, double saved_us) {
+    int64_t rows = 0;
+    double other = saved_us;
+    for (int i = 0; i < count; i++) {
+        if (!few_form(*w[i], n) || w[i]->tf != w[0]->tf || w[i]->cols != w[0]->cols) return false;
+        if (n <= 32 && !few_gemm_takes(*w[i], n, false)) return false;
+        rows += w[i]->rows;
+        if (n > 32) other += large_gemm_us(*w[i], n);
+    }
+    return n <= 32 || few_us(*w[0], rows, n, 2) <= other;
 }
 
 bool few_reads_rows(const TileView &w, int64_t n, const float *x, int64_t ldx) {
@@ -616,8 +636,9 @@ void launch_few_gemm(const FewMat *mats, int nmat, const float *x, int64_t ldx, 
 }
 
 bool few_glu_takes(const TileView &gate, const TileView &up, int64_t n) {
+    const TileView *const mats[2] = {&gate, &up};  // (saves the down product's split and the activation's launch too)
     return gate.tf == up.tf && gate.rows == up.rows && gate.cols == up.cols && gate.units_k == up.units_k &&
-           few_gemm_takes(gate, n, false) && few_gemm_takes(up, n, false) &&
+           few_launch_takes(mats, 2, n, 2 * FEW_SPLIT_US + 5) &&
            gate.scale_type == up.scale_type && gate.group == up.group && gate.block_cols == up.block_cols &&
            gate.side_cols == up.side_cols;
 }

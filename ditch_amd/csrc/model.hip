@@ -1133,12 +1133,19 @@ static bool mx_only(const Mat &mt, int64_t n) { return mt.ok() && mt.rank == 0 &
 // Whether the few-token product takes every one of up to three matrices over
 // one activation in one launch (no deltas, one format and width).
 static bool few_together(std::initializer_list<const Mat *> mats, int64_t n) {
-    const Mat *first = *mats.begin();
-    for (const Mat *m : mats)
-        if (!m->ok() || m->rank != 0 || !few_gemm_takes(m->t->v, n, false) || m->t->v.tf != first->t->v.tf ||
-            m->t->v.cols != first->t->v.cols)
-            return false;
-    return true;
+    const TileView *views[3];
+    int count = 0;
+    for (const Mat *m : mats) {
+        if (!m->ok() || m->rank != 0) return false;
+        views[count++] = &m->t->v;
+    }
+    return few_launch_takes(views, count, n, FEW_SPLIT_US);
+}
+
+// Whether `mt` reads the fragments of at most 127 rows that its input's producer
+// writes. (With a delta the tiled product's own split forms x . A^T on the way.)
+static bool small_frags(const Mat &mt, int64_t n) {
+    return mt.ok() && (few_gemm_takes(mt.t->v, n, false) || frag_only(mt, n));
 }
 
 // Whether a routed layer's grouped products can be planned on the device:
@@ -1596,7 +1603,7 @@ void model_forward(ditch_hip_model *m, const uint32_t *d_tokens, const ditch_row
         if (prompt_attn) aa.dense = dense_flag;
         // few rows: the row kernel writes the o product's fragments (the f32
         // rows too when a delta reads them)
-        if (row_attn && few && !few_rows && L.o.ok() && few_gemm_takes(L.o.t->v, n, false) && (nh * vd) % 128 == 0) {
+        if (row_attn && few && !few_rows && small_frags(L.o, n) && (nh * vd) % 128 == 0) {
             aa.ldk = split_ldk(nh * vd);
             aa.xs = m->atts.get<uint8_t>(split_bytes_ldk(n, aa.ldk, 2));
             if (L.o.rank == 0) aa.out = nullptr;
@@ -1642,8 +1649,8 @@ void model_forward(ditch_hip_model *m, const uint32_t *d_tokens, const ditch_row
             capture(li + 1);
             continue;
         }
-        if (few && !moe_layer && few_together({&L.gate, &L.up}, n) && few_glu_takes(L.gate.t->v, L.up.t->v, n) &&
-            (few_rows || (L.gate.t->v.rows % 128 == 0 && few_gemm_takes(L.down.t->v, n, false)))) {
+        if (few && !moe_layer && L.gate.ok() && L.up.ok() && L.gate.rank == 0 && L.up.rank == 0 &&
+            few_glu_takes(L.gate.t->v, L.up.t->v, n) && (few_rows || L.gate.t->v.rows % 128 == 0)) {
             const int64_t inter = L.gate.t->v.rows, ldk_i = split_ldk(inter);
             if (few_rows) {
                 launch_rmsnorm(h, x, L.ffn_norm.p, L.ffn_norm.len, n, hidden, c.rms_eps, 0, s);
@@ -1653,8 +1660,9 @@ void model_forward(ditch_hip_model *m, const uint32_t *d_tokens, const ditch_row
             } else {
                 void *hs = m->hs.get<uint8_t>(split_bytes_ldk(n, ldk_h, 2));
                 launch_rmsnorm_split(hs, ldk_h, nullptr, x, L.ffn_norm.p, L.ffn_norm.len, n, hidden, c.rms_eps, 0, s);
-                float *g = L.down.rank > 0 ? m->g.get<float>(n * inter) : nullptr;
-                void *as = m->acts.get<uint8_t>(split_bytes_ldk(n, ldk_i, 2));
+                const bool frag_down = small_frags(L.down, n);
+                float *g = L.down.rank > 0 || !frag_down ? m->g.get<float>(n * inter) : nullptr;
+                void *as = frag_down ? m->acts.get<uint8_t>(split_bytes_ldk(n, ldk_i, 2)) : nullptr;
                 launch_few_glu(L.gate.t->v, L.up.t->v, 0, g, as, ldk_i, nullptr, 0, hs, ldk_h, n, s);
                 mm_act(m, L.down, x, Act{g, as, ldk_i}, n, nullptr, 1, s);  // x += down(act)
             }

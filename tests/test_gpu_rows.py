@@ -95,6 +95,28 @@ def test_gate_up_of_few_tokens_matches_oracle(dev, ref, fmt, shape):
         cm.free()
 
 
+# 33 to 127 tokens where the few-token kernel takes a part of a layer: from 65 on all but o and down (16384 rows: two
+# rounds each), which read the fragments of the attention and the gate/up product, or with a delta its f32 rows; all
+# but gate and up (32768 rows: eight rounds). On 48 all of both
+@pytest.mark.parametrize("fmt,hidden,inter", [("bf16", 16384, 256), ("bf16", 256, 32768), ("q8_0", 256, 32768)])
+def test_layers_partly_of_few_token_products_match_oracle(dev, ref, fmt, hidden, inter):
+    spec = mg.dense(fmt, hidden=hidden, inter=inter, heads=2, kv_heads=1, head_dim=128, layers=1, vocab=256, seed=8)
+    gm, cm = Model(dev, spec), RefModel(spec)
+    rng = np.random.default_rng(7)
+    try:
+        for i, lens in enumerate([[48], [65], [60, 51]]):
+            _check(gm, cm, lens, 256, 60 + i)
+        for slot, k in ((abi.SLOT["O"], 256), (abi.SLOT["DOWN"], inter)):
+            a = (rng.standard_normal((2, k)) * 0.05).astype(np.float32)
+            b = (rng.standard_normal((hidden, 2)) * 0.05).astype(np.float32)
+            for m in (gm, cm):
+                m.set_delta(0, slot, -1, a, b)
+        _check(gm, cm, [60, 51], 256, 63)
+    finally:
+        gm.free()
+        cm.free()
+
+
 # one element, the edges of a 2048-element chunk, of the lanes that add 64
 # chunks, and rows that are not whole float4s
 @pytest.mark.parametrize("V", [1, 2047, 2048, 2052, 133120, 131073])
